@@ -210,7 +210,8 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
   if (n < 1 || !ctxs || !params || !e_limits || !species_numbers || !concentrations)
     return fail(BWL_ERR_ARG, "null argument");
   const int lim = lds_limit();
-  size_t lds = 0, total = align256(sizeof(NsArgs) * (size_t)n);
+  SeqPick pick, energies;
+  size_t total = align256(sizeof(NsArgs) * (size_t)n);
   std::vector<size_t> offs((size_t)n);
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
@@ -224,7 +225,8 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
     if (!has_two_species(c->g, species_numbers[i], concentrations[i]))
       return fail(BWL_ERR_ARG, "nested sampling needs at least two species present");
     if (2 * c->g.R > 64) return fail(BWL_ERR_UNSUPPORTED, "too many shells");
-    lds = std::max(lds, ns_lds_bytes(c->g, p->n_walkers));
+    pick.add(c->g, ns_lds_bytes(c->g, p->n_walkers), ns_spec_lds_bytes(c->g, p->n_walkers));
+    energies.add(c->g, ns_energies_lds_bytes(c->g), energies_spec_lds_bytes(c->g));
     offs[(size_t)i] = total;
     const size_t ref = (size_t)c->g.m[0] * c->g.m[1] * c->g.m[2];
     total += align256((size_t)c->g.compact_bytes * p->n_walkers) +
@@ -232,7 +234,9 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
              align256(sizeof(long long) * 3) + align256(sizeof(double) * p->n_iter) +
              align256(ref * p->n_walkers);
   }
-  if (lds > (size_t)lim) return fail(BWL_ERR_UNSUPPORTED, "lattice and walker energies do not fit in LDS");
+  if (pick.lds > (size_t)lim) return fail(BWL_ERR_UNSUPPORTED, "lattice and walker energies do not fit in LDS");
+  pick.settle(lim);
+  energies.settle(lim);
   bwl_ctx *c0 = ctxs[0];
   DevBuf buf;
   if (hipMalloc(&buf.p, total) != hipSuccess) return fail(BWL_ERR_NOMEM, "device allocation failed");
@@ -292,16 +296,8 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
   HIP_OK(hipMemcpyAsync(base, args.data(), sizeof(NsArgs) * (size_t)n, hipMemcpyHostToDevice, c0->stream));
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
   int max_w = 0;
-  size_t lds_e = 0;
-  for (int i = 0; i < n; ++i) {
-    max_w = std::max(max_w, params[i].n_walkers);
-    lds_e = std::max(lds_e, ns_energies_lds_bytes(ctxs[i]->g));
-  }
-  // one pair-sum variant for the launch when every run shares it
-  int key = pair_sum_key(ctxs[0]->g.lattice, ctxs[0]->g.R);
-  for (int i = 1; i < n; ++i)
-    if (pair_sum_key(ctxs[i]->g.lattice, ctxs[i]->g.R) != key) key = -1;
-  HIP_OK(launch_ns((const NsArgs *)base, n, lds, max_w, lds_e, c0->stream, key));
+  for (int i = 0; i < n; ++i) max_w = std::max(max_w, params[i].n_walkers);
+  HIP_OK(launch_ns((const NsArgs *)base, n, pick, max_w, energies, c0->stream));
   HIP_OK(hipEventRecord(c0->ev1, c0->stream));
   HIP_OK(hipStreamSynchronize(c0->stream));
   float ms = 0.f;
@@ -654,8 +650,10 @@ int bwl_wl_sweeps(bwl_wl *w, double wl_f, int32_t average, int64_t *accepted, do
   wl_fill_args(w, wl_f, args);
   HIP_OK(hipMemcpyAsync(w->d_args, args.data(), sizeof(WlArgs) * W, hipMemcpyHostToDevice, s));
   HIP_OK(hipEventRecord(w->ctx->ev0, s));
-  HIP_OK(launch_wl_sweeps(w->d_args, W, wl_lds_bytes(g, w->p.bins, w->hstride), s,
-                          pair_sum_key(g.lattice, g.R)));
+  SeqPick pick;
+  pick.add(g, wl_lds_bytes(g, w->p.bins, w->hstride), wl_spec_lds_bytes(g, w->p.bins, w->hstride));
+  pick.settle(lds_limit());
+  HIP_OK(launch_wl_sweeps(w->d_args, W, pick, s));
   if (average)
     HIP_OK(launch_wl_average(w->d_lng, w->d_hist, w->p.num_windows, w->p.walkers_per_window,
                              w->p.bins, w->hstride, s));
@@ -699,7 +697,10 @@ int bwl_wl_replica_exchange(bwl_wl *w, int32_t *partner, int32_t *exchanged, dou
   x.bins = w->p.bins;
   HIP_OK(hipMemcpyAsync(w->d_args, args.data(), sizeof(WlArgs) * W, hipMemcpyHostToDevice, s));
   HIP_OK(hipEventRecord(w->ctx->ev0, s));
-  HIP_OK(launch_wl_energies(w->d_args, W, w->d_xe, ns_energies_lds_bytes(g), s));
+  SeqPick pick;
+  pick.add(g, ns_energies_lds_bytes(g), energies_spec_lds_bytes(g));
+  pick.settle(lds_limit());
+  HIP_OK(launch_wl_energies(w->d_args, W, w->d_xe, pick, s));
   HIP_OK(launch_wl_exchange(x, xlds, s));
   HIP_OK(launch_wl_swap_configs(w->d_walkers, (long long)g.compact_bytes, x.swaps, x.n_swaps,
                                 W / 2, s));

@@ -51,6 +51,25 @@ __host__ __device__ constexpr int pair_sum_key(int lattice, int R) {
   return ((lattice == 1 || lattice == 2) && R >= 1 && R <= 6) ? lattice * 16 + R : 0;
 }
 
+// Largest |offset component| over shells 1..R, at compile time.
+__host__ __device__ constexpr int spec_rcut(int lattice, int R) {
+  int z = 0, rc = 0;
+  for (int s = 0; s < R; ++s) z += lattice == 1 ? kFccShellSize[s] : kBccShellSize[s];
+  for (int t = 0; t < z; ++t)
+    for (int a = 0; a < 3; ++a) {
+      const int v = lattice == 1 ? kFccOffsets[t][a] : kBccOffsets[t][a];
+      rc = v > rc ? v : (-v > rc ? -v : rc);
+    }
+  return rc;
+}
+
+// Whether a lattice's sequential samplers can run in speculative batches
+// (bwl_spec.h): up to 4 shells, and every axis longer than twice the
+// interaction range.
+inline bool spec_ok(const Geo &g) {
+  return g.R <= 4 && g.m[0] > 2 * g.rcut && g.m[1] > 2 * g.rcut && g.m[2] > 2 * g.rcut;
+}
+
 // Parity bits of each sublattice.
 __host__ __device__ inline void sub_bits(int lattice, int s, int &bx, int &by, int &bz) {
   if (lattice == 1) {

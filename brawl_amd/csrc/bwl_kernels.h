@@ -209,21 +209,46 @@ const void *par_fixed_kernel(int lattice, int R, int words);
 hipError_t launch_metro_par_fn(const void *fn, const ParArgs *args_dev, int n_chains, size_t lds,
                                int threads, hipStream_t s);
 
+// The kernel of a launch of sequential chains and its LDS, from its members.
+// key: the pair-sum variant they share (pair_sum_key), -1 if they differ.
+// spec: the kernel in speculative batches (bwl_spec.h), for launches whose
+// members share a key and can all use it with the LDS there is (it takes
+// about 13 KB more).  It was faster on every lattice it accepts (a walk of
+// nested sampling, quinary fcc 6^3, 4 shells: 0.61 against 1.31 us per trial;
+// a Wang-Landau walker, bcc 16^3, 2 shells: 0.37 against 1.22 us); the kernels of one
+// trial at a time serve the rest: more than 4 shells, boxes as short as the
+// interaction range, launches that mix lattices.
+struct SeqPick {
+  int key = -2;  // no member yet
+  bool spec = true;
+  size_t lds = 0, lds_spec = 0;
+  void add(const Geo &g, size_t lds_one, size_t lds_batches) {
+    const int k = pair_sum_key(g.lattice, g.R);
+    key = key == -2 || key == k ? k : -1;
+    spec = spec && spec_ok(g);
+    lds = lds_one > lds ? lds_one : lds;
+    lds_spec = lds_batches > lds_spec ? lds_batches : lds_spec;
+  }
+  void settle(int limit) { spec = spec && key > 0 && lds_spec <= (size_t)limit; }
+  size_t bytes() const { return spec ? lds_spec : lds; }
+};
+
 size_t ns_lds_bytes(const Geo &g, int n_walkers);
+size_t ns_spec_lds_bytes(const Geo &g, int n_walkers);
 // Initial walker energies (all walkers at once), then the runs (one
-// wavefront each).
-// key: the pair-sum variant shared by every run (pair_sum_key), -1 if mixed
-hipError_t launch_ns(const NsArgs *args_dev, int n, size_t lds, int max_walkers, size_t lds_energies,
-                     hipStream_t s, int key);
+// workgroup each).
+hipError_t launch_ns(const NsArgs *args_dev, int n, const SeqPick &pick, int max_walkers, const SeqPick &energies,
+                     hipStream_t s);
 size_t ns_energies_lds_bytes(const Geo &g);
+size_t energies_spec_lds_bytes(const Geo &g);
 size_t wl_lds_bytes(const Geo &g, int bins, int window_bins);
-// key: the pair-sum variant shared by every walker (pair_sum_key), -1 if mixed
-hipError_t launch_wl_sweeps(const WlArgs *args_dev, int n, size_t lds, hipStream_t s, int key);
+size_t wl_spec_lds_bytes(const Geo &g, int bins, int window_bins);
+hipError_t launch_wl_sweeps(const WlArgs *args_dev, int n, const SeqPick &pick, hipStream_t s);
 hipError_t launch_wl_average(double *lng, double *hist, int n_windows, int walkers_per_window,
                              int bins, int hist_stride, hipStream_t s);
-// Walker energies (ns_energies_lds_bytes of LDS), the exchange decisions
-// (one wavefront) and the exchange of configurations.
-hipError_t launch_wl_energies(const WlArgs *args_dev, int n, double *E, size_t lds, hipStream_t s);
+// Walker energies, the exchange decisions (one wavefront) and the exchange
+// of configurations.
+hipError_t launch_wl_energies(const WlArgs *args_dev, int n, double *E, const SeqPick &pick, hipStream_t s);
 size_t wl_exchange_lds_bytes(int W, int wpw);
 hipError_t launch_wl_exchange(const WlExchangeArgs &a, size_t lds, hipStream_t s);
 hipError_t launch_wl_swap_configs(int8_t *walkers, long long bytes, const int32_t *swaps,

@@ -317,6 +317,21 @@ __device__ inline void pair_sum2_t(const GEO &g, const PairLanes &pl, const doub
     default: return (const void *)kern<-1>;               \
   }
 
+// The speculative kernel of template family `kern` (bwl_spec.h) for a key of
+// up to 4 shells, nullptr for any other.
+#define BWL_KERNEL_FOR_SPEC_KEY(kern, key)                \
+  switch (key) {                                          \
+    case 16 + 1: return (const void *)kern<16 + 1>;       \
+    case 16 + 2: return (const void *)kern<16 + 2>;       \
+    case 16 + 3: return (const void *)kern<16 + 3>;       \
+    case 16 + 4: return (const void *)kern<16 + 4>;       \
+    case 32 + 1: return (const void *)kern<32 + 1>;       \
+    case 32 + 2: return (const void *)kern<32 + 2>;       \
+    case 32 + 3: return (const void *)kern<32 + 3>;       \
+    case 32 + 4: return (const void *)kern<32 + 4>;       \
+    default: return nullptr;                              \
+  }
+
 // Energies of sites A and B in the reference's FP64 order (pair_energy,
 // bw_hamiltonian.f90:99-114): every lane gathers neighbour V entries (one
 // per 64-entry pass), then the entries are added in list order from 0.0

@@ -335,8 +335,13 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   L->kind = KIND_NS;
   L->slot = slot;
   L->reqs = grp;
-  size_t lds = 0;
-  for (Request *r : grp) lds = std::max(lds, ns_lds_bytes(r->g, r->np.n_walkers));
+  SeqPick pick, energies;
+  for (Request *r : grp) {
+    pick.add(r->g, ns_lds_bytes(r->g, r->np.n_walkers), ns_spec_lds_bytes(r->g, r->np.n_walkers));
+    energies.add(r->g, ns_energies_lds_bytes(r->g), energies_spec_lds_bytes(r->g));
+  }
+  pick.settle(lds_limit());
+  energies.settle(lds_limit());
   L->scratch_bytes = al(sizeof(NsArgs) * grp.size());
   L->scratch = s->arena.alloc(L->scratch_bytes);
   if (!L->scratch) return BWL_ERR_NOMEM;
@@ -381,15 +386,8 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
   int max_w = 0;
-  size_t lds_e = 0;
-  for (Request *r : grp) {
-    max_w = std::max(max_w, r->np.n_walkers);
-    lds_e = std::max(lds_e, ns_energies_lds_bytes(r->g));
-  }
-  int key = pair_sum_key(grp[0]->g.lattice, grp[0]->g.R);
-  for (Request *r : grp)
-    if (pair_sum_key(r->g.lattice, r->g.R) != key) key = -1;
-  HIP_OK(launch_ns((const NsArgs *)L->scratch, (int)grp.size(), lds, max_w, lds_e, st, key));
+  for (Request *r : grp) max_w = std::max(max_w, r->np.n_walkers);
+  HIP_OK(launch_ns((const NsArgs *)L->scratch, (int)grp.size(), pick, max_w, energies, st));
   HIP_OK(hipEventRecord(L->ev1, st));
   s->slot_busy[(size_t)slot] = true;
   s->running.push_back(std::move(L));
@@ -402,11 +400,13 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   L->kind = KIND_WL;
   L->slot = slot;
   L->reqs = grp;
-  size_t lds = 0, total_w = 0;
+  SeqPick pick;
+  size_t total_w = 0;
   for (Request *r : grp) {
-    lds = std::max(lds, wl_lds_bytes(r->g, r->wp.bins, r->hstride));
+    pick.add(r->g, wl_lds_bytes(r->g, r->wp.bins, r->hstride), wl_spec_lds_bytes(r->g, r->wp.bins, r->hstride));
     total_w += (size_t)r->wp.num_windows * r->wp.walkers_per_window;
   }
+  pick.settle(lds_limit());
   L->scratch_bytes = al(sizeof(WlArgs) * total_w);
   L->scratch = s->arena.alloc(L->scratch_bytes);
   if (!L->scratch) return BWL_ERR_NOMEM;
@@ -468,11 +468,7 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
-  // one pair-sum variant for the launch when every walker shares it
-  int key = pair_sum_key(L->wl_args[0].g.lattice, L->wl_args[0].g.R);
-  for (const WlArgs &a : L->wl_args)
-    if (pair_sum_key(a.g.lattice, a.g.R) != key) key = -1;
-  HIP_OK(launch_wl_sweeps((const WlArgs *)L->scratch, (int)total_w, lds, st, key));
+  HIP_OK(launch_wl_sweeps((const WlArgs *)L->scratch, (int)total_w, pick, st));
   for (size_t i = 0; i < grp.size(); ++i) {
     Request *r = grp[i];
     const WlArgs &a0 = L->wl_args[L->wl_first[i]];

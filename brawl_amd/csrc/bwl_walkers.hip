@@ -11,7 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bwl_kernels.h"
-#include "bwl_seq.h"
+#include "bwl_spec.h"
 
 namespace bwl {
 
@@ -226,6 +226,347 @@ __global__ __launch_bounds__(64) void k_ns(const NsArgs *__restrict__ args) {
 }
 
 // ------------------------------------------------------------------
+// Nested sampling in speculative batches (bwl_spec.h); the run and its
+// results are those of k_ns.  A walk's trial draws three numbers for its
+// first site, then three per candidate second site until one holds another
+// species, so with the lattice as it is the whole run of trials is fixed by
+// the species of the next 64 triples' sites: lane l holds triple l, finds the
+// first later triple of another species from the ballots per species, and
+// the trials follow by hopping from a trial's last triple to the next.
+//
+// Four trials at a time: trial g = lane >> 4, and within its 16 lanes the
+// shell (lane & 3), the site (lane & 4) and before or after the swap (lane &
+// 8), one chain of ordered additions each.  Early in a run nearly every trial
+// is accepted and on the small lattices of such runs a swap reaches a
+// quarter of the others, so the trials are foreseen to end as most of the
+// last ones did: foreseen accepted, a trial's swap is written before the next
+// trial's neighbours are read (one wavefront's LDS accesses complete in
+// program order), and taken back if the decision falls otherwise.
+// ------------------------------------------------------------------
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_ns_spec(const NsArgs *__restrict__ args) {
+  using D = SpecDims<KEY>;
+  constexpr int ML = D::ML, R = D::R;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const NsArgs &A = args[blockIdx.x];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = wave_uniform(tid >> 6);
+  const SeqGeo g = seq_geo(A.g);
+  const int S = g.S;
+  const uint32_t inv_S = inverse_of(S);
+  uint8_t *p = smem;
+  auto take = [&](size_t bytes) {
+    uint8_t *at = p;
+    p += (bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  int8_t *lat = (int8_t *)take(A.g.lds_bytes);
+  uint32_t *raw = (uint32_t *)take(4 * 624);
+  uint32_t *tem = (uint32_t *)take(4 * kRingWords);
+  uint2 *rsite = (uint2 *)take(8 * kRingWords);
+  // command, walker to clone, walker discarded, walker discarded before
+  volatile int32_t *sh = (volatile int32_t *)take(16);
+  double *vex = (double *)take(sizeof(double) * S * S * R);
+  double *E = (double *)take(sizeof(double) * A.n_walkers);
+  int32_t *offp = (int32_t *)take(4 * D::NSUB * R * ML);
+  uint8_t *adj = take(D::TS * D::TS * D::TS);
+
+  const int nw = A.n_walkers;
+  const size_t cb = (size_t)A.g.compact_bytes;
+  for (int i = tid; i < 624; i += kSpecThreads) raw[i] = A.mt[i];
+  for (int i = tid; i < S * S * R; i += kSpecThreads) vex[i] = A.vex[i];
+  for (int w = tid; w < nw; w += kSpecThreads) E[w] = A.E[w];
+  stage_spec_tables<KEY>(offp, adj, A.off);
+  __syncthreads();
+  ring_start<D::LAT>(g, raw, tem, rsite);
+  const SpecLds L{lat, offp, vex, adj};
+  // the walked lattice over the discarded walker, then the next clone
+  auto turn = [&](int cmd) {
+    const int src = sh[1], last = sh[3];
+    if (cmd != kCmdLoad) {
+      unstage_codes(lat, A.walkers + cb * last, g, D::NSUB, inv_S);
+      __syncthreads();
+    }
+    if (cmd != kCmdStore) {
+      stage_codes(lat, A.walkers + cb * src, g, D::NSUB, S);
+      __syncthreads();
+    }
+  };
+  if (wave != 0) {
+    spec_helper<D::LAT>(g, raw, tem, rsite, sh, turn);
+    return;
+  }
+
+  MtRing ring{raw, tem, rsite, sh, 0, wave_uniform(A.mt_index[0]), false};
+  const int grp = lane >> 4, w = (lane >> 2) & 1, shell = (lane & 3) < R ? lane & 3 : R - 1;
+  const bool after = (lane & 8) != 0;
+  int first, len;
+  lane_shell<KEY>(shell, first, len);
+  const int row = shell * S * S;
+  const unsigned long long later = lane == 63 ? 0ull : ~0ull << (lane + 1);
+  long long trials = 0, accepted = 0;
+  int extra = 0, n_acc = 0, status = 0;
+  bool foresee = true;  // trials foreseen accepted
+  const int half = (int)((float)nw / 2.0f);
+  int it = 1;
+  for (; it <= A.n_iter && status == 0; ++it) {
+    // maxloc: the first maximum (nested_sampling.f90:117)
+    double best = -INFINITY;
+    int bi = 0x7fffffff;  // no walker seen
+    for (int k = lane; k < nw; k += 64)
+      if (bi == 0x7fffffff || E[k] > best) {
+        best = E[k];
+        bi = k;
+      }
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) {
+      const double ob = __shfl_xor(best, m);
+      const int oi = __shfl_xor(bi, m);
+      if (oi != 0x7fffffff && (bi == 0x7fffffff || ob > best || (ob == best && oi < bi))) {
+        best = ob;
+        bi = oi;
+      }
+    }
+    const double limit = best;
+    const int imax = wave_uniform(bi);
+    if (lane == 0) A.e_limits[it - 1] = limit;
+    // walk-length adaptation (nested_sampling.f90:129-144)
+    if (it % half == 0) {
+      if (((float)n_acc < (float)A.n_at * 0.05f) && (extra < A.n_steps * 100)) extra += A.n_steps;
+    }
+    // clone a random walker over the discarded one (nested_sampling.f90:149-152)
+    ring_ensure(ring, 1);
+    const double rnd = (double)*ring_at(ring, tem, 0) * (1.0 / 4294967296.0);
+    ring.q += 1;
+    int irnd = (int)ceil(rnd * (double)nw);
+    if (irnd < 1) irnd = 1;
+    const int src = wave_uniform(irnd - 1);
+    if (lane == 0) {
+      sh[3] = sh[2];
+      sh[1] = src;
+      sh[2] = imax;
+    }
+    const int cmd = it == 1 ? kCmdLoad : kCmdTurn;
+    spec_command(ring, cmd);
+    turn(cmd);
+    double ecur = E[src];
+    n_acc = 0;
+    // the walk (nested_sampling.f90:157-192)
+    int left = A.n_steps + extra;
+    while (left > 0 && status == 0) {
+      ring_ensure(ring, 194);
+      uint2 site = *ring_at(ring, rsite, 3 * lane);
+      int code = lat[site.y];
+      unsigned long long same = 0;
+      for (int s = 0; s < S; ++s) {
+        const unsigned long long m = __ballot(code == s * S);
+        same = code == s * S ? m : same;
+      }
+      const unsigned long long differ = ~same & later;
+      const int second = differ ? __ffsll((long long)differ) - 1 : 64;
+      int j = 0;  // first triple of the next trial
+      if (__builtin_amdgcn_readlane(second, 0) == 64) {
+        // no site of another species in sight: the first site is kept (lane
+        // 0) and the stream searched on, 64 candidates at a time
+        const int c0 = __builtin_amdgcn_readlane(code, 0);
+        long long seen = 63;
+        for (;;) {
+          ring.q += 192;
+          if (seen >= A.max_redraws) {
+            status = 1;
+            break;
+          }
+          ring_ensure(ring, 194);
+          const uint2 s2 = *ring_at(ring, rsite, 3 * lane);
+          const int c2 = lat[s2.y];
+          const unsigned long long m = __ballot(c2 != c0);
+          if (m) {
+            // as if the two had been triples 0 and 1, with the position after them
+            const int k = __ffsll((long long)m) - 1;
+            const uint32_t x1 = (uint32_t)__builtin_amdgcn_readlane((int)s2.x, k);
+            const uint32_t y1 = (uint32_t)__builtin_amdgcn_readlane((int)s2.y, k);
+            const int c1 = __builtin_amdgcn_readlane(c2, k);
+            if (lane == 1) {
+              site = make_uint2(x1, y1);
+              code = c1;
+            }
+            ring.q += 3 * (k + 1) - 6;
+            break;
+          }
+          seen += 64;
+        }
+        if (status) break;
+        j = -1;  // one trial of triples 0 and 1, then a new window
+      }
+      const bool lone = j < 0;
+      if (lone) j = 0;
+      bool stale = false;
+      while (!stale) {
+        // the next trials' triples (j: first site, k: second), each lane
+        // hopping to its own trial's
+        const int most = lone ? 1 : (left < 4 ? left : 4);
+        int my_j = j, my_k = __shfl(second, j);
+        if (lone) my_k = 1;
+#pragma unroll
+        for (int t = 1; t < 4; ++t) {
+          const int k = __shfl(second, (my_k + 1) & 63);
+          const bool hop = grp >= t;
+          my_j = hop ? my_k + 1 : my_j;
+          my_k = hop ? (my_j < 64 ? k : 64) : my_k;
+        }
+        // trials in sight: those before the first without a second site
+        const unsigned long long out = __ballot(my_k >= 64);
+        int ng = out ? (__ffsll((long long)out) - 1) >> 4 : 4;
+        ng = ng < most ? ng : most;
+        if (ng == 0) break;
+        my_j &= 63;
+        my_k &= 63;
+        const uint32_t pa = (uint32_t)__shfl((int)site.x, my_j), pb = (uint32_t)__shfl((int)site.x, my_k);
+        const int aa = __shfl((int)site.y, my_j), ab = __shfl((int)site.y, my_k);
+        const int ca = __shfl(code, my_j), cb2 = __shfl(code, my_k);
+        // Row trial grp against column trial lane & 3, one pair of their
+        // sites per lane: the same site, or a site the column's trial passed
+        // over (the first two are looked at; a trial that passed over more
+        // counts as equal to any), or within reach.
+        const int col = (lane & 3) * 16;
+        const uint32_t qa = (uint32_t)__shfl((int)pa, col), qb = (uint32_t)__shfl((int)pb, col);
+        const int cj = __shfl(my_j, col), ck = __shfl(my_k, col);
+        const uint32_t r1 = (uint32_t)__shfl((int)site.x, (cj + 1) & 63), r2 = (uint32_t)__shfl((int)site.x, (cj + 2) & 63);
+        const uint32_t rp = (lane & 4) ? pb : pa, cp = (lane & 8) ? qb : qa;
+        bool equal = rp == cp;
+        if (!lone) equal = equal || (ck > cj + 1 && rp == r1) || (ck > cj + 2 && rp == r2) || ck > cj + 3;
+        const bool reach = box_gap(unpack_xyz(rp), unpack_xyz(cp), g, D::RC) <= 2u * D::RC;
+        unsigned long long eq = __ballot(equal && grp < (lane & 3));
+        const unsigned long long conf = __ballot(reach);
+        if (eq) {
+          eq |= eq >> 32;
+          eq |= eq >> 16;
+          eq |= eq >> 8;
+          eq |= eq >> 4;
+          const int c = __ffs((int)(eq & 0xeu)) - 1;
+          ng = c < ng ? c : ng;
+        }
+        // triples of the sites that these trials may exchange: once passed, a
+        // later one's species is out of date
+        bool touched = false;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          touched |= q < ng && (site.x == (uint32_t)__builtin_amdgcn_readlane((int)pa, 16 * q) ||
+                                site.x == (uint32_t)__builtin_amdgcn_readlane((int)pb, 16 * q));
+        const unsigned long long hit = __ballot(touched);
+        const SiteXYZ own = unpack_xyz(w ? pb : pa), oth = unpack_xyz(w ? pa : pb);
+        const int c_own = w ? cb2 : ca, c_oth = w ? ca : cb2;
+        // images of both sites over the trial's 16 lanes
+        const SiteXYZ ws = unpack_xyz(after ? pb : pa);
+        const int wat = image_addr<D::LAT>(g, ws, lane & 7);
+        const int wold = after ? cb2 : ca, wnew = after ? ca : cb2;
+        const int addr = w ? ab : aa;
+        const int at = neighbour_index<KEY>(L, g, own, oth) - first;
+        // the shell's cells are read half by the lane before the swap, half
+        // by its partner after it, and exchanged
+        constexpr int MH = ML / 2;
+        int mh[MH];
+        int2 o[MH / 2];
+        {
+          const int2 *op = (const int2 *)(offp + (spec_sub<D::LAT>(own) * R + shell) * ML) + (after ? MH / 2 : 0);
+#pragma unroll
+          for (int q = 0; q < MH / 2; ++q) o[q] = op[q];
+        }
+        if (foresee) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            wave_lds_order();
+            if (grp == t) {
+#pragma unroll
+              for (int q = 0; q < MH / 2; ++q) {
+                mh[2 * q] = lat[addr + o[q].x];
+                mh[2 * q + 1] = lat[addr + o[q].y];
+              }
+              wave_lds_order();
+              if (t < ng && wat >= 0) lat[wat] = (int8_t)wnew;
+            }
+          }
+          wave_lds_order();
+        } else {
+#pragma unroll
+          for (int q = 0; q < MH / 2; ++q) {
+            mh[2 * q] = lat[addr + o[q].x];
+            mh[2 * q + 1] = lat[addr + o[q].y];
+          }
+        }
+        int cd[ML];
+#pragma unroll
+        for (int q = 0; q < MH; ++q) {
+          const int other = __builtin_amdgcn_update_dpp(0, mh[q], kRowRotate8, 0xf, 0xf, true);
+          cd[q] = after ? other : mh[q];
+          cd[MH + q] = after ? mh[q] : other;
+        }
+        const double *vr = vex + row + (int)(__umul24((uint32_t)(after ? c_oth : c_own), inv_S) >> 16);
+        double v[ML];
+#pragma unroll
+        for (int i = 0; i < ML; ++i) v[i] = vr[cd[i]];
+        // after the swap the other site, seen as a neighbour, has this site's species
+        const bool fix = after && at >= 0 && at < len;
+        if (__ballot(fix) != 0) {
+          const double f = vr[c_own];
+#pragma unroll
+          for (int i = 0; i < ML; ++i) v[i] = fix && i == at ? f : v[i];
+        }
+        double e = quad_sum<R>(shell_chain<ML>(v, len));
+        e = e + dpp_d<kRowHalfMirror>(e);
+        const double de = dpp_d<kRowRotate8>(e) - e;  // lanes before: after - before
+        // The decisions, in order and without branches: a trial counts until
+        // one is reached by an earlier one that went otherwise than foreseen
+        // (it was read from the wrong lattice).
+        int swaps = 0, off_course = 0, t = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          uint32_t c = (uint32_t)(conf >> (16 * q)) & 0xffffu;
+          c |= c >> 8;
+          c = (c | c >> 4) & 0xfu & (0xeu << q);
+          const bool counts = q < ng && t == q && !((off_course >> q) & 1);
+          const double en = ecur + readlane_d(de, 16 * q);
+          const bool acc = counts && en < limit;
+          ecur = acc ? en : ecur;
+          swaps |= acc ? 1 << q : 0;
+          off_course |= counts && acc != foresee ? (int)c : 0;
+          t += counts ? 1 : 0;
+        }
+        swaps = wave_uniform(swaps);
+        t = wave_uniform(t);
+        const bool mine = ((swaps >> grp) & 1u) != 0;
+        wave_lds_order();
+        if (grp < ng && mine != foresee && wat >= 0) lat[wat] = (int8_t)(mine ? wnew : wold);
+        wave_lds_order();
+        const int got = __popc((unsigned)swaps);
+        foresee = 2 * got > t;
+        const int next = __builtin_amdgcn_readlane(my_k, 16 * (t - 1)) + 1;
+        left -= t;
+        trials += t;
+        n_acc += got;
+        j = next;
+        stale = lone || left <= 0 || j >= 64 || (hit >> j) != 0;
+      }
+      ring.q += 3 * j;
+    }
+    accepted += n_acc;
+    if (lane == 0) E[imax] = ecur;
+    wave_lds_order();
+  }
+  if (lane == 0) sh[3] = sh[2];
+  spec_command(ring, kCmdStore);
+  turn(kCmdStore);
+  spec_command(ring, kCmdExit);
+  for (int k = lane; k < nw; k += 64) A.E[k] = E[k];
+  ring_finish(ring, A.mt, A.mt_index);
+  if (lane == 0) {
+    A.counters[0] = trials;
+    A.counters[1] = accepted;
+    A.counters[2] = status;
+  }
+}
+
+// ------------------------------------------------------------------
 // Wang-Landau `sweeps` (wang-landau.F90:539-632) for one walker, without the
 // window average (a separate kernel does that after every walker's call).
 // The walker's ln g and visit histogram are staged in LDS.  KEY is the
@@ -356,6 +697,221 @@ __global__ __launch_bounds__(64) void k_wl_sweeps(const WlArgs *__restrict__ arg
   }
 }
 
+// ------------------------------------------------------------------
+// `sweeps` in speculative batches (bwl_spec.h); the call and its results are
+// those of k_wl_sweeps.  A trial whose new energy lies inside the window
+// draws one number after its sites', so trial t of a batch is foreseen to
+// start t * len draws on, len by whether the walker is inside its window; a
+// trial that goes otherwise ends its batch.  The energies of the batch's 8
+// trials are formed together (8 lanes each); the decisions too, from one
+// trial that changes the walker to the next (a decision at a time on the
+// scalar unit costs a round trip of about 60 cycles for every branch on a
+// vector result).
+// ------------------------------------------------------------------
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *__restrict__ args) {
+  using D = SpecDims<KEY>;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const WlArgs &A = args[blockIdx.x];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = wave_uniform(tid >> 6);
+  const SeqGeo g = seq_geo(A.g);
+  const int S = g.S, n_atoms = A.g.n_atoms;
+  const uint32_t inv_S = inverse_of(S);
+  const int bins = A.bins, start_idx = A.start_idx, end_idx = A.end_idx;
+  const int hb = end_idx - start_idx + 1;
+  uint8_t *p = smem;
+  auto take = [&](size_t bytes) {
+    uint8_t *at = p;
+    p += (bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  int8_t *lat = (int8_t *)take(A.g.lds_bytes);
+  uint32_t *raw = (uint32_t *)take(4 * 624);
+  uint32_t *tem = (uint32_t *)take(4 * kRingWords);
+  uint2 *rsite = (uint2 *)take(8 * kRingWords);
+  volatile int32_t *cmd = (volatile int32_t *)take(16);
+  double *vex = (double *)take(sizeof(double) * S * S * D::R);
+  double *lng = (double *)take(sizeof(double) * bins);
+  double *hist = (double *)take(sizeof(double) * hb);
+  double *ebuf = (double *)take(sizeof(double) * 2 * kEnergyChunk);
+  int32_t *offp = (int32_t *)take(4 * D::NSUB * D::R * D::ML);
+  uint8_t *adj = take(D::TS * D::TS * D::TS);
+
+  for (int i = tid; i < 624; i += kSpecThreads) raw[i] = A.mt[i];
+  for (int i = tid; i < S * S * D::R; i += kSpecThreads) vex[i] = A.vex[i];
+  for (int i = tid; i < bins; i += kSpecThreads) lng[i] = A.lng[i];
+  for (int i = tid; i < hb; i += kSpecThreads) hist[i] = A.hist[i];
+  stage_spec_tables<KEY>(offp, adj, A.off);
+  stage_codes(lat, A.compact, g, D::NSUB, S);
+  __syncthreads();
+  ring_start<D::LAT>(g, raw, tem, rsite);
+  const SpecLds L{lat, offp, vex, adj};
+  double e_un = spec_total_energy<KEY>(L, g, n_atoms, S, inv_S, ebuf);
+  if (wave != 0) {
+    spec_helper<D::LAT>(g, raw, tem, rsite, cmd, [](int) {});
+  } else {
+    MtRing ring{raw, tem, rsite, cmd, 0, wave_uniform(A.mt_index[0]), false};
+    const int trial = lane >> 3, w = (lane >> 2) & 1, shell = lane & 3;
+    const bool nbr_swap = A.nbr_swap != 0;
+    const int drawn = nbr_swap ? 4 : 6;  // by a trial's sites
+    const double wl_f = A.wl_f;
+    const int cadence = wave_uniform((int)(0.02 * (double)(float)n_atoms));
+    const BinMap bmap = bin_map(A.bin_edges, bins);
+    // x = (e - e0) / range * bins as one multiply-add, good to 1e-9 while
+    // |e0 / range * bins| and |x| stay below 1e6: the bin is its truncation
+    // unless x lies within 1e-6 of an integer (then the reference's form)
+    const double slope = bmap.rinv * bmap.nb, shift = -(bmap.e0 * slope);
+    const bool quick = wave_uniform(fabs(shift) < 1e6) != 0;
+    int ibin = wave_uniform(wl_bin_index(e_un, A.bin_edges, bins));  // bin of e_un, kept with it
+    auto in_range = [&](int b) { return b >= 1 && b <= bins; };
+    auto in_window = [&](int b) { return b >= start_idx && b <= end_idx; };
+    // ln g of ibin, kept here and written back when the walker leaves the bin
+    double lcur = in_range(ibin) ? lng[ibin - 1] : 0.0;
+    long long accepted = 0;
+    long long left = (long long)wave_uniform(A.mc_sweeps) * n_atoms;
+    int to_hit = cadence;
+    auto count_visits = [&](int n) {  // the cadence-th trials among the next n, all ending in ibin
+      if (cadence <= 0) return;
+      while (__builtin_expect(n >= to_hit, 0)) {
+        n -= to_hit;
+        to_hit = cadence;
+        if (in_window(ibin) && lane == 0) hist[ibin - start_idx] += 1.0;
+      }
+      to_hit -= n;
+    };
+    while (left > 0) {
+      const bool inside = wave_uniform(in_window(ibin)) != 0;  // trials foreseen to draw for the decision
+      const int len = drawn + (inside ? 1 : 0);
+      ring_ensure(ring, 7 * kBatch + 2);
+      const uint2 s1 = *ring_at(ring, rsite, len * trial);
+      const SiteXYZ sa = unpack_xyz(s1.x);
+      uint2 s2;
+      if (nbr_swap) {
+        const SiteXYZ sn = nbr_of_draw(g, sa, *ring_at(ring, tem, len * trial + 3));
+        s2 = make_uint2(pack_xyz(sn), (uint32_t)spec_addr<D::LAT>(g, sn));
+      } else {
+        s2 = *ring_at(ring, rsite, len * trial + 3);
+      }
+      const uint32_t ru = *ring_at(ring, tem, len * trial + drawn);
+      const SiteXYZ sb = unpack_xyz(s2.x);
+      const int ca = lat[s1.y], cb = lat[s2.y];
+      const bool differ = ca != cb;
+      const unsigned long long same = __ballot(!differ);
+      const SiteXYZ own = w ? sb : sa, oth = w ? sa : sb;
+      const int c_own = w ? cb : ca, c_oth = w ? ca : cb;
+      double pu, ps;
+      spec_pair_energies<KEY>(L, g, S, inv_S, shell, own, oth, (int)(w ? s2.y : s1.y), c_own, c_oth, pu, ps);
+      const unsigned long long conf = __ballot(batch_conflict(g, D::RC, s1.x, s2.x));
+      // the float logarithm decides when clear of its threshold by 1e-4
+      // (its error is below 1e-5); a drawn 0 goes to the full comparison
+      const double lf = ru ? (double)__logf((float)((double)ru * (1.0 / 4294967296.0))) : NAN;
+      const double surely = lf + 1e-4, hardly = lf - 1e-4;
+      int nt = wave_uniform(left < kBatch ? (int)left : kBatch);
+      int t0 = 0, off = 0;
+      uint32_t swaps = 0;
+      // The decisions, as far at a time as the next trial that changes the
+      // walker: until then every trial sees the same energy, and a ln g that
+      // has grown by wl_f per trial since (as a product here, which is near
+      // enough for a decision that is clear by 1e-4; added up trial by trial
+      // where it is kept).
+      for (;;) {
+        t0 = wave_uniform(t0);
+        nt = wave_uniform(nt);
+        ibin = wave_uniform(ibin);
+        to_hit = wave_uniform(to_hit);
+        const double e_sw = e_un - pu + ps;
+        const double x = __builtin_fma(e_sw, slope, shift);
+        const int xi = (int)x;
+        const double f = fabs(x - (double)xi);
+        const int jbin = differ ? xi + 1 : ibin;  // equal species: nothing moves
+        const bool inw = in_window(jbin);
+        const double lmem = lng[inw ? jbin - 1 : 0];
+        const double grow = in_range(ibin) ? wl_f : 0.0;
+        const double th = jbin == ibin ? 0.0 : __builtin_fma((double)(trial - t0), grow, lcur - lmem);
+        const bool acc = surely < th;
+        // trials for the full path below: another number of draws than
+        // foreseen, or a bin or a decision too close to call here
+        const bool close = differ & !((fabs(x) < 1e6) & (f > 1e-6) & (f < 1.0 - 1e-6));
+        const bool full = !quick | (inw != inside) | close | (inside & !acc & !(hardly > th));
+        const unsigned long long live = (~0ull << (8 * t0)) & (nt < 8 ? (1ull << (8 * nt)) - 1ull : ~0ull);
+        const unsigned long long fulls = __ballot(full) & live;
+        const unsigned long long events = fulls | (__ballot(acc & inw & differ) & live);
+        const int te = events ? (__ffsll((long long)events) - 1) >> 3 : nt;
+        // trials t0 .. te-1: rejected, or accepted without a change
+        if (te > t0) {
+          if (inside) accepted += __popcll(same & live & (te < 8 ? (1ull << (8 * te)) - 1ull : ~0ull) & 0x0101010101010101ull);
+          const int n = te - t0;
+          if (n & 1) lcur = lcur + grow;
+          if (n & 2) lcur = (lcur + grow) + grow;
+          if (n & 4) lcur = (((lcur + grow) + grow) + grow) + grow;
+          if (n & 8) lcur = (((((((lcur + grow) + grow) + grow) + grow) + grow) + grow) + grow) + grow;
+          count_visits(te - t0);
+        }
+        t0 = te;
+        if (te >= nt) break;
+        const int l = 8 * te;
+        ++t0;
+        if (__builtin_expect((fulls >> l) & 1ull, 0)) {
+          // one trial in the reference's own terms; it ends the batch
+          bool in1 = in_window(ibin), acc1 = in1;  // equal species: accepted (log u < 0) when it draws
+          if (!((same >> l) & 1ull)) {
+            const double e1 = readlane_d(e_sw, l);
+            const int b1 = wave_uniform((int)(((e1 - bmap.e0) / bmap.range) * bmap.nb) + 1);
+            in1 = in_window(b1);
+            acc1 = false;
+            if (in1) {
+              const double l1 = b1 == ibin ? lcur : lng[b1 - 1];
+              const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)ru, l);
+              acc1 = wave_uniform(log_lt_dev((double)r * (1.0 / 4294967296.0), lcur - l1)) != 0;
+              if (acc1) {
+                if (lane == 0 && in_range(ibin)) lng[ibin - 1] = lcur;
+                wave_lds_order();
+                e_un = e1;
+                ibin = b1;
+                lcur = l1;
+                swaps |= 1u << te;
+              }
+            }
+          }
+          accepted += acc1 ? 1 : 0;
+          if (in_range(ibin)) lcur = lcur + wl_f;
+          count_visits(1);
+          off = (in1 ? 1 : 0) - (inside ? 1 : 0);
+          break;
+        }
+        ++accepted;
+        if (lane == 0 && in_range(ibin)) lng[ibin - 1] = lcur;
+        wave_lds_order();
+        e_un = readlane_d(e_sw, l);
+        const int to = __builtin_amdgcn_readlane(jbin, l);
+        lcur = (to == ibin ? lcur : readlane_d(lmem, l)) + wl_f;
+        ibin = to;
+        count_visits(1);
+        swaps |= 1u << te;
+        // the first later trial that the swap reaches ends the batch
+        const uint32_t reached = (uint32_t)(conf >> l) & 0xffu & (0xffu << t0);
+        if (reached) nt = min(nt, __ffs((int)reached) - 1);
+        if (t0 >= nt) break;
+      }
+      t0 = wave_uniform(t0);
+      batch_write<D::LAT>(lat, g, ((swaps >> trial) & 1u) != 0, own, c_oth);
+      ring.q = wave_uniform(ring.q + len * t0 + off);
+      left -= t0;
+    }
+    if (lane == 0) {
+      if (in_range(ibin)) lng[ibin - 1] = lcur;
+      A.accepted[0] = accepted;
+    }
+    spec_command(ring, kCmdExit);
+    ring_finish(ring, A.mt, A.mt_index);
+  }
+  __syncthreads();
+  unstage_codes(lat, A.compact, g, D::NSUB, inv_S);
+  for (int i = tid; i < bins; i += kSpecThreads) A.lng[i] = lng[i];
+  for (int i = tid; i < hb; i += kSpecThreads) A.hist[i] = hist[i];
+}
+
 // Window average after `sweeps` (wang-landau.F90:628-631): ln g and the
 // visit histogram summed over a window's walkers in walker order, divided
 // by the number of walkers, and written back to every walker of the window.
@@ -402,6 +958,51 @@ __global__ __launch_bounds__(64) void k_wl_energies(const WlArgs *__restrict__ a
   __syncthreads();
   const double e = ref_total_energy(lat, g, offl, vex);
   if (threadIdx.x == 0) E[blockIdx.x] = e;
+}
+
+// Reference-order total energies of walkers by whole workgroups
+// (spec_total_energy): block w is Wang-Landau walker w, or walker w of
+// nested-sampling run blockIdx.y with its energy jitter.
+template <int KEY>
+__device__ __forceinline__ double walker_energy(const Geo &geo, const int8_t *compact, const int32_t *off,
+                                                const double *v, uint8_t *smem) {
+  using D = SpecDims<KEY>;
+  const SeqGeo g = seq_geo(geo);
+  const int S = g.S;
+  uint8_t *p = smem;
+  auto take = [&](size_t bytes) {
+    uint8_t *at = p;
+    p += (bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  int8_t *lat = (int8_t *)take(geo.lds_bytes);
+  double *vex = (double *)take(sizeof(double) * S * S * D::R);
+  double *ebuf = (double *)take(sizeof(double) * 2 * kEnergyChunk);
+  int32_t *offp = (int32_t *)take(4 * D::NSUB * D::R * D::ML);
+  uint8_t *adj = take(D::TS * D::TS * D::TS);
+  for (int i = threadIdx.x; i < S * S * D::R; i += kSpecThreads) vex[i] = v[i];
+  stage_spec_tables<KEY>(offp, adj, off);
+  stage_codes(lat, compact, g, D::NSUB, S);
+  __syncthreads();
+  return spec_total_energy<KEY>(SpecLds{lat, offp, vex, adj}, g, geo.n_atoms, S, inverse_of(S), ebuf);
+}
+
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_wl_energies_spec(const WlArgs *__restrict__ args, double *E) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const WlArgs &A = args[blockIdx.x];
+  const double e = walker_energy<KEY>(A.g, A.compact, A.off, A.vex, smem);
+  if (threadIdx.x == 0) E[blockIdx.x] = e;
+}
+
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_ns_energies_spec(const NsArgs *__restrict__ args) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const NsArgs &A = args[blockIdx.y];
+  const int w = blockIdx.x;
+  if (w >= A.n_walkers) return;
+  const double e = walker_energy<KEY>(A.g, A.walkers + (size_t)A.g.compact_bytes * w, A.off, A.vex, smem);
+  if (threadIdx.x == 0) A.E[w] = e + A.rnde[w] * (double)1e-8f;
 }
 
 // The exchange decisions, one wavefront for the whole walker set (a few
@@ -718,7 +1319,29 @@ namespace {
 const void *wl_sweeps_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_wl_sweeps, key) }
 const void *ns_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_ns, key) }
 const void *wl_enter_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_wl_enter, key) }
+const void *wl_sweeps_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_wl_sweeps_spec, key) }
+const void *ns_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_ns_spec, key) }
+const void *wl_energies_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_wl_energies_spec, key) }
+const void *ns_energies_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_ns_energies_spec, key) }
+
+hipError_t launch_dynamic(const void *fn, dim3 grid, int threads, void **kargs, size_t lds, hipStream_t s) {
+  if (!fn) return hipErrorInvalidValue;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  return hipLaunchKernel(fn, grid, dim3(threads), kargs, lds, s);
+}
 }  // namespace
+
+size_t ns_spec_lds_bytes(const Geo &g, int n_walkers) {
+  return spec_table_bytes(g) + spec_ring_bytes() + spec_align(sizeof(double) * (size_t)n_walkers);
+}
+
+size_t wl_spec_lds_bytes(const Geo &g, int bins, int window_bins) {
+  return spec_table_bytes(g) + spec_ring_bytes() + spec_align(sizeof(double) * (size_t)bins) +
+         spec_align(sizeof(double) * (size_t)window_bins) + spec_energy_bytes();
+}
+
+size_t energies_spec_lds_bytes(const Geo &g) { return spec_table_bytes(g) + spec_energy_bytes(); }
 
 size_t ns_lds_bytes(const Geo &g, int n_walkers) {
   return seq_geo_region((size_t)((g.lds_bytes + 15) & ~15) + 624 * 4 + kSumBufBytes +
@@ -726,19 +1349,14 @@ size_t ns_lds_bytes(const Geo &g, int n_walkers) {
                         sizeof(int32_t) * g.nsub * g.z);
 }
 
-hipError_t launch_ns(const NsArgs *args_dev, int n, size_t lds, int max_walkers, size_t lds_energies,
-                     hipStream_t s, int key) {
-  hipError_t e = hipFuncSetAttribute((const void *)k_ns_energies,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_energies);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_ns_energies, dim3(max_walkers, n), dim3(64), lds_energies, s, args_dev);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const void *fn = ns_kernel(key);
-  e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+hipError_t launch_ns(const NsArgs *args_dev, int n, const SeqPick &pick, int max_walkers, const SeqPick &energies,
+                     hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  return hipLaunchKernel(fn, dim3(n), dim3(64), kargs, lds, s);
+  hipError_t e = launch_dynamic(energies.spec ? ns_energies_spec_kernel(energies.key) : (const void *)k_ns_energies,
+                                dim3(max_walkers, n), energies.spec ? kSpecThreads : 64, kargs, energies.bytes(), s);
+  if (e != hipSuccess) return e;
+  return launch_dynamic(pick.spec ? ns_spec_kernel(pick.key) : ns_kernel(pick.key), dim3(n),
+                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
 }
 
 size_t ns_energies_lds_bytes(const Geo &g) {
@@ -752,12 +1370,10 @@ size_t wl_lds_bytes(const Geo &g, int bins, int window_bins) {
                         sizeof(double) * (size_t)(2 * bins + 1 + window_bins) + sizeof(int32_t) * g.nsub * g.z);
 }
 
-hipError_t launch_wl_sweeps(const WlArgs *args_dev, int n, size_t lds, hipStream_t s, int key) {
-  const void *fn = wl_sweeps_kernel(key);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+hipError_t launch_wl_sweeps(const WlArgs *args_dev, int n, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  return hipLaunchKernel(fn, dim3(n), dim3(64), kargs, lds, s);
+  return launch_dynamic(pick.spec ? wl_sweeps_spec_kernel(pick.key) : wl_sweeps_kernel(pick.key), dim3(n),
+                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
 }
 
 hipError_t launch_wl_average(double *lng, double *hist, int n_windows, int wpw, int bins,
@@ -768,12 +1384,10 @@ hipError_t launch_wl_average(double *lng, double *hist, int n_windows, int wpw, 
   return hipGetLastError();
 }
 
-hipError_t launch_wl_energies(const WlArgs *args_dev, int n, double *E, size_t lds, hipStream_t s) {
-  hipError_t e = hipFuncSetAttribute((const void *)k_wl_energies,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_wl_energies, dim3(n), dim3(64), lds, s, args_dev, E);
-  return hipGetLastError();
+hipError_t launch_wl_energies(const WlArgs *args_dev, int n, double *E, const SeqPick &pick, hipStream_t s) {
+  void *kargs[] = {(void *)&args_dev, (void *)&E};
+  return launch_dynamic(pick.spec ? wl_energies_spec_kernel(pick.key) : (const void *)k_wl_energies, dim3(n),
+                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
 }
 
 size_t wl_exchange_lds_bytes(int W, int wpw) {
