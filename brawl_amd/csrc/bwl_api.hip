@@ -334,8 +334,11 @@ int bwl_mc_steps(bwl_ctx *c, double beta, int32_t nbr_swap, int64_t n_trials, in
   if (n_trials < 0) return fail(BWL_ERR_ARG, "negative trial count");
   if (energies && sample_every <= 0) return fail(BWL_ERR_ARG, "sample_every must be positive");
   const Geo &g = c->g;
-  if (seq_lds_bytes(g) > (size_t)lds_limit())
-    return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
+  SeqPick pick;
+  pick.add(g, seq_lds_bytes(g), seq_spec_lds_bytes(g));
+  const int limit = lds_limit();
+  if (pick.lds > (size_t)limit) return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
+  pick.settle(limit);
   if (2 * g.R > 64) return fail(BWL_ERR_UNSUPPORTED, "too many shells");
   // the MT state must be initialised (mti == 625 means "seed with 5489")
   if (c->mt.mti == 625) c->mt.seed(5489u);
@@ -360,7 +363,7 @@ int bwl_mc_steps(bwl_ctx *c, double beta, int32_t nbr_swap, int64_t n_trials, in
   int32_t mti = c->mt.mti;
   HIP_OK(hipMemcpyAsync(a.mt, c->mt.mt, 624 * 4, hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(a.mt_index, &mti, 4, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(launch_metro_seq(a, c->stream));
+  HIP_OK(launch_metro_seq(a, pick, c->stream));
   long long acc = 0;
   HIP_OK(hipMemcpyAsync(c->mt.mt, a.mt, 624 * 4, hipMemcpyDeviceToHost, c->stream));
   HIP_OK(hipMemcpyAsync(&mti, a.mt_index, 4, hipMemcpyDeviceToHost, c->stream));
@@ -380,19 +383,18 @@ int bwl_mc_steps_batch(int32_t n, bwl_ctx *const *ctxs, const double *beta, int3
   if (n < 1 || !ctxs || !beta) return fail(BWL_ERR_ARG, "null argument or empty batch");
   if (n_trials < 0) return fail(BWL_ERR_ARG, "negative trial count");
   if (energies && sample_every <= 0) return fail(BWL_ERR_ARG, "sample_every must be positive");
-  size_t lds = 0;
-  int key = 0;
+  SeqPick pick;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
     int rc = check_ctx(c, true);
     if (rc) return rc;
     if (c->device != ctxs[0]->device) return fail(BWL_ERR_ARG, "all chains of a batch must be on one device");
     if (2 * c->g.R > 64) return fail(BWL_ERR_UNSUPPORTED, "too many shells");
-    lds = std::max(lds, seq_lds_bytes(c->g));
-    const int k = pair_sum_key(c->g.lattice, c->g.R);
-    key = i == 0 ? k : (k == key ? key : -1);
+    pick.add(c->g, seq_lds_bytes(c->g), seq_spec_lds_bytes(c->g));
   }
-  if (lds > (size_t)lds_limit()) return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
+  const int limit = lds_limit();
+  if (pick.lds > (size_t)limit) return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
+  pick.settle(limit);
   HIP_OK(hipSetDevice(ctxs[0]->device));
   // per chain: MT state, index, accepted count, sampled energies
   const long long n_samples = energies ? n_trials / sample_every : 0;
@@ -430,7 +432,7 @@ int bwl_mc_steps_batch(int32_t n, bwl_ctx *const *ctxs, const double *beta, int3
   HIP_OK(hipMemcpyAsync(base, args.data(), sizeof(SeqArgs) * (size_t)n, hipMemcpyHostToDevice, s));
   HIP_OK(hipMemcpyAsync(base + args_bytes, host.data(), host.size(), hipMemcpyHostToDevice, s));
   HIP_OK(hipEventRecord(ctxs[0]->ev0, s));
-  HIP_OK(launch_metro_seq_batch((const SeqArgs *)base, n, lds, s, key));
+  HIP_OK(launch_metro_seq_batch((const SeqArgs *)base, n, pick, s));
   HIP_OK(hipEventRecord(ctxs[0]->ev1, s));
   HIP_OK(hipMemcpyAsync(host.data(), base + args_bytes, host.size(), hipMemcpyDeviceToHost, s));
   HIP_OK(hipStreamSynchronize(s));

@@ -180,15 +180,48 @@ hipError_t launch_histogram(const HistArgs *args_dev, int n, const Geo &g_max, i
                             hipStream_t s);
 size_t site_lds_bytes(const Geo &g);
 hipError_t launch_site_energy(const SiteArgs &a, hipStream_t s);
+// The kernel of a launch of sequential chains and its LDS, from its members.
+// key: the pair-sum variant they share (pair_sum_key), -1 if they differ.
+// spec: the kernel in speculative batches (bwl_spec.h), for launches whose
+// members share a key and can all use it with the LDS there is (it takes
+// about 13 KB more).  It was faster on every lattice it accepts (a walk of
+// nested sampling, quinary fcc 6^3, 4 shells: 0.61 against 1.31 us per trial;
+// a Wang-Landau walker, bcc 16^3, 2 shells: 0.37 against 1.22 us; bit-exact
+// Metropolis, fcc 8^3, 2 shells: 0.25 against 0.81 us); the kernels of one
+// trial at a time serve the rest: more than 4 shells, boxes as short as the
+// interaction range, launches that mix lattices.
+struct SeqPick {
+  int key = -2;  // no member yet
+  bool spec = true;
+  size_t lds = 0, lds_spec = 0;
+  void add(const Geo &g, size_t lds_one, size_t lds_batches) {
+    const int k = pair_sum_key(g.lattice, g.R);
+    key = key == -2 || key == k ? k : -1;
+    spec = spec && spec_ok(g);
+    lds = lds_one > lds ? lds_one : lds;
+    lds_spec = lds_batches > lds_spec ? lds_batches : lds_spec;
+  }
+  void settle(int limit) { spec = spec && key > 0 && lds_spec <= (size_t)limit; }
+  size_t bytes() const { return spec ? lds_spec : lds; }
+};
+
+// Launches `fn` with `lds` bytes of dynamic LDS.
+inline hipError_t launch_dynamic(const void *fn, dim3 grid, int threads, void **kargs, size_t lds, hipStream_t s) {
+  if (!fn) return hipErrorInvalidValue;
+  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  return hipLaunchKernel(fn, grid, dim3(threads), kargs, lds, s);
+}
+
 size_t seq_lds_bytes(const Geo &g);
-hipError_t launch_metro_seq(const SeqArgs &a, hipStream_t s);
+size_t seq_spec_lds_bytes(const Geo &g);
+hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s);
 hipError_t launch_draw_sites(const DrawArgs &a, hipStream_t s);
 // Sets n 64-bit words to zero with a kernel (no memset node in a captured
 // graph).
 hipError_t launch_zero_i64(long long *p, int n, hipStream_t s);
-// n chains (args_dev[0..n)), one wavefront each; key as for launch_wl_sweeps
-hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, size_t lds, hipStream_t s,
-                                  int key);
+// n chains (args_dev[0..n)), one workgroup each
+hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, const SeqPick &pick, hipStream_t s);
 size_t par_lds_bytes(const Geo &g, const NatGeo *nat, int threads);
 // Block size limit of the parallel-sampler kernels: the natural-layout
 // kernels with compile-time neighbour offsets and 32-bit count words run 16
@@ -208,30 +241,6 @@ bool par_specialised(const Geo &g);
 const void *par_fixed_kernel(int lattice, int R, int words);
 hipError_t launch_metro_par_fn(const void *fn, const ParArgs *args_dev, int n_chains, size_t lds,
                                int threads, hipStream_t s);
-
-// The kernel of a launch of sequential chains and its LDS, from its members.
-// key: the pair-sum variant they share (pair_sum_key), -1 if they differ.
-// spec: the kernel in speculative batches (bwl_spec.h), for launches whose
-// members share a key and can all use it with the LDS there is (it takes
-// about 13 KB more).  It was faster on every lattice it accepts (a walk of
-// nested sampling, quinary fcc 6^3, 4 shells: 0.61 against 1.31 us per trial;
-// a Wang-Landau walker, bcc 16^3, 2 shells: 0.37 against 1.22 us); the kernels of one
-// trial at a time serve the rest: more than 4 shells, boxes as short as the
-// interaction range, launches that mix lattices.
-struct SeqPick {
-  int key = -2;  // no member yet
-  bool spec = true;
-  size_t lds = 0, lds_spec = 0;
-  void add(const Geo &g, size_t lds_one, size_t lds_batches) {
-    const int k = pair_sum_key(g.lattice, g.R);
-    key = key == -2 || key == k ? k : -1;
-    spec = spec && spec_ok(g);
-    lds = lds_one > lds ? lds_one : lds;
-    lds_spec = lds_batches > lds_spec ? lds_batches : lds_spec;
-  }
-  void settle(int limit) { spec = spec && key > 0 && lds_spec <= (size_t)limit; }
-  size_t bytes() const { return spec ? lds_spec : lds; }
-};
 
 size_t ns_lds_bytes(const Geo &g, int n_walkers);
 size_t ns_spec_lds_bytes(const Geo &g, int n_walkers);

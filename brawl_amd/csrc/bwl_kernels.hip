@@ -11,7 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bwl_kernels.h"
-#include "bwl_seq.h"
+#include "bwl_spec.h"
 
 namespace bwl {
 
@@ -229,6 +229,124 @@ __device__ __forceinline__ void metro_seq_run(const SeqArgs &A, uint8_t *smem) {
 }
 
 // ------------------------------------------------------------------
+// The same in speculative batches (bwl_spec.h).  A trial draws its sites'
+// numbers and one more when the swap would raise the energy, so where the
+// next trial starts is known only with the energy: every lane takes the trial
+// that would start at its own place in the stream (64 places), forms its
+// energy change and its decision on the lattice as it is, and the batch is
+// the chain of 8 trials found by hopping from place to place, cut at the
+// first that an accepted swap before it reaches.
+// ------------------------------------------------------------------
+template <int KEY>
+__device__ __forceinline__ void metro_seq_spec_run(const SeqArgs &A, uint8_t *smem) {
+  using D = SpecDims<KEY>;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = wave_uniform(tid >> 6);
+  const SeqGeo g = seq_geo(A.g);
+  const int S = g.S, n_atoms = A.g.n_atoms;
+  const uint32_t inv_S = inverse_of(S);
+  uint8_t *p = smem;
+  auto take = [&](size_t bytes) {
+    uint8_t *at = p;
+    p += (bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  int8_t *lat = (int8_t *)take(A.g.lds_bytes);
+  uint32_t *raw = (uint32_t *)take(4 * 624);
+  uint32_t *tem = (uint32_t *)take(4 * kRingWords);
+  uint2 *rsite = (uint2 *)take(8 * kRingWords);
+  volatile int32_t *cmd = (volatile int32_t *)take(16);
+  double *vex = (double *)take(sizeof(double) * S * S * D::R);
+  double *ebuf = (double *)take(sizeof(double) * 2 * kEnergyChunk);
+  int32_t *offp = (int32_t *)take(4 * D::NSUB * D::R * D::ML);
+  uint8_t *adj = take(D::TS * D::TS * D::TS);
+  for (int i = tid; i < 624; i += kSpecThreads) raw[i] = A.mt[i];
+  for (int i = tid; i < S * S * D::R; i += kSpecThreads) vex[i] = A.vex[i];
+  stage_spec_tables<KEY>(offp, adj, A.off);
+  stage_codes(lat, A.compact, g, D::NSUB, S);
+  __syncthreads();
+  ring_start<D::LAT>(g, raw, tem, rsite);
+  const SpecLds L{lat, offp, vex, adj};
+  if (wave != 0) {
+    spec_helper<D::LAT>(g, raw, tem, rsite, cmd,
+                        [&](int) { (void)spec_total_energy<KEY>(L, g, n_atoms, S, inv_S, ebuf); });
+  } else {
+    MtRing ring{raw, tem, rsite, cmd, 0, wave_uniform(A.mt_index[0]), false};
+    const int trial = lane >> 3, w = (lane >> 2) & 1;
+    const bool nbr_swap = A.nbr_swap != 0;
+    const int drawn = nbr_swap ? 4 : 6;  // by a trial's sites
+    const bool sampling = A.energies != nullptr && A.sample_every > 0;
+    const double beta = A.beta;
+    long long left = A.n_trials, to_sample = A.sample_every, sample_k = 0, accepted = 0;
+    while (left > 0) {
+      ring_ensure(ring, 64 + 10);
+      const uint2 s1 = *ring_at(ring, rsite, lane);
+      const SiteXYZ sa = unpack_xyz(s1.x);
+      uint2 s2;
+      if (nbr_swap) {
+        const SiteXYZ sn = nbr_of_draw(g, sa, *ring_at(ring, tem, lane + 3));
+        s2 = make_uint2(pack_xyz(sn), (uint32_t)spec_addr<D::LAT>(g, sn));
+      } else {
+        s2 = *ring_at(ring, rsite, lane + 3);
+      }
+      const uint32_t ru = *ring_at(ring, tem, lane + drawn);
+      const SiteXYZ sb = unpack_xyz(s2.x);
+      const int ca = lat[s1.y], cb = lat[s2.y];
+      const bool same = ca == cb;
+      double ba, aa, bb, ab;
+      spec_site_energies<KEY>(L, g, S, inv_S, sa, sb, (int)s1.y, ca, cb, ba, aa);
+      spec_site_energies<KEY>(L, g, S, inv_S, sb, sa, (int)s2.y, cb, ca, bb, ab);
+      const double de = (aa + ab) - (ba + bb);
+      // equal species are accepted without a draw (metropolis.F90:774-777)
+      const bool draws = !same && !(de < 0.0);
+      bool acc = true;
+      if (draws) acc = lt_exp_dev((double)ru * (1.0 / 4294967296.0), -(beta * de));
+      const int next = lane + drawn + (draws ? 1 : 0);
+      // the 8 trials' places: at most 49, so every hop stays in sight
+      int my = 0, at = 0;
+#pragma unroll
+      for (int t = 1; t < kBatch; ++t) {
+        at = __builtin_amdgcn_readlane(next, at);
+        my = trial >= t ? at : my;
+      }
+      const uint32_t pa = (uint32_t)__shfl((int)s1.x, my), pb = (uint32_t)__shfl((int)s2.x, my);
+      // code of A, code of B, accepted, exchanged
+      const int what = __shfl(ca | (cb << 8) | (acc ? 1 << 16 : 0) | (acc && !same ? 1 << 17 : 0), my);
+      const bool moved = (what >> 17) & 1;
+      const bool reach = batch_conflict(g, D::RC, pa, pb);  // (on all lanes: it reads other lanes' sites)
+      unsigned long long conf = __ballot(reach && moved && trial < (lane & 7));
+      int n = kBatch;
+      conf |= conf >> 32;
+      conf |= conf >> 16;
+      conf |= conf >> 8;
+      if (conf & 0xffu) n = __ffs((int)(conf & 0xffu)) - 1;
+      n = n < left ? n : (int)left;
+      if (sampling && n > to_sample) n = (int)to_sample;
+      const unsigned long long upto = n < kBatch ? (1ull << (8 * n)) - 1ull : ~0ull;
+      accepted += __popcll(__ballot((what >> 16) & 1) & upto & 0x0101010101010101ull);
+      batch_write<D::LAT>(lat, g, moved && trial < n, unpack_xyz(w ? pb : pa), w ? what & 0xff : (what >> 8) & 0xff);
+      ring.q = wave_uniform(ring.q + __shfl(next, __builtin_amdgcn_readlane(my, 8 * (n - 1))));
+      left -= n;
+      if (sampling) {
+        to_sample -= n;
+        if (to_sample == 0) {
+          to_sample = A.sample_every;
+          spec_command(ring, kCmdEnergy);
+          const double e = spec_total_energy<KEY>(L, g, n_atoms, S, inv_S, ebuf);
+          if (lane == 0) A.energies[sample_k] = e;
+          sample_k++;
+        }
+      }
+    }
+    spec_command(ring, kCmdExit);
+    ring_finish(ring, A.mt, A.mt_index);
+    if (lane == 0) A.accepted[0] = accepted;
+  }
+  __syncthreads();
+  unstage_codes(lat, A.compact, g, D::NSUB, inv_S);
+}
+
+// ------------------------------------------------------------------
 // Proposal draws (rdm_site, rdm_nbr, mc_select) from the reference stream,
 // one wavefront (the MT19937 twist is wavefront-wide); lane 0 writes.
 // ------------------------------------------------------------------
@@ -367,28 +485,38 @@ size_t seq_lds_bytes(const Geo &g) {
          64;
 }
 
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_metro_seq_spec(SeqArgs A) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  metro_seq_spec_run<KEY>(A, smem);
+}
+
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_metro_seq_spec_batch(const SeqArgs *__restrict__ args) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  metro_seq_spec_run<KEY>(args[blockIdx.x], smem);
+}
+
 namespace {
 const void *metro_seq_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_metro_seq, key) }
 const void *metro_seq_batch_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_metro_seq_batch, key) }
+const void *metro_seq_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec, key) }
+const void *metro_seq_spec_batch_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec_batch, key) }
 }  // namespace
 
-hipError_t launch_metro_seq(const SeqArgs &a, hipStream_t s) {
-  size_t lds = seq_lds_bytes(a.g);
-  const void *fn = metro_seq_kernel(pair_sum_key(a.g.lattice, a.g.R));
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+size_t seq_spec_lds_bytes(const Geo &g) { return spec_table_bytes(g) + spec_ring_bytes() + spec_energy_bytes(); }
+
+hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s) {
   SeqArgs arg = a;
   void *kargs[] = {(void *)&arg};
-  return hipLaunchKernel(fn, dim3(1), dim3(64), kargs, lds, s);
+  return launch_dynamic(pick.spec ? metro_seq_spec_kernel(pick.key) : metro_seq_kernel(pick.key), dim3(1),
+                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
 }
 
-hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, size_t lds, hipStream_t s,
-                                  int key) {
-  const void *fn = metro_seq_batch_kernel(key);
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
+hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  return hipLaunchKernel(fn, dim3(n), dim3(64), kargs, lds, s);
+  return launch_dynamic(pick.spec ? metro_seq_spec_batch_kernel(pick.key) : metro_seq_batch_kernel(pick.key), dim3(n),
+                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
 }
 
 // ------------------------------------------------------------------

@@ -1324,12 +1324,6 @@ const void *ns_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_ns_spec, key) }
 const void *wl_energies_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_wl_energies_spec, key) }
 const void *ns_energies_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_ns_energies_spec, key) }
 
-hipError_t launch_dynamic(const void *fn, dim3 grid, int threads, void **kargs, size_t lds, hipStream_t s) {
-  if (!fn) return hipErrorInvalidValue;
-  const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  return hipLaunchKernel(fn, grid, dim3(threads), kargs, lds, s);
-}
 }  // namespace
 
 size_t ns_spec_lds_bytes(const Geo &g, int n_walkers) {

@@ -90,3 +90,29 @@ def test_wang_landau_sweeps(hip, oracle, lat, n, S, R, nbr_swap):
         assert np.array_equal(wl.get_walker(k), cfg)
         _same_state(wl.genrand_state(k), gen)
     wl.close()
+
+
+@pytest.mark.parametrize("nbr_swap", [False, True])
+@pytest.mark.parametrize("temp", [200.0, 3000.0])
+@pytest.mark.parametrize("lat,n,S,R", SHAPES)
+def test_sequential_metropolis(hip, oracle, lat, n, S, R, temp, nbr_swap):
+    """Uneven sampling, so that batches end at samples and at the run's end;
+    the second call starts in the middle of the stream's block."""
+    v, ref, counts = _case(hip, oracle, lat, n, S, R, False)
+    gen = oracle.Generator(77)
+    cfg = ref.initial_setup(gen, species_numbers=counts)
+    beta = hip.beta_of(temp)
+    with hip.Lattice(lat, n, v) as L:
+        L.set_config(cfg)
+        L.set_genrand_state(*gen.state_arrays())
+        for trials, every in ((1, 0), (1500, 37)):
+            acc, energies = L.mc_steps(beta, trials, nbr_swap=nbr_swap, sample_every=every)
+            acc_ref, e_ref = 0, []
+            for t in range(1, trials + 1):
+                acc_ref += ref.mc_step(cfg, beta, gen, nbr_swap=nbr_swap)
+                if every and t % every == 0:
+                    e_ref.append(ref.total_energy(cfg))
+            assert acc == acc_ref
+            assert energies is None or np.array_equal(energies, e_ref)
+            assert np.array_equal(L.get_config(), cfg)
+            _same_state(L.genrand_state(), gen)
