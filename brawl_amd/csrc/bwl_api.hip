@@ -1,8 +1,10 @@
 // bwl_api.hip -- the C-ABI (include/brawl_hip.h) over the gfx950 kernels.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -508,23 +510,8 @@ int bwl_metropolis_anneal_rho(bwl_ctx *c, const bwl_anneal_params *p, double *en
     return fail(BWL_ERR_ARG, "null argument");
   if (p->asro_every < 1) return fail(BWL_ERR_ARG, "asro_every must be positive");
   bwl_ctx *cs[1] = {c};
-  AnnealPlan P;
-  int rc = anneal_plan(1, cs, p, P);
-  if (rc) return rc;
-  DevBuf scratch;
-  if (hipMalloc(&scratch.p, P.scratch_bytes) != hipSuccess)
-    return fail(BWL_ERR_NOMEM, "device allocation failed");
-  HIP_OK(hipEventRecord(c->ev0, c->stream));
-  rc = anneal_upload(P, (char *)scratch.p, c->stream);
-  if (rc) return rc;
-  rc = anneal_launch(P, &c->stream);
-  if (rc) return rc;
-  HIP_OK(hipEventRecord(c->ev1, c->stream));
-  HIP_OK(hipStreamSynchronize(c->stream));
-  float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
   double *e[1] = {energies_of_T}, *cv[1] = {C_of_T}, *ac[1] = {acceptance_of_T}, *rh[1] = {rho_of_T};
-  return anneal_collect(P, cs, e, cv, ac, stats, ms, c->stream, rh);
+  return anneal_run(1, cs, p, e, cv, ac, stats, nullptr, rh);
 }
 
 }  // extern "C"
@@ -645,9 +632,84 @@ int anneal_kernel(const Geo &g, ParPlan &plan, NatGeo &nat, const void *&fn, int
   return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
 }
 
-int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P) {
+// Estimated time of a chain's rounds (us), undivided and divided: fitted to
+// runs of 19 shapes with 1-24 chunks of 64 pairs a round and 8-54 gathers a
+// site (z); a divided round takes 2.2-2.6 us whatever its size.
+static double undivided_us(const AnnealPlan::Item &it) {
+  return it.rounds * (0.7 + 0.135 * sqrt((double)it.chunks * (double)it.a.g.z));
+}
+static double divided_us(const AnnealPlan::Item &it) { return it.rounds * 2.4; }
+
+// Divides the longest chains over workgroups (a.parts, lane of their items)
+// where the device would end the whole batch sooner than such a chain alone.
+//
+// A chain is worth dividing from chunks * z = 192 on: 1.16x at 216 (fcc 16^3,
+// 4 shells), 1.27x at 196 (bcc 24^3, 2), 1.67x at 588 (fcc 24^3, 3), 2.1x at
+// 1200 (bcc 32^3, 4), against 0.99x at 144 (fcc 20^3, 2) and 1.00x at 150
+// (bcc 16^3, 4).  One wavefront per SIMD and part (4 half rows) is best where
+// the CUs are there (bcc 32^3: 16 parts 5.1 ms, 8 parts 5.7; fcc 24^3: 7
+// parts 7.4, 4 parts 7.7), else two.
+//
+// The parts of a chain go to one XCD (lane), which has n_cu / 8 CUs: as many
+// as other chains of this and other calls leave free.
+static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu, int lim) {
+  const int n = (int)P.items.size();
+  const int cap = std::max(n_cu / 8 - (n + 7) / 8, n_cu / 16);
+  int lanes[8];
+  bool any = false;
+  for (int x = 0; x < 8; ++x) {
+    lanes[x] = std::min(free_parts.parts[x], cap);
+    any = any || lanes[x] >= 2;
+  }
+  if (!any) return;
+  double load = 0.0;  // CU time
+  auto share = [&](const AnnealPlan::Item &it) {  // of a CU, undivided
+    return std::min(1.0, std::max((double)it.lds / (double)lim, (double)it.threads / (double)kMaxNatThreads));
+  };
+  std::vector<AnnealPlan::Item *> by_time;
+  for (AnnealPlan::Item &it : P.items) {
+    load += undivided_us(it) * share(it);
+    by_time.push_back(&it);
+  }
+  std::stable_sort(by_time.begin(), by_time.end(), [](const AnnealPlan::Item *x, const AnnealPlan::Item *y) {
+    return undivided_us(*x) > undivided_us(*y);
+  });
+  auto divide = [&](AnnealPlan::Item &it) {
+    if (!it.split_fn || it.chunks * it.a.g.z < 192 || par_split_lds_bytes(it.a.g, it.a.nat) > (size_t)lim) return false;
+    const int rows = it.threads / 64;
+    for (int units = 4; units <= 8; units += 4) {
+      const int rows_each = std::max(1, units / (2 * it.passes));
+      const int parts = (rows + rows_each - 1) / rows_each;
+      if (!par_split_fits(it.a.nat, it.threads, parts, it.passes)) continue;
+      const double load_then = load + parts * divided_us(it) - undivided_us(it) * share(it);
+      int to = 0;
+      for (int x = 1; x < 8; ++x)
+        if (lanes[x] > lanes[to]) to = x;
+      if (parts > lanes[to] || load_then > n_cu * undivided_us(it)) continue;
+      load = load_then;
+      lanes[to] -= parts;
+      it.a.parts = parts;
+      it.lane = to;
+      return true;
+    }
+    return false;
+  };
+  for (AnnealPlan::Item *it : by_time)
+    if (!divide(*it)) break;
+  // a division that leaves the batch waiting for chains as long is undone
+  double longest = 0.0;
+  for (const AnnealPlan::Item &it : P.items)
+    longest = std::max(longest, it.a.parts > 1 ? divided_us(it) : undivided_us(it));
+  const bool gains = longest < 0.95 * undivided_us(*by_time[0]);
+  for (AnnealPlan::Item &it : P.items)
+    if (!gains || undivided_us(it) <= longest) it.a.parts = 1;
+}
+
+int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P,
+                const SplitLanes *split) {
   P.items.assign((size_t)n, AnnealPlan::Item());
   P.groups.clear();
+  P.split = SplitLanes();
   size_t total = 0;
   const int lim = lds_limit();
   for (int i = 0; i < n; ++i) {
@@ -681,6 +743,16 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
     }
     it.threads = threads;
     it.lds = lds;
+    int max_pairs = 0;
+    for (const RoundVar &v : it.plan.vars) max_pairs = std::max(max_pairs, (int)v.n2);
+    it.chunks = (max_pairs + 63) / 64;
+    it.passes = (max_pairs + threads - 1) / threads;
+    it.rounds = (double)p->T_steps * (double)(p->n_sweeps + p->burn_in_sweeps) * (double)g.n_atoms / (double)max_pairs;
+    // (a layout other than the rule's, where the caller asked for one, has
+    // run-time neighbour offsets or none in lattice coordinates)
+    if (natural) it.split_fn = par_split_kernel(g, it.fn == par_fixed_kernel(g.lattice, g.R, par_count_words(g, true)));
+    if (natural && it.split_fn && it.fn != par_fixed_kernel(g.lattice, g.R, par_count_words(g, true)) && !par_specialised(g))
+      it.split_fn = nullptr;
     ParArgs &a = it.a;
     memset(&a, 0, sizeof(a));
     a.g = g;
@@ -723,6 +795,23 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
     it.off_rho = total;
     total += 256 * ((it.rho_n * sizeof(double) + 255) / 256);
     it.work = (double)g.n_atoms * (double)p->T_steps * (double)(p->n_sweeps + p->burn_in_sweeps);
+    a.parts = 1;
+    a.passes = it.passes;
+  }
+  int n_cu = 0;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctxs[0]->device) != hipSuccess) n_cu = 0;
+  if (split) divide_chains(P, *split, n_cu, lim);
+  int blocks = 0;
+  for (AnnealPlan::Item &it : P.items) {
+    it.mail_n = it.a.parts > 1 ? par_split_mail_words(it.a.g, it.threads, it.a.parts) : 0;
+    it.off_mail = total;
+    total += 256 * ((it.mail_n * sizeof(unsigned long long) + 255) / 256);
+    if (it.a.parts > 1) {
+      it.fn = it.split_fn;
+      it.lds = par_split_lds_bytes(it.a.g, it.a.nat);
+      P.split.parts[it.lane] += it.a.parts;
+    }
+    blocks += it.a.parts;
   }
   // group chains that run the same kernel (one launch each, the block size
   // of its largest member; each chain loops over its own pairs with the
@@ -732,13 +821,15 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
   for (int i = 0; i < n; ++i) order[(size_t)i] = i;
   std::sort(order.begin(), order.end(), [&](int x, int y) {
     const AnnealPlan::Item &A = P.items[(size_t)x], &B = P.items[(size_t)y];
+    // divided chains first: all of their workgroups have to be on the device
+    if ((A.a.parts > 1) != (B.a.parts > 1)) return A.a.parts > 1;
     if (A.fn != B.fn) return A.fn < B.fn;
     return A.work > B.work;
   });
   for (int i : order) {
     const AnnealPlan::Item &it = P.items[(size_t)i];
     if (P.groups.empty() || P.groups.back().fn != it.fn)
-      P.groups.push_back(AnnealPlan::Group{it.fn, it.threads, 0, {}, 0});
+      P.groups.push_back(AnnealPlan::Group{it.fn, it.threads, 0, {}, 0, it.a.parts > 1, {}, 0});
     AnnealPlan::Group &gr = P.groups.back();
     gr.members.push_back(i);
     if (it.threads > gr.threads) gr.threads = it.threads;
@@ -747,24 +838,35 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
   for (AnnealPlan::Group &gr : P.groups)
     for (int i : gr.members) {
       const AnnealPlan::Item &it = P.items[(size_t)i];
-      const size_t need = it.lds + sizeof(double) * (size_t)(gr.threads - it.threads) / 64;
+      const size_t need = it.lds + (gr.split ? 0 : sizeof(double) * (size_t)(gr.threads - it.threads) / 64);
       if (need > gr.lds) gr.lds = need;
     }
   // With no more chains than compute units, give every chain a CU of its
   // own: ask each block for more than half the LDS so no two share a CU
   // (the largest chains set the makespan; sharing a CU would halve them).
-  int n_cu = 0;
-  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctxs[0]->device) !=
-      hipSuccess)
-    n_cu = 0;
-  if (n_cu > 0 && n <= n_cu) {
-    const size_t exclusive = (size_t)lim / 2 + 1024;
-    for (AnnealPlan::Group &gr : P.groups)
+  const size_t exclusive = (size_t)lim / 2 + 1024;
+  for (AnnealPlan::Group &gr : P.groups)
+    if (gr.split || blocks <= n_cu)
       if (gr.lds < exclusive && exclusive <= (size_t)lim) gr.lds = exclusive;
-  }
   for (AnnealPlan::Group &gr : P.groups) {
     gr.off_args = total;
     total += 256 * ((sizeof(ParArgs) * gr.members.size() + 255) / 256);
+    // Workgroups go to the 8 XCDs in turn, so block b lands on XCD b mod 8:
+    // the parts of a chain take blocks of one residue.
+    if (gr.split) {
+      std::vector<int2> lane[8];
+      for (size_t k = 0; k < gr.members.size(); ++k) {
+        const AnnealPlan::Item &it = P.items[(size_t)gr.members[k]];
+        for (int p = 0; p < it.a.parts; ++p) lane[it.lane].push_back(make_int2((int)k, p));
+      }
+      size_t rows = 0;
+      for (const auto &l : lane) rows = std::max(rows, l.size());
+      gr.map.assign(8 * rows, make_int2(-1, 0));
+      for (size_t x = 0; x < 8; ++x)
+        for (size_t k = 0; k < lane[x].size(); ++k) gr.map[8 * k + x] = lane[x][k];
+      gr.off_map = total;
+      total += 256 * ((sizeof(int2) * gr.map.size() + 255) / 256);
+    }
   }
   P.scratch_bytes = total;
   return BWL_OK;
@@ -783,10 +885,12 @@ int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, bool zero_by_kernel)
     it.a.rho_of_T = it.rho_n ? (double *)(base + it.off_rho) : nullptr;
     HIP_OK(hipMemcpyAsync(base + it.off_muls, it.plan.muls.data(), it.plan.muls.size() * 4,
                           hipMemcpyHostToDevice, s));
+    it.a.mail = it.mail_n ? (unsigned long long *)(base + it.off_mail) : nullptr;
     if (zero_by_kernel)
-      HIP_OK(launch_zero_i64(it.a.counters, 3, s));
+      HIP_OK(launch_zero_i64(it.a.counters, 4, s));
     else
-      HIP_OK(hipMemsetAsync(it.a.counters, 0, 3 * sizeof(long long), s));
+      HIP_OK(hipMemsetAsync(it.a.counters, 0, 4 * sizeof(long long), s));
+    if (it.mail_n) HIP_OK(hipMemsetAsync(it.a.mail, 0, it.mail_n * sizeof(unsigned long long), s));
   }
   for (AnnealPlan::Group &gr : P.groups) {
     std::vector<ParArgs> host;
@@ -794,6 +898,8 @@ int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, bool zero_by_kernel)
     P.host_args.push_back(std::move(host));
     HIP_OK(hipMemcpyAsync(base + gr.off_args, P.host_args.back().data(),
                           sizeof(ParArgs) * P.host_args.back().size(), hipMemcpyHostToDevice, s));
+    if (gr.split)
+      HIP_OK(hipMemcpyAsync(base + gr.off_map, gr.map.data(), sizeof(int2) * gr.map.size(), hipMemcpyHostToDevice, s));
   }
   return BWL_OK;
 }
@@ -801,6 +907,11 @@ int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, bool zero_by_kernel)
 int anneal_launch(const AnnealPlan &P, const hipStream_t *streams) {
   for (size_t k = 0; k < P.groups.size(); ++k) {
     const AnnealPlan::Group &gr = P.groups[k];
+    if (gr.split) {
+      HIP_OK(launch_metro_split(gr.fn, (const ParArgs *)(P.base + gr.off_args), (const int2 *)(P.base + gr.off_map),
+                                (int)gr.map.size(), gr.lds, streams[k]));
+      continue;
+    }
     HIP_OK(launch_metro_par_fn(gr.fn, (const ParArgs *)(P.base + gr.off_args),
                                (int)gr.members.size(), gr.lds, gr.threads, streams[k]));
   }
@@ -809,16 +920,16 @@ int anneal_launch(const AnnealPlan &P, const hipStream_t *streams) {
 
 int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *energies_of_T,
                    double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats,
-                   double kernel_ms, hipStream_t s, double *const *rho_of_T) {
+                   double kernel_ms, hipStream_t s, double *const *rho_of_T, std::vector<int> *again) {
   const size_t n = P.items.size();
   std::vector<std::vector<double>> out(n);
-  std::vector<long long> cnt(3 * n);
+  std::vector<long long> cnt(4 * n);
   for (size_t i = 0; i < n; ++i) {
     const AnnealPlan::Item &it = P.items[i];
     out[i].resize(5 * it.T);
     HIP_OK(hipMemcpyAsync(out[i].data(), it.a.energies_of_T, 5 * it.T * sizeof(double),
                           hipMemcpyDeviceToHost, s));
-    HIP_OK(hipMemcpyAsync(&cnt[3 * i], it.a.counters, 3 * sizeof(long long), hipMemcpyDeviceToHost, s));
+    HIP_OK(hipMemcpyAsync(&cnt[4 * i], it.a.counters, 4 * sizeof(long long), hipMemcpyDeviceToHost, s));
     if (rho_of_T && rho_of_T[i] && it.rho_n)
       HIP_OK(hipMemcpyAsync(rho_of_T[i], it.a.rho_of_T, it.rho_n * sizeof(double),
                             hipMemcpyDeviceToHost, s));
@@ -826,13 +937,20 @@ int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *ene
   HIP_OK(hipStreamSynchronize(s));
   for (size_t i = 0; i < n; ++i) {
     const size_t T = P.items[i].T;
+    if (P.items[i].a.parts > 1 && cnt[4 * i + 3] == 0) {
+      // a divided chain whose parts did not all get onto the device in time:
+      // its configuration and stream are as they were
+      if (!again) return fail(BWL_ERR_DEVICE, "a divided chain was given up");
+      again->push_back((int)i);
+      continue;
+    }
     if (energies_of_T && energies_of_T[i]) memcpy(energies_of_T[i], out[i].data(), T * sizeof(double));
     if (C_of_T && C_of_T[i]) memcpy(C_of_T[i], out[i].data() + T, T * sizeof(double));
     if (acceptance_of_T && acceptance_of_T[i])
       memcpy(acceptance_of_T[i], out[i].data() + 2 * T, T * sizeof(double));
     if (stats) {
-      stats[i].trials = cnt[3 * i + 2];
-      stats[i].accepted = cnt[3 * i + 1];
+      stats[i].trials = cnt[4 * i + 2];
+      stats[i].accepted = cnt[4 * i + 1];
       stats[i].kernel_ms = kernel_ms;
       // largest difference between the carried energy and its recount over
       // the T steps, absolute (Ry) and relative to the recounted energy
@@ -845,7 +963,7 @@ int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *ene
       stats[i].e_drift_abs = da;
       stats[i].e_drift_rel = dr;
     }
-    ctxs[i]->phase = (unsigned long long)cnt[3 * i];
+    ctxs[i]->phase = (unsigned long long)cnt[4 * i];
   }
   return BWL_OK;
 }
@@ -858,13 +976,64 @@ int bwl_metropolis_anneal_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_annea
                                 double *const *energies_of_T, double *const *C_of_T,
                                 double *const *acceptance_of_T, bwl_run_stats *stats,
                                 double *makespan_ms) {
+  return anneal_run(n, ctxs, params, energies_of_T, C_of_T, acceptance_of_T, stats, makespan_ms, nullptr);
+}
+
+}  // extern "C"
+
+namespace {
+
+// The workgroups of divided chains on each of a device's XCDs, over all calls
+// in this process: the parts of a chain wait for each other, so together they
+// must not outnumber the CUs.  A call takes what is free, keeps what its plan
+// uses and gives it back when its launches have ended.
+constexpr int kMaxSplitDevices = 64;
+std::mutex g_split_mu;
+SplitLanes g_split_used[kMaxSplitDevices];
+
+struct SplitShare {
+  int device = -1;
+  SplitLanes held;
+  SplitShare(int dev, int n_cu) {
+    if (dev < 0 || dev >= kMaxSplitDevices) return;
+    std::lock_guard<std::mutex> lock(g_split_mu);
+    device = dev;
+    for (int x = 0; x < 8; ++x) {
+      held.parts[x] = std::max(0, n_cu / 8 - g_split_used[dev].parts[x]);
+      g_split_used[dev].parts[x] += held.parts[x];
+    }
+  }
+  void keep(const SplitLanes &used) {
+    if (device < 0) return;
+    std::lock_guard<std::mutex> lock(g_split_mu);
+    for (int x = 0; x < 8; ++x) g_split_used[device].parts[x] -= held.parts[x] - used.parts[x];
+    held = used;
+  }
+  ~SplitShare() { keep(SplitLanes()); }
+  SplitShare(const SplitShare &) = delete;
+  SplitShare &operator=(const SplitShare &) = delete;
+};
+
+}  // namespace
+
+namespace bwl {
+
+int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, double *const *energies_of_T,
+               double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats, double *makespan_ms,
+               double *const *rho_of_T, bool divide) {
   if (n < 1 || !ctxs || !params || !energies_of_T || !C_of_T || !acceptance_of_T)
     return fail(BWL_ERR_ARG, "null argument");
   for (int i = 0; i < n; ++i)
     if (!energies_of_T[i] || !C_of_T[i] || !acceptance_of_T[i]) return fail(BWL_ERR_ARG, "null output");
   AnnealPlan P;
-  int rc = anneal_plan(n, ctxs, params, P);
+  int n_cu = 0;
+  if (divide && ctxs[0] &&
+      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctxs[0]->device) != hipSuccess)
+    n_cu = 0;
+  SplitShare share(ctxs[0] ? ctxs[0]->device : -1, n_cu);
+  int rc = anneal_plan(n, ctxs, params, P, &share.held);
   if (rc) return rc;
+  share.keep(P.split);
   bwl_ctx *c0 = ctxs[0];
   DevBuf scratch;
   if (hipMalloc(&scratch.p, P.scratch_bytes) != hipSuccess)
@@ -908,7 +1077,30 @@ int bwl_metropolis_anneal_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_annea
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, c0->ev0, c0->ev1);
   if (makespan_ms) *makespan_ms = ms;
-  return anneal_collect(P, ctxs, energies_of_T, C_of_T, acceptance_of_T, stats, ms, c0->stream);
+  std::vector<int> again;
+  rc = anneal_collect(P, ctxs, energies_of_T, C_of_T, acceptance_of_T, stats, ms, c0->stream, rho_of_T, &again);
+  if (rc || again.empty()) return rc;
+  // chains whose division was given up run undivided, with the same results
+  std::vector<bwl_ctx *> cs;
+  std::vector<bwl_anneal_params> ps;
+  std::vector<double *> e, cv, ac, rh;
+  for (int i : again) {
+    cs.push_back(ctxs[i]);
+    ps.push_back(params[i]);
+    e.push_back(energies_of_T[i]);
+    cv.push_back(C_of_T[i]);
+    ac.push_back(acceptance_of_T[i]);
+    rh.push_back(rho_of_T ? rho_of_T[i] : nullptr);
+  }
+  std::vector<bwl_run_stats> st(again.size());
+  double more_ms = 0.0;
+  rc = anneal_run((int)again.size(), cs.data(), ps.data(), e.data(), cv.data(), ac.data(), st.data(), &more_ms,
+                  rho_of_T ? rh.data() : nullptr, false);
+  if (rc) return rc;
+  for (size_t k = 0; k < again.size(); ++k)
+    if (stats) stats[again[k]] = st[k];
+  if (makespan_ms) *makespan_ms = ms + more_ms;
+  return BWL_OK;
 }
 
-}  // extern "C"
+}  // namespace bwl

@@ -87,6 +87,11 @@ size_t ctx_device_bytes(const bwl_lattice_desc &d);
 int ctx_create_borrowed(const bwl_lattice_desc &d, const double *v_ex, char *mem, size_t bytes,
                         hipStream_t stream, bwl_ctx **out);
 
+// Workgroups of divided chains on each XCD of a device.
+struct SplitLanes {
+  int parts[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+};
+
 // A batch of anneals prepared on the host (anneal_plan), its arguments and
 // buffers placed in caller-provided device memory (anneal_upload), its
 // launches enqueued one group per stream (anneal_launch), and its outputs
@@ -100,6 +105,11 @@ struct AnnealPlan {
     ParArgs a;
     ParPlan plan;
     size_t T = 0, off_muls = 0, off_out = 0, off_cnt = 0, off_rho = 0, rho_n = 0;
+    size_t off_mail = 0, mail_n = 0;  // mailbox of a divided chain, in words
+    const void *split_fn = nullptr;   // kernel that can divide the chain, if any
+    int chunks = 0, passes = 0;       // most pairs of a round, in 64s and per thread
+    int lane = 0;                     // XCD of a divided chain's parts
+    double rounds = 0.0;              // rounds of the whole anneal, about
     double work = 0.0;
   };
   struct Group {
@@ -108,12 +118,16 @@ struct AnnealPlan {
     size_t lds;
     std::vector<int> members;
     size_t off_args;
+    bool split;                 // a divided group: block b runs map[b]
+    std::vector<int2> map;
+    size_t off_map;
   };
   std::vector<Item> items;
   std::vector<Group> groups;
   std::vector<std::vector<ParArgs>> host_args;  // kept alive until the uploads finish
   size_t scratch_bytes = 0;
   char *base = nullptr;
+  SplitLanes split;  // workgroups of its divided chains
 };
 // The parallel-sampler kernel variant, block size and LDS for a lattice:
 // layout 0 takes the first that fits of fixed pitch, own pitch, per
@@ -122,13 +136,22 @@ struct AnnealPlan {
 // 0 then takes the first layout that can run them).
 int anneal_kernel(const Geo &g, ParPlan &plan, NatGeo &nat, const void *&fn, int &threads,
                   size_t &lds, bool *natural = nullptr, int layout = 0, int threads_req = 0);
-int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P);
+// split: the workgroups that chains may be divided into (none: no chain is
+// divided); AnnealPlan::split says how many the divided chains take.
+int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P,
+                const SplitLanes *split = nullptr);
 // zero_by_kernel: clear the counters with a kernel instead of a memset
 int anneal_upload(AnnealPlan &P, char *scratch_dev, hipStream_t s, bool zero_by_kernel = false);
 int anneal_launch(const AnnealPlan &P, const hipStream_t *streams);
 int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *energies_of_T,
                    double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats,
-                   double kernel_ms, hipStream_t s, double *const *rho_of_T = nullptr);
+                   double kernel_ms, hipStream_t s, double *const *rho_of_T = nullptr,
+                   std::vector<int> *again = nullptr);
+// The whole call: plan (dividing chains over idle CUs), upload, launch, wait,
+// collect.
+int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, double *const *energies_of_T,
+               double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats, double *makespan_ms,
+               double *const *rho_of_T, bool divide = true);
 
 // Device buffer freed at scope exit.
 struct DevBuf {

@@ -84,7 +84,12 @@ struct ParArgs {
   double *e_trace;       // optional [T_steps][n_sweeps]
   int32_t asro_every;    // sampled sweeps between radial-density samples (0: none)
   double *rho_of_T;      // (S, S, R+1, T_steps) when asro_every > 0
-  long long *counters;   // [0] = next round counter, [1] += accepted, [2] += trials
+  long long *counters;   // [0] = next round counter, [1] += accepted, [2] += trials,
+                         // [3] = 1 when a divided chain is complete
+  // a chain divided over several workgroups (bwl_metro_split.hip)
+  int32_t parts;         // workgroups
+  int32_t passes;        // most pairs a thread has in a round
+  unsigned long long *mail;  // par_split_mail_words words, zeroed
 };
 
 // Nested sampling (nested_sampling.f90:45-206), one wavefront per run.
@@ -239,6 +244,16 @@ const void *par_kernel_for(const Geo &g, bool nat, bool fixed);
 bool par_specialised(const Geo &g);
 // the fixed-pitch kernel for (lattice, R, count words), nullptr if none
 const void *par_fixed_kernel(int lattice, int R, int words);
+// The kernel that runs a chain over several workgroups, nullptr if there is
+// none for the lattice in that layout; its LDS, its mailbox, whether a
+// division suits the kernel's shape, and its launch (block b runs part
+// map[b].y of chain map[b].x, or nothing when that is negative).
+const void *par_split_kernel(const Geo &g, bool fixed);
+size_t par_split_lds_bytes(const Geo &g, const NatGeo &nat);
+size_t par_split_mail_words(const Geo &g, int threads, int parts);
+bool par_split_fits(const NatGeo &nat, int threads, int parts, int passes);
+hipError_t launch_metro_split(const void *fn, const ParArgs *args_dev, const int2 *map_dev, int blocks, size_t lds,
+                              hipStream_t s);
 hipError_t launch_metro_par_fn(const void *fn, const ParArgs *args_dev, int n_chains, size_t lds,
                                int threads, hipStream_t s);
 

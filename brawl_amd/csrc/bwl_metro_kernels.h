@@ -562,6 +562,134 @@ __device__ __forceinline__ void asro_sample(const int8_t *lat, const ND N, const
   }
 }
 
+// dtab[alpha][beta][n][s<S1P]: (V(beta,s,n)-V(alpha,s,n)) - (same for
+// s=S-1) for s < S-1, zero beyond; the S-1 independent count differences
+// suffice since each shell is full.  Rows are padded to S1P (the most
+// species the count word holds, less one) so the contraction is unrolled at
+// compile time (the zero terms leave every sum unchanged), and the row stride
+// is odd in doubles so the lanes' row gathers spread over the banks.
+template <typename CW, int FIELD>
+constexpr int kS1P = 8 * (int)sizeof(CW) / FIELD - 1;
+template <int R, typename CW, int FIELD>
+constexpr int kRowStride = (R * kS1P<CW, FIELD>) | 1;
+
+// Fills dtab and vrow ([x][n][s]: V(x,s,n)).
+template <int R, typename CW, int FIELD>
+__device__ __forceinline__ void fill_tables(double *dtab, double *vrow, const double *V, int S) {
+  constexpr int S1P = kS1P<CW, FIELD>, RSTR = kRowStride<R, CW, FIELD>;
+  for (int i = threadIdx.x; i < S * S * RSTR; i += blockDim.x) {
+    const int row = i / RSTR, k = i - row * RSTR;
+    const int s = k % S1P, n = k / S1P, be = row % S, al = row / S;
+    double v = 0.0;
+    if (n < R && s < S - 1) {
+      double d_s = V[be + S * (s + S * n)] - V[al + S * (s + S * n)];
+      double d_l = V[be + S * ((S - 1) + S * n)] - V[al + S * ((S - 1) + S * n)];
+      v = d_s - d_l;
+    }
+    dtab[i] = v;
+  }
+  for (int i = threadIdx.x; i < S * R * S; i += blockDim.x) {
+    int s = i % S, n = (i / S) % R, x = i / (S * R);
+    vrow[i] = V[x + S * (s + S * n)];
+  }
+}
+
+// Energy change of exchanging species codes codeA and codeB at two sites with
+// shell counts ca and cb.
+template <int R, typename CW, int FIELD>
+__device__ __forceinline__ double pair_delta(const double *dtab, int S, int codeA, int codeB, const CW (&ca)[R],
+                                             const CW (&cb)[R]) {
+  constexpr int S1P = kS1P<CW, FIELD>, RSTR = kRowStride<R, CW, FIELD>;
+  // codes are FIELD*(species-1) >= 0: unsigned division is a shift
+  // (or a multiply-shift) without a sign fix-up
+  const int alpha = (int)((uint32_t)codeA / FIELD), betasp = (int)((uint32_t)codeB / FIELD);
+  const double *dt = dtab + __umul24((uint32_t)(alpha * S + betasp), (uint32_t)RSTR);
+  // a short table row is read into registers in one burst (the
+  // loads then overlap instead of one round trip per term)
+  constexpr bool kRowRegs = R * S1P <= 16;
+  double dv[kRowRegs ? R * S1P : 1];
+  if constexpr (kRowRegs) {
+#pragma unroll
+    for (int i = 0; i < R * S1P; ++i) dv[i] = dt[i];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto dtv = [&](int i) { return kRowRegs ? dv[kRowRegs ? i : 0] : dt[i]; };
+  // fused multiply-adds: each product enters the sum unrounded (one
+  // rounding per term instead of two, one instruction instead of two)
+  double dE = 0.0;
+#pragma unroll
+  for (int n = 0; n < R; ++n) {
+    constexpr uint32_t kM = (1u << FIELD) - 1;
+    constexpr int kB = 1 << (FIELD - 1), kLo = sizeof(CW) == 4 ? S1P : 4;
+    const uint32_t d0 = biased_diff<FIELD>((uint32_t)ca[n], (uint32_t)cb[n]);
+#pragma unroll
+    for (int s = 0; s < kLo; ++s)
+      dE = __builtin_fma((double)((int)((d0 >> (FIELD * s)) & kM) - kB), dtv(n * S1P + s), dE);
+    if constexpr (sizeof(CW) > 4) {
+      const uint32_t d1 = biased_diff<FIELD>((uint32_t)((uint64_t)ca[n] >> 32), (uint32_t)((uint64_t)cb[n] >> 32));
+#pragma unroll
+      for (int s = 4; s < S1P; ++s)
+        dE = __builtin_fma((double)((int)((d1 >> (FIELD * (s - 4))) & kM) - kB), dtv(n * S1P + s), dE);
+    }
+  }
+  return dE;
+}
+
+// One site's term of the recounted energy (twice the energy's share).
+template <int LAT, int R, typename CW, int NC, int FIELD, int ZN>
+__device__ __forceinline__ void add_site_energy(const int8_t *lat, const ND &N, const int (&off)[ZN],
+                                                const double *vrow, int S, int i, double &part) {
+  int c = i / (N.D0 * N.D1);
+  int r = i - c * N.D0 * N.D1;
+  int b = r / N.D0;
+  int a = r - b * N.D0;
+  int ad = nat_addr(N, a, b, c);
+  int sp = lat[ad] / FIELD;
+  CW cnt[R];
+  if constexpr (NC != 0)
+    count_c<LAT, R, CW, NC>(lat, ad, cnt);
+  else
+    count_nat<LAT, R, CW>(lat, ad, off, cnt);
+#pragma unroll
+  for (int n = 0; n < R; ++n) {
+    const double *vr = vrow + (sp * R + n) * S;
+    for (int s = 0; s < S; ++s) part += (double)((cnt[n] >> (FIELD * s)) & ((1u << FIELD) - 1)) * vr[s];
+  }
+}
+
+// rho(a, b, l) of a temperature step from its shell pair counts H(a, b, n):
+// mean over the samples of H / N_a, shell 0 on-site (the reference's
+// radial_densities layout, wc_range = R + 1).
+template <int LAT, int R>
+__device__ __forceinline__ void write_rho(const ParArgs &C, const unsigned long long *hacc, int S, int t) {
+  const int ns_asro = C.n_sweeps / C.asro_every;
+  for (int i = threadIdx.x; i < S * S * (R + 1); i += blockDim.x) {
+    const int a = i % S, b = (i / S) % S, l = i / (S * S);
+    unsigned long long tot = 0;
+    for (int b2 = 0; b2 < S; ++b2) tot += hacc[(a * S + b2) * R + 0];
+    const double na = (double)(tot / (unsigned long long)(shell_size<LAT>(0) * (ns_asro > 0 ? ns_asro : 1)));
+    double v;
+    if (l == 0)
+      v = (a == b ? na : 0.0) / na;
+    else
+      v = ((double)hacc[(a * S + b) * R + (l - 1)] / na) / (double)ns_asro;
+    C.rho_of_T[(size_t)t * S * S * (R + 1) + i] = v;
+  }
+}
+
+// A temperature step's averages (one thread).
+__device__ __forceinline__ void write_step(const ParArgs &C, int t, double temp, double sim_temp, double step_E,
+                                           double step_Esq, unsigned long long accepted, long long trials) {
+  const double ns = (double)C.n_sweeps;
+  const double na = (double)C.g.n_atoms;
+  C.energies_of_T[t] = step_E / ns / na;
+  double Cv = (step_Esq / ns - (step_E / ns) * (step_E / ns)) / (sim_temp * temp) / na;
+  if (Cv < 0.0) Cv = 0.0;
+  if (temp <= 0.0) Cv = 0.0;
+  C.C_of_T[t] = Cv;
+  C.acc_of_T[t] = (double)accepted / (double)trials;
+}
+
 template <int LAT, int R, typename CW, int NC, int FIELD>
 __global__ __launch_bounds__(NC != 0 && sizeof(CW) == 4 ? kMaxNatThreads : 512) void k_metro_nat(
     const ParArgs *__restrict__ chains) {
@@ -588,15 +716,7 @@ __global__ __launch_bounds__(NC != 0 && sizeof(CW) == 4 ? kMaxNatThreads : 512) 
   const int nthr = C.threads;
   const bool active = tid < nthr;
   const int S = g.S;
-  // dtab[alpha][beta][n][s<S1P]: (V(beta,s,n)-V(alpha,s,n)) - (same for
-  // s=S-1) for s < S-1, zero beyond; the S-1 independent count differences
-  // suffice since each shell is full.  Rows are padded to S1P (the most
-  // species the count word holds, less one) so the contraction below is
-  // unrolled at compile time (the zero terms leave every sum unchanged), and
-  // the row stride is odd in doubles so the lanes' row gathers spread over
-  // the banks.
-  constexpr int S1P = 8 * (int)sizeof(CW) / FIELD - 1;
-  constexpr int RSTR = (R * S1P) | 1;
+  constexpr int S1P = kS1P<CW, FIELD>, RSTR = kRowStride<R, CW, FIELD>;  // of dtab (see fill_tables)
   int8_t *lat = (int8_t *)smem;
   size_t o = ((N.P0 * N.P1 * N.P2) + 15) & ~15;
   double *dtab = (double *)(smem + o);
@@ -616,22 +736,7 @@ __global__ __launch_bounds__(NC != 0 && sizeof(CW) == 4 ? kMaxNatThreads : 512) 
 
   for (int i = tid; i < Z; i += blockDim.x) offl[i] = C.nat.off[i];
   for (int i = tid; i < S * S * R; i += blockDim.x) hacc[i] = 0ull;
-  for (int i = tid; i < S * S * RSTR; i += blockDim.x) {
-    const int row = i / RSTR, k = i - row * RSTR;
-    const int s = k % S1P, n = k / S1P, be = row % S, al = row / S;
-    const double *V = C.vex;
-    double v = 0.0;
-    if (n < R && s < S - 1) {
-      double d_s = V[be + S * (s + S * n)] - V[al + S * (s + S * n)];
-      double d_l = V[be + S * ((S - 1) + S * n)] - V[al + S * ((S - 1) + S * n)];
-      v = d_s - d_l;
-    }
-    dtab[i] = v;
-  }
-  for (int i = tid; i < S * R * S; i += blockDim.x) {
-    int s = i % S, n = (i / S) % R, x = i / (S * R);
-    vrow[i] = C.vex[x + S * (s + S * n)];
-  }
+  fill_tables<R, CW, FIELD>(dtab, vrow, C.vex, S);
   nat_stage<LAT>(lat, C.compact, g, N, FIELD);
   __syncthreads();
   int off[NC ? 1 : Z];
@@ -662,24 +767,8 @@ __global__ __launch_bounds__(NC != 0 && sizeof(CW) == 4 ? kMaxNatThreads : 512) 
   auto recount = [&]() -> double {
     double part = 0.0;
     const int nsites = N.D0 * N.D1 * N.D2;
-    for (int i = active ? tid : nsites; i < nsites; i += nthr) {
-      int c = i / (N.D0 * N.D1);
-      int r = i - c * N.D0 * N.D1;
-      int b = r / N.D0;
-      int a = r - b * N.D0;
-      int ad = nat_addr(N, a, b, c);
-      int sp = lat[ad] / FIELD;
-      CW cnt[R];
-      if constexpr (NC != 0)
-        count_c<LAT, R, CW, NC>(lat, ad, cnt);
-      else
-        count_nat<LAT, R, CW>(lat, ad, off, cnt);
-#pragma unroll
-      for (int n = 0; n < R; ++n) {
-        const double *vr = vrow + (sp * R + n) * S;
-        for (int s = 0; s < S; ++s) part += (double)((cnt[n] >> (FIELD * s)) & ((1u << FIELD) - 1)) * vr[s];
-      }
-    }
+    for (int i = active ? tid : nsites; i < nsites; i += nthr)
+      add_site_energy<LAT, R, CW, NC, FIELD>(lat, N, off, vrow, S, i, part);
     return 0.5 * block_sum(part, red);
   };
   // The energy is recounted before the first temperature step and at the end
@@ -829,33 +918,12 @@ __global__ __launch_bounds__(NC != 0 && sizeof(CW) == 4 ? kMaxNatThreads : 512) 
     }
     unsigned long long acc_sum = block_sum_u64(acc_local, redu);
     if (C.asro_every > 0) {
-      // rho(a, b, l) = mean over samples of H(a, b, l) / N_a, shell 0 on-site
-      // (the reference's radial_densities layout, wc_range = R + 1)
-      const int ns_asro = C.n_sweeps / C.asro_every;
-      for (int i = tid; i < S * S * (R + 1); i += blockDim.x) {
-        const int a = i % S, b = (i / S) % S, l = i / (S * S);
-        unsigned long long tot = 0;
-        for (int b2 = 0; b2 < S; ++b2) tot += hacc[(a * S + b2) * R + 0];
-        const double na = (double)(tot / (unsigned long long)(shell_size<LAT>(0) * (ns_asro > 0 ? ns_asro : 1)));
-        double v;
-        if (l == 0)
-          v = (a == b ? na : 0.0) / na;
-        else
-          v = ((double)hacc[(a * S + b) * R + (l - 1)] / na) / (double)ns_asro;
-        C.rho_of_T[(size_t)t * S * S * (R + 1) + i] = v;
-      }
+      write_rho<LAT, R>(C, hacc, S, t);
       __syncthreads();
       for (int i = tid; i < S * S * R; i += blockDim.x) hacc[i] = 0ull;
     }
     if (tid == 0) {
-      const double ns = (double)C.n_sweeps;
-      const double na = (double)g.n_atoms;
-      C.energies_of_T[t] = step_E / ns / na;
-      double Cv = (step_Esq / ns - (step_E / ns) * (step_E / ns)) / (sim_temp * temp) / na;
-      if (Cv < 0.0) Cv = 0.0;
-      if (temp <= 0.0) Cv = 0.0;
-      C.C_of_T[t] = Cv;
-      C.acc_of_T[t] = (double)acc_sum / (double)trials_sampled;
+      write_step(C, t, temp, sim_temp, step_E, step_Esq, acc_sum, trials_sampled);
       acc_total += (long long)acc_sum;
     }
     const double Er = recount();
@@ -1033,14 +1101,7 @@ __global__ __launch_bounds__(512) void k_metro_cmp(const ParArgs *__restrict__ c
     }
     unsigned long long acc_sum = block_sum_u64(acc_local, redu);
     if (tid == 0) {
-      const double ns = (double)C.n_sweeps;
-      const double na = (double)g.n_atoms;
-      C.energies_of_T[t] = step_E / ns / na;
-      double Cv = (step_Esq / ns - (step_E / ns) * (step_E / ns)) / (sim_temp * temp) / na;
-      if (Cv < 0.0) Cv = 0.0;
-      if (temp <= 0.0) Cv = 0.0;
-      C.C_of_T[t] = Cv;
-      C.acc_of_T[t] = (double)acc_sum / (double)trials_sampled;
+      write_step(C, t, temp, sim_temp, step_E, step_Esq, acc_sum, trials_sampled);
       acc_total += (long long)acc_sum;
     }
     const double Er = recount();
