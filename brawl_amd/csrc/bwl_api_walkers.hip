@@ -211,8 +211,13 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
     return fail(BWL_ERR_ARG, "null argument");
   const int lim = lds_limit();
   SeqPick pick, energies;
-  size_t total = align256(sizeof(NsArgs) * (size_t)n);
-  std::vector<size_t> offs((size_t)n);
+  // Device memory: the arguments and, per run, its stream and results (copied
+  // up and down in one piece each), then the walkers.
+  const size_t args_bytes = align256(sizeof(NsArgs) * (size_t)n), set_bytes = align256(sizeof(SetupArgs) * (size_t)n);
+  size_t total = args_bytes + set_bytes;
+  std::vector<size_t> io((size_t)n), offs((size_t)n);
+  std::vector<SetupArgs> sets((size_t)n);
+  int max_w = 0, max_atoms = 0;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
     int rc = check_ctx(c, false);
@@ -227,45 +232,62 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
     if (2 * c->g.R > 64) return fail(BWL_ERR_UNSUPPORTED, "too many shells");
     pick.add(c->g, ns_lds_bytes(c->g, p->n_walkers), ns_spec_lds_bytes(c->g, p->n_walkers));
     energies.add(c->g, ns_energies_lds_bytes(c->g), energies_spec_lds_bytes(c->g));
-    offs[(size_t)i] = total;
-    const size_t ref = (size_t)c->g.m[0] * c->g.m[1] * c->g.m[2];
-    total += align256((size_t)c->g.compact_bytes * p->n_walkers) +
-             align256(sizeof(double) * 2 * p->n_walkers) + align256(624 * 4 + 64) +
-             align256(sizeof(long long) * 3) + align256(sizeof(double) * p->n_iter) +
-             align256(ref * p->n_walkers);
+    io[(size_t)i] = total;
+    total += align256(624 * 4 + 64 + sizeof(double) * (size_t)p->n_iter);
+    max_w = std::max(max_w, p->n_walkers);
+    max_atoms = std::max(max_atoms, c->g.n_atoms);
   }
   if (pick.lds > (size_t)lim) return fail(BWL_ERR_UNSUPPORTED, "lattice and walker energies do not fit in LDS");
   pick.settle(lim);
   energies.settle(lim);
+  for (int i = 0; i < n; ++i) {
+    const int rc = setup_rule(ctxs[i]->g, species_numbers[i], concentrations[i], sets[(size_t)i].rule, g_err);
+    if (rc) return rc;
+  }
+  const size_t io_bytes = total;
+  for (int i = 0; i < n; ++i) {
+    const Geo &g = ctxs[i]->g;
+    const size_t W = (size_t)params[i].n_walkers;
+    offs[(size_t)i] = total;
+    total += align256((size_t)g.compact_bytes * W) + align256((size_t)g.n_atoms * W) + align256(sizeof(double) * 2 * W);
+  }
   bwl_ctx *c0 = ctxs[0];
   DevBuf buf;
   if (hipMalloc(&buf.p, total) != hipSuccess) return fail(BWL_ERR_NOMEM, "device allocation failed");
   char *base = (char *)buf.p;
   std::vector<NsArgs> args((size_t)n);
-  std::vector<std::vector<double>> rnde((size_t)n);
+  std::vector<char> host(io_bytes, 0);
+  // a context that appears twice gives both its runs one stream, the second's
+  // walkers after the first's: those are drawn on the host, in turn
+  std::vector<const bwl_ctx *> seen(ctxs, ctxs + n);
+  std::sort(seen.begin(), seen.end());
+  auto shared = [&](const bwl_ctx *c) {
+    const auto r = std::equal_range(seen.begin(), seen.end(), c);
+    return r.second - r.first > 1;
+  };
+  bool any_drawn = false;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
     const Geo &g = c->g;
     const bwl_ns_params *p = &params[i];
     NsArgs &a = args[(size_t)i];
     memset(&a, 0, sizeof(a));
-    char *q = base + offs[(size_t)i];
+    char *q = base + offs[(size_t)i], *r = base + io[(size_t)i];
+    const size_t W = (size_t)p->n_walkers;
     a.g = g;
     a.off = c->d_off;
     a.vex = c->d_vex;
     a.walkers = (int8_t *)q;
-    q += align256((size_t)g.compact_bytes * p->n_walkers);
-    a.rnde = (const double *)q;
-    a.E = (double *)q + p->n_walkers;
-    q += align256(sizeof(double) * 2 * p->n_walkers);
-    a.mt = (uint32_t *)q;
-    a.mt_index = (int32_t *)(q + 624 * 4);
-    q += align256(624 * 4 + 64);
-    a.counters = (long long *)q;
-    q += align256(sizeof(long long) * 3);
-    a.e_limits = (double *)q;
-    q += align256(sizeof(double) * p->n_iter);
-    int8_t *staging = (int8_t *)q;  // the walkers in the reference layout
+    q += align256((size_t)g.compact_bytes * W);
+    int8_t *order = (int8_t *)q;
+    q += align256((size_t)g.n_atoms * W);
+    double *rnde = (double *)q;
+    a.rnde = rnde;
+    a.E = rnde + W;
+    a.mt = (uint32_t *)r;
+    a.mt_index = (int32_t *)(r + 624 * 4);
+    a.counters = (long long *)(r + 624 * 4 + 16);
+    a.e_limits = (double *)(r + 624 * 4 + 64);
     a.n_walkers = p->n_walkers;
     a.n_steps = p->n_steps;
     a.n_iter = p->n_iter;
@@ -275,30 +297,41 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
     // walkers from the run's MT19937 stream: initial_setup, then one draw
     // for the energy jitter (nested_sampling.f90:88-96)
     if (c->mt.mti == 625) c->mt.seed(5489u);
-    const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
-    std::vector<int8_t> cfgs(ref * (size_t)p->n_walkers);
-    rnde[(size_t)i].resize((size_t)p->n_walkers);
-    for (int w = 0; w < p->n_walkers; ++w) {
-      int rc = initial_setup_host(g, species_numbers[i], concentrations[i], c->mt,
-                                  cfgs.data() + ref * (size_t)w, g_err);
-      if (rc) return rc;
-      rnde[(size_t)i][(size_t)w] = c->mt.genrand();
+    SetupArgs &u = sets[(size_t)i];
+    u.g = g;
+    u.mt = a.mt;
+    u.mt_index = a.mt_index;
+    u.order = order;
+    u.walkers = a.walkers;
+    u.rnde = rnde;
+    u.n_walkers = p->n_walkers;
+    u.made = setup_on_device(g, u.rule) && !shared(c) ? 0 : 1;
+    u.status = (int32_t *)(r + 624 * 4 + 48);
+    if (u.made) {
+      std::vector<int8_t> cfgs((size_t)g.n_atoms * W);
+      std::vector<double> after(W);
+      for (size_t w = 0; w < W; ++w) {
+        if (!setup_order(g, u.rule, c->mt, cfgs.data() + (size_t)g.n_atoms * w))
+          return fail(BWL_ERR_ARG, "initial_setup did not terminate");
+        after[w] = c->mt.genrand();
+      }
+      HIP_OK(hipMemcpyAsync(order, cfgs.data(), cfgs.size(), hipMemcpyHostToDevice, c0->stream));
+      HIP_OK(hipMemcpyAsync(rnde, after.data(), sizeof(double) * W, hipMemcpyHostToDevice, c0->stream));
+      HIP_OK(hipStreamSynchronize(c0->stream));
+    } else {
+      any_drawn = true;
     }
-    HIP_OK(hipMemcpyAsync(staging, cfgs.data(), cfgs.size(), hipMemcpyHostToDevice, c0->stream));
-    HIP_OK(launch_pack_many(staging, a.walkers, g, p->n_walkers, c0->stream));
-    HIP_OK(hipMemcpyAsync((void *)a.rnde, rnde[(size_t)i].data(), sizeof(double) * p->n_walkers,
-                          hipMemcpyHostToDevice, c0->stream));
-    HIP_OK(hipMemcpyAsync(a.mt, c->mt.mt, 624 * 4, hipMemcpyHostToDevice, c0->stream));
-    int32_t mti = c->mt.mti;
-    HIP_OK(hipMemcpyAsync(a.mt_index, &mti, 4, hipMemcpyHostToDevice, c0->stream));
-    HIP_OK(hipStreamSynchronize(c0->stream));
+    memcpy(host.data() + io[(size_t)i], c->mt.mt, 624 * 4);
+    memcpy(host.data() + io[(size_t)i] + 624 * 4, &c->mt.mti, 4);
   }
-  HIP_OK(hipMemcpyAsync(base, args.data(), sizeof(NsArgs) * (size_t)n, hipMemcpyHostToDevice, c0->stream));
+  memcpy(host.data(), args.data(), sizeof(NsArgs) * (size_t)n);
+  memcpy(host.data() + args_bytes, sets.data(), sizeof(SetupArgs) * (size_t)n);
+  HIP_OK(hipMemcpyAsync(base, host.data(), io_bytes, hipMemcpyHostToDevice, c0->stream));
+  HIP_OK(launch_setup((const SetupArgs *)(base + args_bytes), n, max_w, max_atoms, any_drawn, c0->stream));
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
-  int max_w = 0;
-  for (int i = 0; i < n; ++i) max_w = std::max(max_w, params[i].n_walkers);
   HIP_OK(launch_ns((const NsArgs *)base, n, pick, max_w, energies, c0->stream));
   HIP_OK(hipEventRecord(c0->ev1, c0->stream));
+  HIP_OK(hipMemcpyAsync(host.data(), base, io_bytes, hipMemcpyDeviceToHost, c0->stream));
   HIP_OK(hipStreamSynchronize(c0->stream));
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, c0->ev0, c0->ev1);
@@ -306,20 +339,21 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
   int status = BWL_OK;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
-    const NsArgs &a = args[(size_t)i];
+    const char *r = host.data() + io[(size_t)i];
     long long cnt[3];
-    int32_t mti = 0;
-    HIP_OK(hipMemcpy(e_limits[i], a.e_limits, sizeof(double) * a.n_iter, hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(cnt, a.counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(c->mt.mt, a.mt, 624 * 4, hipMemcpyDeviceToHost));
-    HIP_OK(hipMemcpy(&mti, a.mt_index, 4, hipMemcpyDeviceToHost));
-    c->mt.mti = mti;
+    int32_t set_status = 0;
+    memcpy(e_limits[i], r + 624 * 4 + 64, sizeof(double) * (size_t)params[i].n_iter);
+    memcpy(cnt, r + 624 * 4 + 16, sizeof(cnt));
+    memcpy(&set_status, r + 624 * 4 + 48, sizeof(set_status));
+    memcpy(c->mt.mt, r, 624 * 4);
+    memcpy(&c->mt.mti, r + 624 * 4, 4);
     if (stats) {
       stats[i].trials = cnt[0];
       stats[i].accepted = cnt[1];
       stats[i].kernel_ms = ms;
       stats[i].e_drift_abs = stats[i].e_drift_rel = 0.0;
     }
+    if (set_status != 0) return fail(BWL_ERR_ARG, "initial_setup did not terminate");
     if (cnt[2] != 0) status = fail(BWL_ERR_STATE, "nested sampling: no second species found for a trial");
   }
   return status;

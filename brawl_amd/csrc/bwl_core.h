@@ -44,6 +44,14 @@ struct Geo {
   int32_t shell_start[kMaxShells + 1];
 };
 
+// What initial_setup draws by: a draw (32 bits) names species s when it lies
+// in [lo, hi] (inclusive, as the cumulative bounds are; empty when lo > hi),
+// and places one of its count atoms.
+struct SetupRule {
+  uint32_t lo[kMaxSpecies], hi[kMaxSpecies];
+  int32_t count[kMaxSpecies];
+};
+
 // The straight-line variant of the sequential walkers' ordered pair-energy
 // sum for a lattice: lattice*16 + R for fcc and bcc up to 6 shells, 0 for
 // the mask-driven loop (bwl_seq.h).

@@ -110,11 +110,14 @@ uint32_t MT19937::next() {
 // initialise.F90:468-472) or from concentrations (nint + round-robin
 // correction, :480-504); then rejection sampling site by site, in the
 // reference's loop order, against inclusive cumulative bounds.
-int initial_setup_host(const Geo &g, const int64_t *species_numbers, const double *concentrations,
-                       MT19937 &mt, int8_t *config, std::string &err) {
+// A draw on the bound of two species places an atom of the first that has one
+// left (the reference would count one of each and then never fill its last
+// site).
+int setup_rule(const Geo &g, const int64_t *species_numbers, const double *concentrations, SetupRule &rule,
+               std::string &err) {
   const int S = g.S;
   const int n_sites = g.n_atoms;
-  std::vector<int64_t> count(S, 0), placed(S, 0);
+  std::vector<int64_t> count(S, 0);
   std::vector<double> conc(S + 1, 0.0);
   int64_t total_numbers = 0;
   if (species_numbers)
@@ -167,41 +170,71 @@ int initial_setup_host(const Geo &g, const int64_t *species_numbers, const doubl
   for (int l = 0; l <= S; ++l) {
     double acc = 0.0;
     for (int q = 0; q <= l; ++q) acc = acc + conc[q];
-    bound[l] = acc;
+    bound[l] = acc * 4294967296.0;  // in units of a draw, exactly
+  }
+  memset(&rule, 0, sizeof(rule));
+  for (int s = 0; s < kMaxSpecies; ++s) rule.lo[s] = 1;  // empty
+  for (int s = 0; s < S; ++s) {
+    rule.count[s] = (int32_t)count[s];
+    const double lo = ceil(bound[s]), hi = floor(bound[s + 1]);
+    if (!(lo <= 4294967295.0) || !(hi >= 0.0) || !(lo <= hi)) continue;
+    rule.lo[s] = lo <= 0.0 ? 0u : (uint32_t)lo;
+    rule.hi[s] = hi >= 4294967295.0 ? 0xffffffffu : (uint32_t)hi;
+  }
+  return BWL_OK;
+}
+
+bool setup_on_device(const Geo &g, const SetupRule &rule) {
+  for (int s = 0; s < g.S; ++s)
+    if (rule.count[s] > 0 && (rule.lo[s] > rule.hi[s] || rule.hi[s] - rule.lo[s] < 429497u)) return false;
+  return true;
+}
+
+bool setup_order(const Geo &g, const SetupRule &rule, MT19937 &mt, int8_t *order) {
+  int32_t room[kMaxSpecies];
+  memcpy(room, rule.count, sizeof(room));
+  const int S = g.S;
+  for (int i = 0; i < g.n_atoms; ++i) {
+    int8_t sp = 0;
+    for (long long draws = 0; sp == 0; ++draws) {
+      if (draws > (1LL << 40)) return false;
+      const uint32_t k = mt.next();
+      for (int s = 0; s < S && sp == 0; ++s)
+        if (k >= rule.lo[s] && k <= rule.hi[s] && room[s] > 0) sp = (int8_t)(s + 1);
+    }
+    room[sp - 1]--;
+    order[i] = sp;
+  }
+  return true;
+}
+
+int initial_setup_host(const Geo &g, const int64_t *species_numbers, const double *concentrations,
+                       MT19937 &mt, int8_t *config, std::string &err) {
+  SetupRule rule;
+  const int rc = setup_rule(g, species_numbers, concentrations, rule, err);
+  if (rc) return rc;
+  std::vector<int8_t> order((size_t)g.n_atoms);
+  if (!setup_order(g, rule, mt, order.data())) {
+    err = "initial_setup did not terminate";
+    return BWL_ERR_ARG;
   }
   const size_t cells = (size_t)g.m[0] * g.m[1] * g.m[2];
   memset(config, 0, cells);
-  auto fill = [&](size_t idx) -> bool {
-    long long draws = 0;
-    while (config[idx] == 0) {
-      double r = mt.genrand();
-      for (int l = 1; l <= S; ++l) {
-        if (r >= bound[l - 1] && r <= bound[l] && placed[l - 1] < count[l - 1]) {
-          config[idx] = (int8_t)l;
-          placed[l - 1]++;
-        }
-      }
-      if (++draws > (1LL << 40)) return false;
-    }
-    return true;
-  };
+  const int8_t *next = order.data();
   const int m0 = g.m[0], m1 = g.m[1], m2 = g.m[2];
   for (int k = 1; k <= m2; ++k) {
     if (g.lattice == BWL_BCC) {
       // sites (2i - mod(k,2), 2j - mod(k,2), k), initialise.F90:540-570
       const int sh = k & 1;
       for (int j = 1; j <= m1 / 2; ++j)
-        for (int i = 1; i <= m0 / 2; ++i) {
-          size_t idx = (size_t)(2 * i - sh - 1) + (size_t)m0 * ((2 * j - sh - 1) + (size_t)m1 * (k - 1));
-          if (!fill(idx)) { err = "initial_setup did not terminate"; return BWL_ERR_ARG; }
-        }
+        for (int i = 1; i <= m0 / 2; ++i)
+          config[(size_t)(2 * i - sh - 1) + (size_t)m0 * ((2 * j - sh - 1) + (size_t)m1 * (k - 1))] = *next++;
     } else {
       // fcc, initialise.F90:572-611
       for (int j = 1; j <= m1; ++j)
         for (int i = 1; i <= m0 / 2; ++i) {
-          int x = 2 * i - (k & 1) * (j & 1) - ((k + 1) & 1) * ((j + 1) & 1);
-          size_t idx = (size_t)(x - 1) + (size_t)m0 * ((j - 1) + (size_t)m1 * (k - 1));
-          if (!fill(idx)) { err = "initial_setup did not terminate"; return BWL_ERR_ARG; }
+          const int x = 2 * i - (k & 1) * (j & 1) - ((k + 1) & 1) * ((j + 1) & 1);
+          config[(size_t)(x - 1) + (size_t)m0 * ((j - 1) + (size_t)m1 * (k - 1))] = *next++;
         }
     }
   }

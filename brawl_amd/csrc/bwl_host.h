@@ -26,6 +26,16 @@ struct MT19937 {
   double genrand() { return (double)next() * (1.0 / 4294967296.0); }
 };
 
+// What initial_setup draws by, from species numbers or concentrations.
+int setup_rule(const Geo &g, const int64_t *species_numbers, const double *concentrations, SetupRule &rule,
+               std::string &err);
+// Whether the device may make the draws (bwl_setup.hip): every species with
+// atoms is named by one draw in 10^4 at least, so a walker is soon complete.
+// Others (a concentration that rounds to one atom and back to no bound, say)
+// are drawn on the host, without end if need be.
+bool setup_on_device(const Geo &g, const SetupRule &rule);
+// The draws on the host: species in the order in which sites are filled.
+bool setup_order(const Geo &g, const SetupRule &rule, MT19937 &mt, int8_t *order);
 // initial_setup (initialise.F90:434-617) into a reference-layout config.
 int initial_setup_host(const Geo &g, const int64_t *species_numbers, const double *concentrations,
                        MT19937 &mt, int8_t *config, std::string &err);

@@ -92,6 +92,20 @@ struct ParArgs {
   unsigned long long *mail;  // par_split_mail_words words, zeroed
 };
 
+// Initial configurations of one stream's walkers (bwl_setup.hip).
+struct SetupArgs {
+  Geo g;
+  SetupRule rule;
+  uint32_t *mt;           // 624 words, in/out
+  int32_t *mt_index;      // in/out, at most 624
+  int8_t *order;          // species of n_walkers lattices in the order of set-up, g.n_atoms apart
+  int8_t *walkers;        // out: the same as compact lattices, g.compact_bytes apart
+  double *rnde;           // out, optional: a draw after each walker's set-up
+  int32_t n_walkers;
+  int32_t made;           // `order` and `rnde` hold the host's own draws
+  int32_t *status;        // out: 1 when a walker took too many draws (not written if made)
+};
+
 // Nested sampling (nested_sampling.f90:45-206), one wavefront per run.
 struct NsArgs {
   Geo g;
@@ -177,6 +191,8 @@ hipError_t launch_pack(const int8_t *ref, int8_t *compact, const Geo &g, hipStre
 // `count` reference-layout lattices back to back -> compact lattices back to back
 hipError_t launch_pack_many(const int8_t *ref, int8_t *compact, const Geo &g, int count,
                             hipStream_t s);
+// n streams (args_dev[0..n)); any_drawn: not all of them were made on the host
+hipError_t launch_setup(const SetupArgs *args_dev, int n, int max_walkers, int max_atoms, bool any_drawn, hipStream_t s);
 hipError_t launch_unpack(const int8_t *compact, int8_t *ref, const Geo &g, hipStream_t s);
 // LDS read-bandwidth probe: blocks x 1024 threads, iters 16-byte reads each
 hipError_t launch_lds_bandwidth(int blocks, int iters, uint32_t *sink, hipStream_t s);

@@ -97,21 +97,26 @@ struct Request {
   double *E = nullptr, *Cv = nullptr, *acc = nullptr;
   int8_t *config_out = nullptr;
   const void *fn = nullptr;  // kernel variant (grouping key)
-  // nested sampling: walkers prepared on the host at submission
+  // walkers' set-up, on the device unless its rule has to be drawn on the host
+  // (setup_on_device), which is done at submission
+  SetupRule rule;
+  bool made = false;
+  std::vector<int8_t> order;  // if made: species of all walkers in the order of set-up
+  // nested sampling: the run's stream
   bwl_ns_params np;
-  std::vector<int8_t> walkers_ref;  // n_walkers reference-layout configs
-  std::vector<double> rnde;
+  std::vector<double> rnde;  // if made
   uint32_t mt[624];
   int32_t mti = 0;
+  int32_t index[2] = {0, 0};  // mti and the set-up's status as uploaded
   double *e_limits = nullptr;
-  // Wang-Landau window: walkers prepared on the host at submission
+  // Wang-Landau windows
   bwl_wl_params wp;
   double wl_f = 0.0;
   int32_t hstride = 0;
   std::vector<int32_t> windows;
   std::vector<double> edges;
   std::vector<uint32_t> wl_mt;   // 624 words per walker
-  std::vector<int32_t> wl_mti;
+  std::vector<int32_t> wl_mti;    // a position per walker, then the set-ups' statuses
   double *lng_out = nullptr, *hist_out = nullptr;
   // device residency
   size_t block_bytes = 0;
@@ -129,6 +134,7 @@ struct Launch {
   std::unique_ptr<AnnealPlan> plan;
   std::vector<NsArgs> ns_args;
   std::vector<WlArgs> wl_args;
+  std::vector<SetupArgs> setups;
   std::vector<size_t> wl_first;  // first walker of each request in wl_args
   char *scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -160,19 +166,17 @@ namespace {
 
 size_t ns_block_bytes(const Request &r) {
   const Geo &g = r.g;
-  const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
   const size_t W = (size_t)r.np.n_walkers;
-  return ctx_device_bytes(r.desc) + al((size_t)g.compact_bytes * W) + al(ref * W) +
+  return ctx_device_bytes(r.desc) + al((size_t)g.compact_bytes * W) + al((size_t)g.n_atoms * W) +
          al(sizeof(double) * 2 * W) + al(624 * 4 + 64) + al(sizeof(long long) * 3) +
          al(sizeof(double) * (size_t)r.np.n_iter);
 }
 
 size_t wl_block_bytes(const Request &r) {
   const Geo &g = r.g;
-  const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
   const size_t W = (size_t)r.wp.num_windows * r.wp.walkers_per_window;
-  return ctx_device_bytes(r.desc) + al((size_t)g.compact_bytes * W) + al(ref * W) + al(W * 624 * 4) +
-         al(W * 4) + al(sizeof(double) * (r.wp.bins + 1)) + al(sizeof(double) * W * r.wp.bins) +
+  return ctx_device_bytes(r.desc) + al((size_t)g.compact_bytes * W) + al((size_t)g.n_atoms * W) + al(W * 624 * 4) +
+         al(W * 8) + al(sizeof(double) * (r.wp.bins + 1)) + al(sizeof(double) * W * r.wp.bins) +
          al(sizeof(double) * W * r.hstride) + al(8 * W);
 }
 
@@ -239,12 +243,15 @@ int retire(bwl_server *s, Launch &L) {
       }
       if (hipMemcpyAsync(acc.data(), L.wl_args[f].accepted, 8 * W, hipMemcpyDeviceToHost, st) !=
               hipSuccess ||
+          hipMemcpyAsync(r->wl_mti.data(), L.wl_args[f].mt_index, 8 * W, hipMemcpyDeviceToHost, st) != hipSuccess ||
           hipStreamSynchronize(st) != hipSuccess) {
         status = fail(BWL_ERR_DEVICE, "result download failed");
         continue;
       }
       r->accepted = 0;
       for (long long a : acc) r->accepted += a;
+      for (size_t k = 0; k < W; ++k)
+        if (r->wl_mti[W + k] != 0) r->error = BWL_ERR_ARG;  // initial_setup did not terminate
       r->trials = (int64_t)W * r->wp.mc_sweeps * r->g.n_atoms;
     }
   } else {
@@ -254,6 +261,7 @@ int retire(bwl_server *s, Launch &L) {
       long long cnt[3] = {0, 0, 0};
       if (hipMemcpyAsync(r->e_limits, a.e_limits, sizeof(double) * a.n_iter, hipMemcpyDeviceToHost,
                          st) != hipSuccess ||
+          hipMemcpyAsync(r->index, a.mt_index, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
           hipMemcpyAsync(cnt, a.counters, sizeof(cnt), hipMemcpyDeviceToHost, st) != hipSuccess ||
           hipStreamSynchronize(st) != hipSuccess) {
         status = fail(BWL_ERR_DEVICE, "result download failed");
@@ -262,6 +270,7 @@ int retire(bwl_server *s, Launch &L) {
       r->trials = cnt[0];
       r->accepted = cnt[1];
       if (cnt[2] != 0) r->error = BWL_ERR_STATE;
+      if (r->index[1] != 0) r->error = BWL_ERR_ARG;  // initial_setup did not terminate
     }
   }
   if (hipStreamSynchronize(st) != hipSuccess && status == BWL_OK)
@@ -329,6 +338,19 @@ int launch_anneal_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   return BWL_OK;
 }
 
+// The walkers' set-up of a launch on its stream.
+int launch_setups(Launch &L, char *args_dev, int max_walkers, hipStream_t st) {
+  int max_atoms = 0;
+  bool any_drawn = false;
+  for (const SetupArgs &u : L.setups) {
+    max_atoms = std::max(max_atoms, u.g.n_atoms);
+    any_drawn = any_drawn || !u.made;
+  }
+  HIP_OK(hipMemcpyAsync(args_dev, L.setups.data(), sizeof(SetupArgs) * L.setups.size(), hipMemcpyHostToDevice, st));
+  HIP_OK(launch_setup((const SetupArgs *)args_dev, (int)L.setups.size(), max_walkers, max_atoms, any_drawn, st));
+  return BWL_OK;
+}
+
 int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   hipStream_t st = s->streams[(size_t)slot];
   auto L = std::make_unique<Launch>();
@@ -342,13 +364,12 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   }
   pick.settle(lds_limit());
   energies.settle(lds_limit());
-  L->scratch_bytes = al(sizeof(NsArgs) * grp.size());
+  L->scratch_bytes = al(sizeof(NsArgs) * grp.size()) + al(sizeof(SetupArgs) * grp.size());
   L->scratch = s->arena.alloc(L->scratch_bytes);
   if (!L->scratch) return BWL_ERR_NOMEM;
   for (Request *r : grp) {
     const Geo &g = r->g;
     const size_t W = (size_t)r->np.n_walkers;
-    const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
     char *q = r->block + ctx_device_bytes(r->desc);
     NsArgs a;
     memset(&a, 0, sizeof(a));
@@ -357,10 +378,13 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
     a.vex = r->ctx->d_vex;
     a.walkers = (int8_t *)q;
     q += al((size_t)g.compact_bytes * W);
-    int8_t *staging = (int8_t *)q;
-    q += al(ref * W);
-    a.rnde = (const double *)q;
-    a.E = (double *)q + W;
+    SetupArgs u;
+    memset(&u, 0, sizeof(u));
+    u.order = (int8_t *)q;
+    q += al((size_t)g.n_atoms * W);
+    u.rnde = (double *)q;
+    a.rnde = u.rnde;
+    a.E = u.rnde + W;
     q += al(sizeof(double) * 2 * W);
     a.mt = (uint32_t *)q;
     a.mt_index = (int32_t *)(q + 624 * 4);
@@ -373,20 +397,33 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
     a.n_iter = r->np.n_iter;
     a.n_at = g.n[0] * g.n[1] * g.n[2] * 1 * g.S;  // nested_sampling.f90:82
     a.max_redraws = 1LL << 24;
-    HIP_OK(hipMemcpyAsync(staging, r->walkers_ref.data(), ref * W, hipMemcpyHostToDevice, st));
-    HIP_OK(launch_pack_many(staging, a.walkers, g, (int)W, st));
-    HIP_OK(hipMemcpyAsync((void *)a.rnde, r->rnde.data(), sizeof(double) * W, hipMemcpyHostToDevice, st));
+    u.g = g;
+    u.rule = r->rule;
+    u.mt = a.mt;
+    u.mt_index = a.mt_index;
+    u.walkers = a.walkers;
+    u.n_walkers = r->np.n_walkers;
+    u.made = r->made ? 1 : 0;
+    u.status = a.mt_index + 1;
+    if (r->made) {
+      HIP_OK(hipMemcpyAsync(u.order, r->order.data(), r->order.size(), hipMemcpyHostToDevice, st));
+      HIP_OK(hipMemcpyAsync(u.rnde, r->rnde.data(), sizeof(double) * W, hipMemcpyHostToDevice, st));
+    }
+    L->setups.push_back(u);
     HIP_OK(hipMemcpyAsync(a.mt, r->mt, 624 * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(a.mt_index, &r->mti, 4, hipMemcpyHostToDevice, st));
+    r->index[0] = r->mti;
+    HIP_OK(hipMemcpyAsync(a.mt_index, r->index, 8, hipMemcpyHostToDevice, st));
     L->ns_args.push_back(a);
   }
   HIP_OK(hipMemcpyAsync(L->scratch, L->ns_args.data(), sizeof(NsArgs) * grp.size(),
                         hipMemcpyHostToDevice, st));
+  int max_w = 0;
+  for (Request *r : grp) max_w = std::max(max_w, r->np.n_walkers);
+  const int rc = launch_setups(*L, L->scratch + al(sizeof(NsArgs) * grp.size()), max_w, st);
+  if (rc) return rc;
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
-  int max_w = 0;
-  for (Request *r : grp) max_w = std::max(max_w, r->np.n_walkers);
   HIP_OK(launch_ns((const NsArgs *)L->scratch, (int)grp.size(), pick, max_w, energies, st));
   HIP_OK(hipEventRecord(L->ev1, st));
   s->slot_busy[(size_t)slot] = true;
@@ -407,23 +444,22 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
     total_w += (size_t)r->wp.num_windows * r->wp.walkers_per_window;
   }
   pick.settle(lds_limit());
-  L->scratch_bytes = al(sizeof(WlArgs) * total_w);
+  L->scratch_bytes = al(sizeof(WlArgs) * total_w) + al(sizeof(SetupArgs) * total_w);
   L->scratch = s->arena.alloc(L->scratch_bytes);
   if (!L->scratch) return BWL_ERR_NOMEM;
   for (Request *r : grp) {
     const Geo &g = r->g;
     const int wpw = r->wp.walkers_per_window;
     const size_t W = (size_t)r->wp.num_windows * wpw;
-    const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
     char *q = r->block + ctx_device_bytes(r->desc);
     int8_t *walkers = (int8_t *)q;
     q += al((size_t)g.compact_bytes * W);
-    int8_t *staging = (int8_t *)q;
-    q += al(ref * W);
+    int8_t *order = (int8_t *)q;
+    q += al((size_t)g.n_atoms * W);
     uint32_t *mt = (uint32_t *)q;
     q += al(W * 624 * 4);
-    int32_t *mti = (int32_t *)q;
-    q += al(W * 4);
+    int32_t *mti = (int32_t *)q;  // W positions, then the set-ups' statuses
+    q += al(W * 8);
     double *edges = (double *)q;
     q += al(sizeof(double) * (r->wp.bins + 1));
     double *lng = (double *)q;
@@ -431,10 +467,9 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
     double *hist = (double *)q;
     q += al(sizeof(double) * W * r->hstride);
     long long *acc = (long long *)q;
-    HIP_OK(hipMemcpyAsync(staging, r->walkers_ref.data(), ref * W, hipMemcpyHostToDevice, st));
-    HIP_OK(launch_pack_many(staging, walkers, g, (int)W, st));
+    if (r->made) HIP_OK(hipMemcpyAsync(order, r->order.data(), r->order.size(), hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(mt, r->wl_mt.data(), W * 624 * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(mti, r->wl_mti.data(), W * 4, hipMemcpyHostToDevice, st));
+    HIP_OK(hipMemcpyAsync(mti, r->wl_mti.data(), W * 8, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(edges, r->edges.data(), sizeof(double) * (r->wp.bins + 1),
                           hipMemcpyHostToDevice, st));
     HIP_OK(hipMemsetAsync(lng, 0, sizeof(double) * W * r->wp.bins, st));
@@ -461,10 +496,24 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
       a.hist = hist + (size_t)r->hstride * k;
       a.accepted = acc + k;
       L->wl_args.push_back(a);
+      SetupArgs u;
+      memset(&u, 0, sizeof(u));
+      u.g = g;
+      u.rule = r->rule;
+      u.mt = a.mt;
+      u.mt_index = a.mt_index;
+      u.order = order + (size_t)g.n_atoms * k;
+      u.walkers = a.compact;
+      u.n_walkers = 1;
+      u.made = r->made ? 1 : 0;
+      u.status = mti + W + k;
+      L->setups.push_back(u);
     }
   }
   HIP_OK(hipMemcpyAsync(L->scratch, L->wl_args.data(), sizeof(WlArgs) * total_w,
                         hipMemcpyHostToDevice, st));
+  const int rc = launch_setups(*L, L->scratch + al(sizeof(WlArgs) * total_w), 1, st);
+  if (rc) return rc;
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
@@ -692,29 +741,27 @@ int bwl_server_submit_ns(bwl_server *s, const bwl_lattice_desc *desc, const doub
   // walkers from the run's own MT19937 stream (nested_sampling.f90:88-96)
   MT19937 mt;
   mt.seed(seed);
-  const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
-  r->walkers_ref.assign(ref * (size_t)p->n_walkers, 0);
-  r->rnde.resize((size_t)p->n_walkers);
-  bool two = false;
-  for (int w = 0; w < p->n_walkers; ++w) {
-    rc = initial_setup_host(g, species_numbers, concentrations, mt, r->walkers_ref.data() + ref * w,
-                            g_err);
-    if (rc) {
-      s->reqs.erase(r->id);
-      return rc;
-    }
-    r->rnde[(size_t)w] = mt.genrand();
-    if (w == 0) {
-      int first = 0;
-      for (size_t i = 0; i < ref && !two; ++i) {
-        const int v = r->walkers_ref[i];
-        if (!v) continue;
-        if (!first) first = v;
-        else if (v != first) two = true;
+  rc = setup_rule(g, species_numbers, concentrations, r->rule, g_err);
+  if (rc) {
+    s->reqs.erase(r->id);
+    return rc;
+  }
+  r->made = !setup_on_device(g, r->rule);
+  if (r->made) {
+    const size_t N = (size_t)g.n_atoms;
+    r->order.resize(N * (size_t)p->n_walkers);
+    r->rnde.resize((size_t)p->n_walkers);
+    for (int w = 0; w < p->n_walkers; ++w) {
+      if (!setup_order(g, r->rule, mt, r->order.data() + N * (size_t)w)) {
+        s->reqs.erase(r->id);
+        return fail(BWL_ERR_ARG, "initial_setup did not terminate");
       }
+      r->rnde[(size_t)w] = mt.genrand();
     }
   }
-  if (!two) {
+  int present = 0;
+  for (int k = 0; k < g.S; ++k) present += r->rule.count[k] > 0;
+  if (present < 2) {
     s->reqs.erase(r->id);
     return fail(BWL_ERR_ARG, "nested sampling needs at least two species present");
   }
@@ -764,18 +811,22 @@ int bwl_server_submit_wl(bwl_server *s, const bwl_lattice_desc *desc, const doub
   }
   // each walker from its own stream, seeded as rank rank_offset + k
   const size_t W = (size_t)p->num_windows * p->walkers_per_window;
-  const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
-  r->walkers_ref.assign(ref * W, 0);
+  rc = setup_rule(g, species_numbers, concentrations, r->rule, g_err);
+  if (rc) {
+    s->reqs.erase(r->id);
+    return rc;
+  }
+  r->made = !setup_on_device(g, r->rule);
+  const size_t N = (size_t)g.n_atoms;
+  if (r->made) r->order.resize(N * W);
   r->wl_mt.resize(W * 624);
-  r->wl_mti.resize(W);
+  r->wl_mti.assign(2 * W, 0);
   for (size_t k = 0; k < W; ++k) {
     MT19937 mt;
     mt.seed(110179u + 11u * (p->rank_offset + (uint32_t)k));
-    rc = initial_setup_host(g, species_numbers, concentrations, mt, r->walkers_ref.data() + ref * k,
-                            g_err);
-    if (rc) {
+    if (r->made && !setup_order(g, r->rule, mt, r->order.data() + N * k)) {
       s->reqs.erase(r->id);
-      return rc;
+      return fail(BWL_ERR_ARG, "initial_setup did not terminate");
     }
     memcpy(&r->wl_mt[624 * k], mt.mt, 624 * 4);
     r->wl_mti[k] = mt.mti;
