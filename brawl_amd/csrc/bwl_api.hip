@@ -91,6 +91,8 @@ int bwl_create(const bwl_lattice_desc *desc, const double *v_ex, bwl_ctx **out) 
     bwl_destroy(c);
     return fail(BWL_ERR_DEVICE, "upload failed");
   }
+  pinned_hold();
+  c->held = true;
   c->mt.seed(110179u);  // f90_init_genrand static seed, rank 0 (mt19937ar.c:138)
   *out = c;
   return BWL_OK;
@@ -110,6 +112,7 @@ int bwl_destroy(bwl_ctx *c) {
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->stream && !c->borrowed) (void)hipStreamDestroy(c->stream);
+  if (c->held) pinned_drop();
   delete c;
   return BWL_OK;
 }
@@ -127,9 +130,18 @@ int bwl_set_config(bwl_ctx *c, const int8_t *config) {
   rc = check_config(c->g, config, g_err);
   if (rc) return rc;
   size_t ref_bytes = (size_t)c->g.m[0] * c->g.m[1] * c->g.m[2];
-  HIP_OK(hipMemcpyAsync(c->d_ref, config, ref_bytes, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(launch_pack(c->d_ref, c->d_compact, c->g, c->stream));
+  Pinned pin;
+  const int8_t *from = c->d_ref;
+  if (ref_bytes <= kPinnedConfig) {
+    if (!pin.take(ref_bytes, c->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+    memcpy(pin.p, config, ref_bytes);
+    from = (const int8_t *)pin.p;
+  } else {
+    HIP_OK(hipMemcpyAsync(c->d_ref, config, ref_bytes, hipMemcpyHostToDevice, c->stream));
+  }
+  HIP_OK(launch_pack(from, c->d_compact, c->g, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
+  pin.settled();
   c->has_config = true;
   return BWL_OK;
 }
@@ -139,9 +151,18 @@ int bwl_get_config(bwl_ctx *c, int8_t *config) {
   if (rc) return rc;
   if (!config) return fail(BWL_ERR_ARG, "null config");
   size_t ref_bytes = (size_t)c->g.m[0] * c->g.m[1] * c->g.m[2];
-  HIP_OK(launch_unpack(c->d_compact, c->d_ref, c->g, c->stream));
-  HIP_OK(hipMemcpyAsync(config, c->d_ref, ref_bytes, hipMemcpyDeviceToHost, c->stream));
+  if (ref_bytes > kPinnedConfig) {
+    HIP_OK(launch_unpack(c->d_compact, c->d_ref, c->g, c->stream));
+    HIP_OK(hipMemcpyAsync(config, c->d_ref, ref_bytes, hipMemcpyDeviceToHost, c->stream));
+    HIP_OK(hipStreamSynchronize(c->stream));
+    return BWL_OK;
+  }
+  Pinned pin;
+  if (!pin.take(ref_bytes, c->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+  HIP_OK(launch_unpack(c->d_compact, (int8_t *)pin.p, c->g, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
+  pin.settled();
+  memcpy(config, pin.p, ref_bytes);
   return BWL_OK;
 }
 
@@ -153,19 +174,21 @@ int bwl_pair_histogram(bwl_ctx *c, int64_t *hist) {
   const int threads = 512;
   if (hist_lds_bytes(g, threads) > (size_t)lds_limit())
     return fail(BWL_ERR_UNSUPPORTED, "lattice does not fit in LDS");
-  const size_t hbytes = sizeof(long long) * g.S * g.S * g.R;
-  rc = ensure_scratch(c, sizeof(HistArgs) + hbytes + 64);
-  if (rc) return rc;
+  const int hsize = g.S * g.S * g.R, blocks = hist_blocks(g);
+  Pinned pin;
+  if (!pin.take(sizeof(uint32_t) * (size_t)hsize * (size_t)blocks, c->stream))
+    return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
   HistArgs a;
   a.g = g;
   a.compact = c->d_compact;
   a.off = c->d_off;
-  a.hist = (long long *)((char *)c->d_scratch + ((sizeof(HistArgs) + 63) & ~63));
-  HIP_OK(hipMemcpyAsync(c->d_scratch, &a, sizeof(a), hipMemcpyHostToDevice, c->stream));
-  HIP_OK(hipMemsetAsync(a.hist, 0, hbytes, c->stream));
-  HIP_OK(launch_histogram((const HistArgs *)c->d_scratch, 1, g, threads, c->stream));
-  HIP_OK(hipMemcpyAsync(hist, a.hist, hbytes, hipMemcpyDeviceToHost, c->stream));
+  a.parts = (uint32_t *)pin.p;
+  HIP_OK(launch_histogram(a, blocks, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
+  pin.settled();
+  for (int i = 0; i < hsize; ++i) hist[i] = 0;
+  for (int k = 0; k < blocks; ++k)
+    for (int i = 0; i < hsize; ++i) hist[i] += a.parts[(size_t)k * hsize + i];
   return BWL_OK;
 }
 
@@ -206,15 +229,15 @@ static int site_pair(bwl_ctx *c, const int32_t *s1, const int32_t *s2, double *o
     if (!occ) return fail(BWL_ERR_ARG, "site is not a lattice site");
     a.x[w] = x; a.y[w] = y; a.z[w] = z;
   }
-  rc = ensure_scratch(c, 64);
-  if (rc) return rc;
+  Pinned pin;
+  if (!pin.take(2 * sizeof(double), c->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
   a.compact = c->d_compact;
-  a.off = c->d_off;
   a.vex = c->d_vex;
-  a.out = (double *)c->d_scratch;
+  a.out = (double *)pin.p;
   HIP_OK(launch_site_energy(a, c->stream));
-  HIP_OK(hipMemcpyAsync(out2, a.out, 2 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
+  pin.settled();
+  memcpy(out2, pin.p, 2 * sizeof(double));
   return BWL_OK;
 }
 
@@ -345,37 +368,41 @@ int bwl_mc_steps(bwl_ctx *c, double beta, int32_t nbr_swap, int64_t n_trials, in
   // the MT state must be initialised (mti == 625 means "seed with 5489")
   if (c->mt.mti == 625) c->mt.seed(5489u);
   const long long n_samples = energies ? n_trials / sample_every : 0;
-  const size_t need = 624 * 4 + 64 + sizeof(long long) + sizeof(double) * (size_t)n_samples + 256;
-  rc = ensure_scratch(c, need);
-  if (rc) return rc;
-  char *base = (char *)c->d_scratch;
+  // the stream and the results lie in pinned memory, but for long series of
+  // energies
+  const size_t e_bytes = sizeof(double) * (size_t)n_samples;
+  const bool e_pinned = e_bytes <= kPinnedSeries;
+  Pinned pin;
+  if (!pin.take(624 * 4 + 64 + (e_pinned ? e_bytes : 0), c->stream))
+    return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+  if (!e_pinned) {
+    rc = ensure_scratch(c, e_bytes);
+    if (rc) return rc;
+  }
   SeqArgs a;
   a.g = g;
   a.compact = c->d_compact;
   a.off = c->d_off;
   a.vex = c->d_vex;
-  a.mt = (uint32_t *)base;
-  a.mt_index = (int32_t *)(base + 624 * 4);
-  a.accepted = (long long *)(base + 624 * 4 + 16);
-  a.energies = n_samples ? (double *)(base + 624 * 4 + 64) : nullptr;
+  a.mt = (uint32_t *)pin.p;
+  a.mt_index = (int32_t *)(pin.p + 624 * 4);
+  a.accepted = (long long *)(pin.p + 624 * 4 + 16);
+  a.energies = !n_samples ? nullptr : e_pinned ? (double *)(pin.p + 624 * 4 + 64) : (double *)c->d_scratch;
   a.beta = beta;
   a.nbr_swap = nbr_swap ? 1 : 0;
   a.n_trials = n_trials;
   a.sample_every = energies ? sample_every : 0;
-  int32_t mti = c->mt.mti;
-  HIP_OK(hipMemcpyAsync(a.mt, c->mt.mt, 624 * 4, hipMemcpyHostToDevice, c->stream));
-  HIP_OK(hipMemcpyAsync(a.mt_index, &mti, 4, hipMemcpyHostToDevice, c->stream));
+  memcpy(a.mt, c->mt.mt, 624 * 4);
+  *a.mt_index = c->mt.mti;
   HIP_OK(launch_metro_seq(a, pick, c->stream));
-  long long acc = 0;
-  HIP_OK(hipMemcpyAsync(c->mt.mt, a.mt, 624 * 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(&mti, a.mt_index, 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(&acc, a.accepted, sizeof(acc), hipMemcpyDeviceToHost, c->stream));
-  if (n_samples)
-    HIP_OK(hipMemcpyAsync(energies, a.energies, sizeof(double) * n_samples, hipMemcpyDeviceToHost,
-                          c->stream));
+  if (n_samples && !e_pinned)
+    HIP_OK(hipMemcpyAsync(energies, a.energies, e_bytes, hipMemcpyDeviceToHost, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
-  c->mt.mti = mti;
-  if (accepted) *accepted = acc;
+  pin.settled();
+  memcpy(c->mt.mt, a.mt, 624 * 4);
+  c->mt.mti = *a.mt_index;
+  if (n_samples && e_pinned) memcpy(energies, a.energies, e_bytes);
+  if (accepted) *accepted = *a.accepted;
   return BWL_OK;
 }
 
@@ -401,21 +428,28 @@ int bwl_mc_steps_batch(int32_t n, bwl_ctx *const *ctxs, const double *beta, int3
   // per chain: MT state, index, accepted count, sampled energies
   const long long n_samples = energies ? n_trials / sample_every : 0;
   const size_t stride = ((624 * 4 + 64 + sizeof(double) * (size_t)n_samples) + 255) & ~(size_t)255;
-  const size_t args_bytes = (sizeof(SeqArgs) * (size_t)n + 255) & ~(size_t)255;
-  DevBuf buf;
-  if (hipMalloc(&buf.p, args_bytes + stride * (size_t)n) != hipSuccess)
-    return fail(BWL_ERR_NOMEM, "device allocation failed");
-  char *base = (char *)buf.p;
-  std::vector<SeqArgs> args((size_t)n);
-  std::vector<char> host(stride * (size_t)n, 0);
+  const size_t args_bytes = (sizeof(SeqArgs) * (size_t)n + 255) & ~(size_t)255, io_bytes = stride * (size_t)n;
+  hipStream_t s = ctxs[0]->stream;
+  // the chains' arguments on the device; their streams and results in pinned
+  // memory unless there are many
+  const bool io_pinned = io_bytes <= kPinnedSeries;
+  Pinned pin;
+  if (!pin.take(args_bytes + (io_pinned ? io_bytes : 0), s)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+  int rc_s = ensure_scratch(ctxs[0], args_bytes + (io_pinned ? 0 : io_bytes));
+  if (rc_s) return rc_s;
+  char *base = (char *)ctxs[0]->d_scratch;
+  std::vector<char> far(io_pinned ? 0 : io_bytes);
+  char *const host = io_pinned ? pin.p + args_bytes : far.data();  // the streams and results here,
+  char *const io = io_pinned ? host : base + args_bytes;           // and where the kernel finds them
+  SeqArgs *args = (SeqArgs *)pin.p;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
     if (c->mt.mti == 625) c->mt.seed(5489u);
-    HIP_OK(hipStreamSynchronize(c->stream));  // the chain's own earlier work
-    char *h = host.data() + stride * (size_t)i;
+    if (i > 0) HIP_OK(hipStreamSynchronize(c->stream));  // the chain's own earlier work
+    char *h = host + stride * (size_t)i;
     memcpy(h, c->mt.mt, 624 * 4);
     memcpy(h + 624 * 4, &c->mt.mti, 4);
-    char *d = base + args_bytes + stride * (size_t)i;
+    char *d = io + stride * (size_t)i;
     SeqArgs &a = args[(size_t)i];
     a.g = c->g;
     a.compact = c->d_compact;
@@ -430,20 +464,20 @@ int bwl_mc_steps_batch(int32_t n, bwl_ctx *const *ctxs, const double *beta, int3
     a.n_trials = n_trials;
     a.sample_every = energies ? sample_every : 0;
   }
-  hipStream_t s = ctxs[0]->stream;
-  HIP_OK(hipMemcpyAsync(base, args.data(), sizeof(SeqArgs) * (size_t)n, hipMemcpyHostToDevice, s));
-  HIP_OK(hipMemcpyAsync(base + args_bytes, host.data(), host.size(), hipMemcpyHostToDevice, s));
+  HIP_OK(hipMemcpyAsync(base, args, sizeof(SeqArgs) * (size_t)n, hipMemcpyHostToDevice, s));
+  if (!io_pinned) HIP_OK(hipMemcpyAsync(io, host, io_bytes, hipMemcpyHostToDevice, s));
   HIP_OK(hipEventRecord(ctxs[0]->ev0, s));
   HIP_OK(launch_metro_seq_batch((const SeqArgs *)base, n, pick, s));
   HIP_OK(hipEventRecord(ctxs[0]->ev1, s));
-  HIP_OK(hipMemcpyAsync(host.data(), base + args_bytes, host.size(), hipMemcpyDeviceToHost, s));
+  if (!io_pinned) HIP_OK(hipMemcpyAsync(host, io, io_bytes, hipMemcpyDeviceToHost, s));
   HIP_OK(hipStreamSynchronize(s));
+  pin.settled();
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, ctxs[0]->ev0, ctxs[0]->ev1);
   if (kernel_ms) *kernel_ms = ms;
   for (int i = 0; i < n; ++i) {
     bwl_ctx *c = ctxs[i];
-    const char *h = host.data() + stride * (size_t)i;
+    const char *h = host + stride * (size_t)i;
     memcpy(c->mt.mt, h, 624 * 4);
     memcpy(&c->mt.mti, h + 624 * 4, 4);
     long long acc = 0;

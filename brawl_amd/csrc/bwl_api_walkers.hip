@@ -163,23 +163,32 @@ int bwl_radial_densities(bwl_ctx *c, int32_t wc_range, double *rho) {
   asro_offsets_host(g, wc_range, shells.data(), off3, a.shell_start);
   const int S = g.S;
   const size_t hn = (size_t)S * S * wc_range;
-  rc = ensure_scratch(c, align256(sizeof(unsigned long long) * hn) + sizeof(int32_t) * (off3.size() + 3));
-  if (rc) return rc;
-  char *base = (char *)c->d_scratch;
+  const size_t entries = off3.size() / 3;
+  std::vector<int32_t> packed(entries);
+  for (size_t t = 0; t < entries; ++t)
+    packed[t] = (off3[3 * t] & 0xff) | ((off3[3 * t + 1] & 0xff) << 8) | ((off3[3 * t + 2] & 0xff) << 16);
+  const int blocks = asro_blocks(g, wc_range);
+  Pinned pin;
+  if (!pin.take(sizeof(uint32_t) * hn * (size_t)blocks, c->stream))
+    return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
   a.g = g;
   a.compact = c->d_compact;
   a.wc = wc_range;
-  a.hist = (unsigned long long *)base;
-  a.off = (const int32_t *)(base + align256(sizeof(unsigned long long) * hn));
-  HIP_OK(hipMemsetAsync(a.hist, 0, sizeof(unsigned long long) * hn, c->stream));
-  if (!off3.empty())
-    HIP_OK(hipMemcpyAsync((void *)a.off, off3.data(), sizeof(int32_t) * off3.size(),
-                          hipMemcpyHostToDevice, c->stream));
-  HIP_OK(launch_asro(a, c->stream));
-  std::vector<unsigned long long> h(hn);
-  HIP_OK(hipMemcpyAsync(h.data(), a.hist, sizeof(unsigned long long) * hn, hipMemcpyDeviceToHost,
-                        c->stream));
+  a.parts = (uint32_t *)pin.p;
+  if (entries <= (size_t)kAsroNear) {
+    std::copy(packed.begin(), packed.end(), a.near);
+  } else {
+    rc = ensure_scratch(c, sizeof(int32_t) * entries);
+    if (rc) return rc;
+    a.off = (const int32_t *)c->d_scratch;
+    HIP_OK(hipMemcpyAsync(c->d_scratch, packed.data(), sizeof(int32_t) * entries, hipMemcpyHostToDevice, c->stream));
+  }
+  HIP_OK(launch_asro(a, blocks, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
+  pin.settled();
+  std::vector<unsigned long long> h(hn, 0);
+  for (int k = 0; k < blocks; ++k)
+    for (size_t i = 0; i < hn; ++i) h[i] += a.parts[(size_t)k * hn + i];
   // the on-site shell (distance 0, offset 0 only) counts each species
   for (int l = 0; l < wc_range; ++l)
     for (int b = 0; b < S; ++b)

@@ -11,6 +11,7 @@
 #include "../../include/brawl_hip.h"
 #include "bwl_host.h"
 #include "bwl_kernels.h"
+#include "bwl_pinned.h"
 
 namespace bwl {
 // message of the last failure on this thread (bwl_last_error)
@@ -46,12 +47,18 @@ struct bwl_ctx {
   bwl::MT19937 mt;
   unsigned long long phase = 0;  // parallel-sampler round counter
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  bool held = false;      // counted by pinned_hold
   bool borrowed = false;  // device memory and stream belong to someone else
   int32_t layout = 0;     // parallel-sampler layout: 0 by rule, else BWL_LAYOUT_*
   int32_t threads = 0;    // parallel-sampler threads per chain: 0 by rule
 };
 
 namespace bwl {
+
+// Most bytes of streams and results that a call keeps in pinned memory.
+constexpr size_t kPinnedSeries = size_t(4) << 20;
+// Largest configuration (reference layout) that goes through pinned memory.
+constexpr size_t kPinnedConfig = size_t(16) << 20;
 
 inline int ensure_scratch(bwl_ctx *c, size_t bytes) {
   if (bytes <= c->scratch_bytes) return BWL_OK;

@@ -13,13 +13,12 @@ struct HistArgs {
   Geo g;
   const int8_t *compact;  // lattice, compact layout
   const int32_t *off;     // [nsub][z] padded-layout neighbour offsets
-  long long *hist;        // H(S,S,R), Fortran layout
+  uint32_t *parts;        // out: H(S,S,R), Fortran layout, of each block's sites
 };
 
 struct SiteArgs {
   Geo g;
   const int8_t *compact;
-  const int32_t *off;
   const double *vex;  // V_ex(S,S,R)
   int x[2], y[2], z[2];  // 0-based doubled coordinates of two sites
   double *out;           // out[0] = e(site 0), out[1] = e(site 0) + e(site 1)
@@ -177,13 +176,17 @@ struct WlEnterArgs {
 };
 
 // Windowed pair-count histogram of radial_densities (analytics.f90:293-404).
+constexpr int kAsroNear = 256;
 struct AsroArgs {
   Geo g;
   const int8_t *compact;
   int32_t wc;                 // shells including the on-site one
   int32_t shell_start[17];    // offsets of shell l: [shell_start[l], shell_start[l+1])
-  const int32_t *off;         // 3 ints (dx, dy, dz) per entry, doubled-grid units
-  unsigned long long *hist;   // H(S, S, wc), zeroed by the caller
+  // (dx, dy, dz) of an entry in doubled-grid units, a signed byte each from
+  // the lowest: `near` where they fit, else `off`
+  const int32_t *off;
+  int32_t near[kAsroNear];
+  uint32_t *parts;            // out: H(S, S, wc) of each block's sites
 };
 constexpr int kMaxAsroShells = 16;
 
@@ -196,9 +199,11 @@ hipError_t launch_setup(const SetupArgs *args_dev, int n, int max_walkers, int m
 hipError_t launch_unpack(const int8_t *compact, int8_t *ref, const Geo &g, hipStream_t s);
 // LDS read-bandwidth probe: blocks x 1024 threads, iters 16-byte reads each
 hipError_t launch_lds_bandwidth(int blocks, int iters, uint32_t *sink, hipStream_t s);
+// LDS of a lattice held whole beside its tables: larger ones are refused by
+// the calls that measure a configuration
 size_t hist_lds_bytes(const Geo &g, int threads);
-hipError_t launch_histogram(const HistArgs *args_dev, int n, const Geo &g_max, int threads,
-                            hipStream_t s);
+int hist_blocks(const Geo &g);
+hipError_t launch_histogram(const HistArgs &a, int blocks, hipStream_t s);
 size_t site_lds_bytes(const Geo &g);
 hipError_t launch_site_energy(const SiteArgs &a, hipStream_t s);
 // The kernel of a launch of sequential chains and its LDS, from its members.
@@ -295,6 +300,7 @@ hipError_t launch_wl_swap_configs(int8_t *walkers, long long bytes, const int32_
                                   const int32_t *n_swaps, int max_pairs, hipStream_t s);
 size_t wl_enter_lds_bytes(const Geo &g);
 hipError_t launch_wl_enter(const WlEnterArgs *args_dev, int n, size_t lds, hipStream_t s, int key);
-hipError_t launch_asro(const AsroArgs &a, hipStream_t s);
+int asro_blocks(const Geo &g, int wc);
+hipError_t launch_asro(const AsroArgs &a, int blocks, hipStream_t s);
 
 }  // namespace bwl

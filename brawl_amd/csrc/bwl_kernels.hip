@@ -19,79 +19,105 @@ namespace bwl {
 // ------------------------------------------------------------------
 // layout conversion
 // ------------------------------------------------------------------
+// Eight cells of the reference layout a thread, in one access: `ref` may be
+// pinned host memory, where each access is a transfer of its own.  (The cells
+// of a lattice are a multiple of 8: every extent is even.)
+struct RefWalk {  // cells of the doubled grid in memory order
+  int x, y, z;
+};
+__device__ inline RefWalk ref_walk(const Geo &g, int idx) {
+  const int r = idx / g.m[0], z = r / g.m[1];
+  return RefWalk{idx - r * g.m[0], r - z * g.m[1], z};
+}
+__device__ inline void ref_step(const Geo &g, RefWalk &w) {
+  if (++w.x < g.m[0]) return;
+  w.x = 0;
+  if (++w.y < g.m[1]) return;
+  w.y = 0;
+  ++w.z;
+}
+__device__ inline bool ref_site(const Geo &g, const RefWalk &w) {
+  return g.lattice == 1 ? ((w.x + w.y + w.z) & 1) == 0 : ((w.x ^ w.y) & 1) == 0 && ((w.y ^ w.z) & 1) == 0;
+}
+__device__ inline int ref_to_compact(const Geo &g, const RefWalk &w) {
+  return compact_addr(g, sub_of(g.lattice, w.x & 1, w.y & 1), w.x >> 1, w.y >> 1, w.z >> 1);
+}
+
 __global__ void k_pack(const int8_t *__restrict__ ref, int8_t *__restrict__ compact, Geo g) {
   // blockIdx.y selects one of several lattices laid out back to back
-  ref += (size_t)blockIdx.y * g.m[0] * g.m[1] * g.m[2];
+  const int total = g.m[0] * g.m[1] * g.m[2];
+  ref += (size_t)blockIdx.y * total;
   compact += (size_t)blockIdx.y * g.compact_bytes;
-  const int cells = g.n[0] * g.n[1] * g.n[2];
-  const int total = g.nsub * cells;
-  for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += gridDim.x * blockDim.x) {
-    int s = idx / cells;
-    int r = idx - s * cells;
-    int cz = r / (g.n[0] * g.n[1]);
-    r -= cz * g.n[0] * g.n[1];
-    int cy = r / g.n[0];
-    int cx = r - cy * g.n[0];
-    int bx, by, bz;
-    sub_bits(g.lattice, s, bx, by, bz);
-    int x = 2 * cx + bx, y = 2 * cy + by, z = 2 * cz + bz;
-    compact[idx] = ref[x + g.m[0] * (y + g.m[1] * z)];
+  for (int idx = 8 * (blockIdx.x * blockDim.x + threadIdx.x); idx < total; idx += 8 * gridDim.x * blockDim.x) {
+    const uint64_t v = *(const uint64_t *)(ref + idx);
+    RefWalk w = ref_walk(g, idx);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (ref_site(g, w)) compact[ref_to_compact(g, w)] = (int8_t)(v >> (8 * k));
+      ref_step(g, w);
+    }
   }
 }
 
 __global__ void k_unpack(const int8_t *__restrict__ compact, int8_t *__restrict__ ref, Geo g) {
   const int total = g.m[0] * g.m[1] * g.m[2];
-  for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += gridDim.x * blockDim.x) {
-    int x = idx % g.m[0];
-    int y = (idx / g.m[0]) % g.m[1];
-    int z = idx / (g.m[0] * g.m[1]);
-    bool occ = g.lattice == 1 ? (((x + y + z) & 1) == 0)
-                              : ((x & 1) == (y & 1) && (y & 1) == (z & 1));
-    int8_t v = 0;
-    if (occ)
-      v = compact[compact_addr(g, sub_of(g.lattice, x & 1, y & 1), x >> 1, y >> 1, z >> 1)];
-    ref[idx] = v;
+  for (int idx = 8 * (blockIdx.x * blockDim.x + threadIdx.x); idx < total; idx += 8 * gridDim.x * blockDim.x) {
+    RefWalk w = ref_walk(g, idx);
+    uint64_t v = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if (ref_site(g, w)) v |= (uint64_t)(uint8_t)compact[ref_to_compact(g, w)] << (8 * k);
+      ref_step(g, w);
+    }
+    *(uint64_t *)(ref + idx) = v;
   }
 }
 
 // ------------------------------------------------------------------
 // pair-count histogram: H[n][b][a] += number of shell-n neighbours of
 // species b around sites of species a (Fortran H(a,b,n) layout).
-// Block (x, y) stages lattice y whole in LDS and counts the x-th of
-// gridDim.x equal slices of its sites into per-wave private copies in LDS;
-// the block's sums are added to the (zeroed) output with 64-bit atomics.
-// Integer sums: the result does not depend on the slicing.
+// A block counts part of one plane of cells (all sublattices) on the planes
+// within the halo's reach, staged in LDS; the staging of the lattice bounded
+// it when every block held it whole (bcc 32^3, four shells: 122 us in 32
+// blocks, 21 here in 256).  The block's counts go to its own part of the
+// output, which the host adds up: integers, so the split does not show.
 // ------------------------------------------------------------------
-__global__ __launch_bounds__(512) void k_histogram(const HistArgs *__restrict__ args) {
+constexpr int kHistThreads = 256;
+
+__global__ __launch_bounds__(kHistThreads) void k_histogram(HistArgs A, int per_plane) {
   extern __shared__ __align__(16) uint8_t smem[];
-  const HistArgs &A = args[blockIdx.y];
   const Geo &g = A.g;
   int8_t *lat = (int8_t *)smem;
   const int hsize = g.S * g.S * g.R;
-  const int nw = blockDim.x >> 6;
-  uint32_t *hw = (uint32_t *)(smem + ((g.lds_bytes + 15) & ~15));
+  constexpr int nw = kHistThreads / 64;
+  const int plane = g.P[0] * g.P[1], planes = 2 * g.h + 1, slab = plane * planes;
+  uint32_t *hw = (uint32_t *)(smem + ((g.nsub * slab + 15) & ~15));
   int32_t *offl = (int32_t *)(hw + hsize * nw);
-  for (int i = threadIdx.x; i < hsize * nw; i += blockDim.x) hw[i] = 0;
-  stage_offsets(offl, A.off, g);
-  stage_lattice(lat, A.compact, g, 0);
+  for (int i = threadIdx.x; i < hsize * nw; i += kHistThreads) hw[i] = 0;
+  // offsets (ds * sub_stride + rest, |rest| < sub_stride / 2) in the slab's
+  // shorter sublattices
+  for (int i = threadIdx.x; i < g.nsub * g.z; i += kHistThreads) {
+    const int o = A.off[i] + g.nsub * g.sub_stride + g.sub_stride / 2;
+    const int ds = o / g.sub_stride - g.nsub;
+    offl[i] = A.off[i] + ds * (slab - g.sub_stride);
+  }
+  const int cz = blockIdx.x / per_plane, part = blockIdx.x - cz * per_plane;
+  for (int i = threadIdx.x; i < g.nsub * slab; i += kHistThreads) {
+    const int s = i / slab;
+    int r = i - s * slab;
+    const int pz = r / plane;
+    r -= pz * plane;
+    const int py = r / g.P[0], px = r - py * g.P[0];
+    lat[i] = A.compact[compact_addr(g, s, pmod(px - g.h, g.n[0]), pmod(py - g.h, g.n[1]), pmod(cz + pz - g.h, g.n[2]))];
+  }
   __syncthreads();
   uint32_t *mine = hw + (threadIdx.x >> 6) * hsize;
-  const int cells = g.n[0] * g.n[1] * g.n[2];
-  const int nsites = g.nsub * cells;
-  const int per = (nsites + gridDim.x - 1) / gridDim.x;
-  const int i0 = blockIdx.x * per;
-  const int i1 = i0 + per < nsites ? i0 + per : nsites;
-  for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    int s = i / cells;
-    int r = i - s * cells;
-    int cz = r / (g.n[0] * g.n[1]);
-    r -= cz * g.n[0] * g.n[1];
-    int cy = r / g.n[0];
-    int cx = r - cy * g.n[0];
-    int addr = padded_addr(g, s, cx, cy, cz);
-    int a = lat[addr];
+  const int cells = g.n[0] * g.n[1], nsites = g.nsub * cells;
+  for (int i = part * kHistThreads + threadIdx.x; i < nsites; i += per_plane * kHistThreads) {
+    const int s = i / cells, r = i - s * cells;
+    const int cy = r / g.n[0], cx = r - cy * g.n[0];
+    const int addr = s * slab + g.h * plane + (cy + g.h) * g.P[0] + cx + g.h;
+    const int a = lat[addr];
     if (a <= 0) continue;
     const int32_t *off = offl + s * g.z;
     for (int n = 0; n < g.R; ++n) {
@@ -100,37 +126,47 @@ __global__ __launch_bounds__(512) void k_histogram(const HistArgs *__restrict__ 
       for (int t = g.shell_start[n]; t < g.shell_start[n + 1]; ++t)
         c += (uint64_t)1 << (8 * (lat[addr + off[t]] - 1));
       for (int b = 0; b < g.S; ++b) {
-        uint32_t k = (uint32_t)(c >> (8 * b)) & 0xffu;
+        const uint32_t k = (uint32_t)(c >> (8 * b)) & 0xffu;
         if (k) atomicAdd(&mine[(a - 1) + g.S * (b + g.S * n)], k);
       }
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < hsize; i += blockDim.x) {
-    unsigned long long t = 0;
+  for (int i = threadIdx.x; i < hsize; i += kHistThreads) {
+    uint32_t t = 0;
     for (int w = 0; w < nw; ++w) t += hw[w * hsize + i];
-    if (t) atomicAdd((unsigned long long *)&A.hist[i], t);
+    A.parts[(size_t)blockIdx.x * hsize + i] = t;
   }
 }
 
+// Energies of two sites, one wavefront: each lane gathers its neighbours from
+// the lattice as it lies in memory (2 z bytes of it are wanted, so none is
+// staged), then the entries are added in the reference's order.
 __global__ __launch_bounds__(64) void k_site_energy(SiteArgs A) {
-  extern __shared__ __align__(16) uint8_t smem[];
   const Geo &g = A.g;
-  int8_t *lat = (int8_t *)smem;
-  double *vex = (double *)(smem + ((g.lds_bytes + 15) & ~15));
-  int32_t *offl = (int32_t *)(vex + g.S * g.S * g.R);
-  for (int i = threadIdx.x; i < g.S * g.S * g.R; i += blockDim.x) vex[i] = A.vex[i];
-  stage_offsets(offl, A.off, g);
   PairLanes pl;
   init_pair_lanes(g, pl);
-  stage_lattice(lat, A.compact, g, 0);
-  __syncthreads();
+  auto at = [&](int x, int y, int z) {
+    return (int)A.compact[compact_addr(g, sub_of(g.lattice, x & 1, y & 1), x >> 1, y >> 1, z >> 1)];
+  };
+  const int sp0 = at(A.x[0], A.y[0], A.z[0]), sp1 = at(A.x[1], A.y[1], A.z[1]);
+  double vals[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    vals[k] = 0.0;
+    const int t = 64 * k + (int)threadIdx.x;
+    if (k < pl.passes && t < 2 * g.z) {
+      const int w = t < g.z ? 0 : 1;
+      // the offset mod the box is below the extent: one subtraction wraps
+      int x = A.x[w] + (pl.dmod[k] & 1023), y = A.y[w] + ((pl.dmod[k] >> 10) & 1023), z = A.z[w] + (pl.dmod[k] >> 20);
+      x -= x >= g.m[0] ? g.m[0] : 0;
+      y -= y >= g.m[1] ? g.m[1] : 0;
+      z -= z >= g.m[2] ? g.m[2] : 0;
+      vals[k] = A.vex[((w ? sp1 : sp0) - 1) + g.S * ((at(x, y, z) - 1) + g.S * pl.shell[k])];
+    }
+  }
   double eA = 0.0;
-  int addrA = padded_addr_xyz(g, A.x[0], A.y[0], A.z[0]);
-  int addrB = padded_addr_xyz(g, A.x[1], A.y[1], A.z[1]);
-  int subA = sub_of(g.lattice, A.x[0] & 1, A.y[0] & 1);
-  int subB = sub_of(g.lattice, A.x[1] & 1, A.y[1] & 1);
-  double e = pair_energy_lanes(lat, g, offl, vex, pl, addrA, subA, addrB, subB, &eA);
+  const double e = pair_sum(g, pl, vals, &eA);
   if (threadIdx.x == 0) {
     A.out[0] = eA;
     A.out[1] = e;
@@ -411,7 +447,7 @@ hipError_t launch_pack(const int8_t *ref, int8_t *compact, const Geo &g, hipStre
 
 hipError_t launch_pack_many(const int8_t *ref, int8_t *compact, const Geo &g, int count,
                             hipStream_t s) {
-  int total = g.compact_bytes;
+  int total = g.m[0] * g.m[1] * g.m[2] / 8;
   int blocks = (total + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   for (int first = 0; first < count; first += 65535) {
@@ -424,7 +460,7 @@ hipError_t launch_pack_many(const int8_t *ref, int8_t *compact, const Geo &g, in
 }
 
 hipError_t launch_unpack(const int8_t *compact, int8_t *ref, const Geo &g, hipStream_t s) {
-  int total = g.m[0] * g.m[1] * g.m[2];
+  int total = g.m[0] * g.m[1] * g.m[2] / 8;
   int blocks = (total + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(k_unpack, dim3(blocks), dim3(256), 0, s, compact, ref, g);
@@ -436,18 +472,22 @@ size_t hist_lds_bytes(const Geo &g, int threads) {
          sizeof(int32_t) * g.nsub * g.z;
 }
 
-hipError_t launch_histogram(const HistArgs *args_dev, int n, const Geo &g_max, int threads,
-                            hipStream_t s) {
-  size_t lds = hist_lds_bytes(g_max, threads);
-  hipError_t e = hipFuncSetAttribute((const void *)k_histogram,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  // slices of about 2048 sites (each block restages the lattice, from L2)
-  const int nsites = g_max.nsub * g_max.n[0] * g_max.n[1] * g_max.n[2];
-  int parts = nsites / 2048;
-  parts = parts < 1 ? 1 : (parts > 256 ? 256 : parts);
-  hipLaunchKernelGGL(k_histogram, dim3(parts, n), dim3(threads), lds, s, args_dev);
-  return hipGetLastError();
+// blocks of about 256 sites, at most 8 to a plane of cells
+static int hist_per_plane(const Geo &g) {
+  const int q = (g.nsub * g.n[0] * g.n[1] + kHistThreads - 1) / kHistThreads;
+  return q < 8 ? q : 8;
+}
+
+int hist_blocks(const Geo &g) { return hist_per_plane(g) * g.n[2]; }
+
+hipError_t launch_histogram(const HistArgs &a, int blocks, hipStream_t s) {
+  const Geo &g = a.g;
+  const size_t lds = (size_t)((g.nsub * g.P[0] * g.P[1] * (2 * g.h + 1) + 15) & ~15) +
+                     sizeof(uint32_t) * g.S * g.S * g.R * (kHistThreads / 64) + sizeof(int32_t) * g.nsub * g.z;
+  HistArgs arg = a;
+  int per_plane = hist_per_plane(g);
+  void *kargs[] = {(void *)&arg, (void *)&per_plane};
+  return launch_dynamic((const void *)k_histogram, dim3(blocks), kHistThreads, kargs, lds, s);
 }
 
 size_t site_lds_bytes(const Geo &g) {
@@ -456,11 +496,7 @@ size_t site_lds_bytes(const Geo &g) {
 }
 
 hipError_t launch_site_energy(const SiteArgs &a, hipStream_t s) {
-  size_t lds = site_lds_bytes(a.g);
-  hipError_t e = hipFuncSetAttribute((const void *)k_site_energy,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_site_energy, dim3(1), dim3(64), lds, s, a);
+  hipLaunchKernelGGL(k_site_energy, dim3(1), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 

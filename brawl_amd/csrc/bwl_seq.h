@@ -37,7 +37,7 @@ __device__ inline void stage_offsets(int32_t *dst, const int32_t *__restrict__ s
   for (int i = threadIdx.x; i < g.nsub * g.z; i += blockDim.x) dst[i] = src[i];
 }
 
-// Per-lane constants of pair_energy_lanes, computed once per kernel: the
+// Per-lane constants of the pair sums, computed once per kernel: the
 // shell of each lane's entries and, per 64-entry pass, the mask of entries
 // that end a shell.  Entries 0..z-1 are site A's neighbours in list order,
 // z..2z-1 site B's.
@@ -86,7 +86,7 @@ __host__ __device__ constexpr int shell_max(int lattice, int r) {
   return m;
 }
 
-// The ordered sum of pair_energy_lanes with the shell structure known at
+// The ordered sum of pair_sum with the shell structure known at
 // compile time: straight-line readlane/add code, no loop or branches.
 template <int LAT, int R>
 __device__ __forceinline__ double fixed_pair_sum(const double (&vals)[6], double *eA_out) {
@@ -150,7 +150,7 @@ __device__ inline void init_pair_lanes(const Geo &g, PairLanes &pl) {
   pl.fixed = pair_sum_key(g.lattice, g.R);
 }
 
-// The ordered sum of pair_energy_lanes from the lanes' values (entries
+// The ordered sum of a pair energy (pair_energy, bw_hamiltonian.f90:99-114) from the lanes' values (entries
 // 0..z-1 site A's, z..2z-1 site B's): e_A + e_B, each site's shells left to
 // right, each shell from 0.0 in list order.
 template <class GEO>
@@ -331,34 +331,6 @@ __device__ inline void pair_sum2_t(const GEO &g, const PairLanes &pl, const doub
     case 32 + 4: return (const void *)kern<32 + 4>;       \
     default: return nullptr;                              \
   }
-
-// Energies of sites A and B in the reference's FP64 order (pair_energy,
-// bw_hamiltonian.f90:99-114): every lane gathers neighbour V entries (one
-// per 64-entry pass), then the entries are added in list order from 0.0
-// per shell, shells left to right per site, and e_A + e_B -- on every lane,
-// from the lanes' values.  `off` is the offset table and `vex` V_ex, both
-// in LDS.
-__device__ inline double pair_energy_lanes(const int8_t *lat, const Geo &g, const int32_t *off,
-                                           const double *vex, const PairLanes &pl, int addrA,
-                                           int subA, int addrB, int subB, double *eA_out) {
-  const int lane = threadIdx.x & 63;
-  const int z = g.z, S = g.S;
-  const int spA = lat[addrA], spB = lat[addrB];
-  double vals[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    vals[k] = 0.0;
-    const int t = 64 * k + lane;
-    if (k < pl.passes && t < 2 * z) {
-      const bool isA = t < z;
-      const int tt = isA ? t : t - z;
-      const int addr = isA ? addrA : addrB, sub = isA ? subA : subB, sp = isA ? spA : spB;
-      const int nb = lat[addr + off[sub * z + tt]];
-      vals[k] = vex[(sp - 1) + S * ((nb - 1) + S * pl.shell[k])];
-    }
-  }
-  return pair_sum(g, pl, vals, eA_out);
-}
 
 // pair_energy of sites A and B (species spA, spB, doubled coordinates sA,
 // sB) before and after the exchange of their species, in the reference's

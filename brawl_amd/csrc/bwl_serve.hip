@@ -158,6 +158,7 @@ struct bwl_server {
   std::unordered_map<int64_t, std::unique_ptr<Request>> reqs;
   std::vector<int64_t> done_unpolled;
   int64_t next_id = 1;
+  bool held = false;  // counted by pinned_hold
   double batch_wait_ms = 0.0;
   std::chrono::steady_clock::time_point t0;
 };
@@ -662,6 +663,8 @@ int bwl_server_create(const bwl_server_params *p, bwl_server **out) {
   }
   s->batch_wait_ms = p->batch_wait_us / 1000.0;
   s->t0 = std::chrono::steady_clock::now();
+  pinned_hold();
+  s->held = true;
   *out = s.release();
   return BWL_OK;
 }
@@ -678,6 +681,7 @@ int bwl_server_destroy(bwl_server *s) {
     if (kv.second->ctx) bwl_destroy(kv.second->ctx);
   for (hipStream_t st : s->streams) (void)hipStreamDestroy(st);
   if (s->arena_mem) (void)hipFree(s->arena_mem);
+  if (s->held) pinned_drop();
   delete s;
   return BWL_OK;
 }

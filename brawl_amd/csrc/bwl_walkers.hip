@@ -1259,10 +1259,11 @@ __global__ __launch_bounds__(64) void k_wl_enter(const WlEnterArgs *__restrict__
 // species a and every window offset whose minimum-image distance falls on
 // shell l, the species b at that offset: H(a, b, l) += 1.  The lattice is
 // read from HBM (it is small and stays in L2); counts are packed 8 bits per
-// species per shell and flushed to a per-block LDS histogram, then added to
-// the global one with 64-bit atomics (integer sums, so the result does not
-// depend on the order).
+// species per shell and flushed to a per-block LDS histogram, which goes to
+// the block's part of the output (the host adds the parts up: integers, so
+// the split does not show).
 // ------------------------------------------------------------------
+template <bool NEAR>
 __global__ __launch_bounds__(256) void k_asro(AsroArgs A) {
   __shared__ unsigned int lh[kMaxSpecies * kMaxSpecies * kMaxAsroShells];
   const Geo &g = A.g;
@@ -1289,7 +1290,8 @@ __global__ __launch_bounds__(256) void k_asro(AsroArgs A) {
       uint64_t c = 0;
       int k = 0;
       for (int t = A.shell_start[l]; t < A.shell_start[l + 1]; ++t) {
-        int xx = x + A.off[3 * t], yy = y + A.off[3 * t + 1], zz = z + A.off[3 * t + 2];
+        const int32_t d = NEAR ? A.near[t] : A.off[t];
+        int xx = x + (int8_t)d, yy = y + (int8_t)(d >> 8), zz = z + (int8_t)(d >> 16);
         xx = xx < 0 ? xx + g.m[0] : (xx >= g.m[0] ? xx - g.m[0] : xx);
         yy = yy < 0 ? yy + g.m[1] : (yy >= g.m[1] ? yy - g.m[1] : yy);
         zz = zz < 0 ? zz + g.m[2] : (zz >= g.m[2] ? zz - g.m[2] : zz);
@@ -1309,7 +1311,7 @@ __global__ __launch_bounds__(256) void k_asro(AsroArgs A) {
   }
   __syncthreads();
   for (int i = threadIdx.x; i < hsize; i += blockDim.x)
-    if (lh[i]) atomicAdd(&A.hist[i], (unsigned long long)lh[i]);
+    A.parts[(size_t)blockIdx.x * hsize + i] = lh[i];
 }
 
 // ------------------------------------------------------------------
@@ -1416,11 +1418,18 @@ hipError_t launch_wl_enter(const WlEnterArgs *args_dev, int n, size_t lds, hipSt
   return hipLaunchKernel(fn, dim3(n), dim3(64), kargs, lds, s);
 }
 
-hipError_t launch_asro(const AsroArgs &a, hipStream_t s) {
-  const int nsites = a.g.nsub * a.g.n[0] * a.g.n[1] * a.g.n[2];
-  int blocks = (nsites + 255) / 256;
-  if (blocks > 1024) blocks = 1024;
-  hipLaunchKernelGGL(k_asro, dim3(blocks), dim3(256), 0, s, a);
+// blocks of 256 sites or more, at most 1024 with at most 2^18 counts between
+// them
+int asro_blocks(const Geo &g, int wc) {
+  const int b = (g.nsub * g.n[0] * g.n[1] * g.n[2] + 255) / 256, most = (1 << 18) / (g.S * g.S * wc);
+  return b < most ? (b < 1024 ? b : 1024) : (most < 1024 ? most : 1024);
+}
+
+hipError_t launch_asro(const AsroArgs &a, int blocks, hipStream_t s) {
+  if (a.off)
+    hipLaunchKernelGGL(k_asro<false>, dim3(blocks), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_asro<true>, dim3(blocks), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
