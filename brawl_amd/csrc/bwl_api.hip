@@ -102,6 +102,7 @@ int bwl_destroy(bwl_ctx *c) {
   if (!c) return BWL_OK;
   (void)hipSetDevice(c->device);
   if (c->stream && !c->borrowed) (void)hipStreamSynchronize(c->stream);
+  for (hipStream_t s : c->side) (void)hipStreamDestroy(s);
   if (!c->borrowed) {
     (void)hipFree(c->d_compact);
     (void)hipFree(c->d_ref);
@@ -563,8 +564,13 @@ size_t ctx_device_bytes(const bwl_lattice_desc &d) {
          a(sizeof(double) * (size_t)g.S * g.S * g.R);
 }
 
+size_t ctx_tables_bytes(const Geo &g) {
+  auto a = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  return a(sizeof(int32_t) * (size_t)g.nsub * g.z) + sizeof(double) * (size_t)g.S * g.S * g.R;
+}
+
 int ctx_create_borrowed(const bwl_lattice_desc &d, const double *v_ex, char *mem, size_t bytes,
-                        hipStream_t stream, bwl_ctx **out) {
+                        hipStream_t stream, char *tables, bwl_ctx **out) {
   *out = nullptr;
   bwl_ctx *c = new bwl_ctx();
   c->desc = d;
@@ -591,11 +597,11 @@ int ctx_create_borrowed(const bwl_lattice_desc &d, const double *v_ex, char *mem
   q += a(sizeof(int32_t) * c->off.size());
   c->d_vex = (double *)q;
   c->stream = stream;
-  bool ok = hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess &&
-            hipMemcpyAsync(c->d_off, c->off.data(), sizeof(int32_t) * c->off.size(),
-                           hipMemcpyHostToDevice, stream) == hipSuccess &&
-            hipMemcpyAsync(c->d_vex, c->vex.data(), sizeof(double) * c->vex.size(),
-                           hipMemcpyHostToDevice, stream) == hipSuccess;
+  // the offset table and V_ex, which follow each other in the block
+  memcpy(tables, c->off.data(), sizeof(int32_t) * c->off.size());
+  memcpy(tables + ((char *)c->d_vex - (char *)c->d_off), c->vex.data(), sizeof(double) * c->vex.size());
+  const bool ok = hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess &&
+                  hipMemcpyAsync(c->d_off, tables, ctx_tables_bytes(g), hipMemcpyHostToDevice, stream) == hipSuccess;
   if (!ok) {
     bwl_destroy(c);
     return fail(BWL_ERR_DEVICE, "borrowed context set-up failed");
@@ -819,8 +825,6 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
     a.asro_every = p->asro_every;
     a.rho_of_T = nullptr;
     it.T = (size_t)p->T_steps;
-    it.off_muls = total;
-    total += 256 * ((it.plan.muls.size() * 4 + 255) / 256);
     it.off_out = total;
     total += 256 * ((5 * it.T * sizeof(double) + 255) / 256);
     it.off_cnt = total;
@@ -835,11 +839,16 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
   int n_cu = 0;
   if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctxs[0]->device) != hipSuccess) n_cu = 0;
   if (split) divide_chains(P, *split, n_cu, lim);
+  // The scratch: the chains' results (copied down in one piece), what goes up
+  // (counters among the results, then multipliers, arguments and maps, copied
+  // in one piece), and the divided chains' mailboxes (cleared in one piece).
+  P.out_bytes = total;
+  for (AnnealPlan::Item &it : P.items) {
+    it.off_muls = total;
+    total += 256 * ((it.plan.muls.size() * 4 + 255) / 256);
+  }
   int blocks = 0;
   for (AnnealPlan::Item &it : P.items) {
-    it.mail_n = it.a.parts > 1 ? par_split_mail_words(it.a.g, it.threads, it.a.parts) : 0;
-    it.off_mail = total;
-    total += 256 * ((it.mail_n * sizeof(unsigned long long) + 255) / 256);
     if (it.a.parts > 1) {
       it.fn = it.split_fn;
       it.lds = par_split_lds_bytes(it.a.g, it.a.nat);
@@ -902,13 +911,23 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
       total += 256 * ((sizeof(int2) * gr.map.size() + 255) / 256);
     }
   }
+  P.up_bytes = total;
+  for (AnnealPlan::Item &it : P.items) {
+    it.mail_n = it.a.parts > 1 ? par_split_mail_words(it.a.g, it.threads, it.a.parts) : 0;
+    it.off_mail = total;
+    total += 256 * ((it.mail_n * sizeof(unsigned long long) + 255) / 256);
+  }
   P.scratch_bytes = total;
   return BWL_OK;
 }
 
-int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, bool zero_by_kernel) {
+int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, char *image) {
   P.base = base;
-  P.host_args.clear();
+  if (!image) {
+    P.image.resize(P.up_bytes);
+    image = P.image.data();
+  }
+  memset(image, 0, P.up_bytes);  // the counters start at 0
   for (AnnealPlan::Item &it : P.items) {
     it.a.muls = (const uint32_t *)(base + it.off_muls);
     it.a.energies_of_T = (double *)(base + it.off_out);
@@ -917,24 +936,19 @@ int anneal_upload(AnnealPlan &P, char *base, hipStream_t s, bool zero_by_kernel)
     it.a.e_drift = it.a.acc_of_T + it.T;
     it.a.counters = (long long *)(base + it.off_cnt);
     it.a.rho_of_T = it.rho_n ? (double *)(base + it.off_rho) : nullptr;
-    HIP_OK(hipMemcpyAsync(base + it.off_muls, it.plan.muls.data(), it.plan.muls.size() * 4,
-                          hipMemcpyHostToDevice, s));
     it.a.mail = it.mail_n ? (unsigned long long *)(base + it.off_mail) : nullptr;
-    if (zero_by_kernel)
-      HIP_OK(launch_zero_i64(it.a.counters, 4, s));
-    else
-      HIP_OK(hipMemsetAsync(it.a.counters, 0, 4 * sizeof(long long), s));
-    if (it.mail_n) HIP_OK(hipMemsetAsync(it.a.mail, 0, it.mail_n * sizeof(unsigned long long), s));
+    memcpy(image + it.off_muls, it.plan.muls.data(), it.plan.muls.size() * 4);
   }
   for (AnnealPlan::Group &gr : P.groups) {
-    std::vector<ParArgs> host;
-    for (int i : gr.members) host.push_back(P.items[(size_t)i].a);
-    P.host_args.push_back(std::move(host));
-    HIP_OK(hipMemcpyAsync(base + gr.off_args, P.host_args.back().data(),
-                          sizeof(ParArgs) * P.host_args.back().size(), hipMemcpyHostToDevice, s));
-    if (gr.split)
-      HIP_OK(hipMemcpyAsync(base + gr.off_map, gr.map.data(), sizeof(int2) * gr.map.size(), hipMemcpyHostToDevice, s));
+    char *to = image + gr.off_args;
+    for (int i : gr.members) {
+      memcpy(to, &P.items[(size_t)i].a, sizeof(ParArgs));
+      to += sizeof(ParArgs);
+    }
+    if (gr.split) memcpy(image + gr.off_map, gr.map.data(), sizeof(int2) * gr.map.size());
   }
+  HIP_OK(hipMemcpyAsync(base, image, P.up_bytes, hipMemcpyHostToDevice, s));
+  if (P.scratch_bytes > P.up_bytes) HIP_OK(hipMemsetAsync(base + P.up_bytes, 0, P.scratch_bytes - P.up_bytes, s));
   return BWL_OK;
 }
 
@@ -954,21 +968,23 @@ int anneal_launch(const AnnealPlan &P, const hipStream_t *streams) {
 
 int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *energies_of_T,
                    double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats,
-                   double kernel_ms, hipStream_t s, double *const *rho_of_T, std::vector<int> *again) {
+                   double kernel_ms, hipStream_t s, double *const *rho_of_T, std::vector<int> *again,
+                   char *host) {
   const size_t n = P.items.size();
-  std::vector<std::vector<double>> out(n);
+  std::vector<char> own;
+  if (!host) {
+    own.resize(P.out_bytes);
+    host = own.data();
+  }
+  HIP_OK(hipMemcpyAsync(host, P.base, P.out_bytes, hipMemcpyDeviceToHost, s));
+  HIP_OK(hipStreamSynchronize(s));
+  std::vector<const double *> out(n);
   std::vector<long long> cnt(4 * n);
   for (size_t i = 0; i < n; ++i) {
     const AnnealPlan::Item &it = P.items[i];
-    out[i].resize(5 * it.T);
-    HIP_OK(hipMemcpyAsync(out[i].data(), it.a.energies_of_T, 5 * it.T * sizeof(double),
-                          hipMemcpyDeviceToHost, s));
-    HIP_OK(hipMemcpyAsync(&cnt[4 * i], it.a.counters, 4 * sizeof(long long), hipMemcpyDeviceToHost, s));
-    if (rho_of_T && rho_of_T[i] && it.rho_n)
-      HIP_OK(hipMemcpyAsync(rho_of_T[i], it.a.rho_of_T, it.rho_n * sizeof(double),
-                            hipMemcpyDeviceToHost, s));
+    out[i] = (const double *)(host + it.off_out);
+    memcpy(&cnt[4 * i], host + it.off_cnt, 4 * sizeof(long long));
   }
-  HIP_OK(hipStreamSynchronize(s));
   for (size_t i = 0; i < n; ++i) {
     const size_t T = P.items[i].T;
     if (P.items[i].a.parts > 1 && cnt[4 * i + 3] == 0) {
@@ -978,10 +994,11 @@ int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *ene
       again->push_back((int)i);
       continue;
     }
-    if (energies_of_T && energies_of_T[i]) memcpy(energies_of_T[i], out[i].data(), T * sizeof(double));
-    if (C_of_T && C_of_T[i]) memcpy(C_of_T[i], out[i].data() + T, T * sizeof(double));
-    if (acceptance_of_T && acceptance_of_T[i])
-      memcpy(acceptance_of_T[i], out[i].data() + 2 * T, T * sizeof(double));
+    if (energies_of_T && energies_of_T[i]) memcpy(energies_of_T[i], out[i], T * sizeof(double));
+    if (C_of_T && C_of_T[i]) memcpy(C_of_T[i], out[i] + T, T * sizeof(double));
+    if (acceptance_of_T && acceptance_of_T[i]) memcpy(acceptance_of_T[i], out[i] + 2 * T, T * sizeof(double));
+    if (rho_of_T && rho_of_T[i] && P.items[i].rho_n)
+      memcpy(rho_of_T[i], host + P.items[i].off_rho, P.items[i].rho_n * sizeof(double));
     if (stats) {
       stats[i].trials = cnt[4 * i + 2];
       stats[i].accepted = cnt[4 * i + 1];
@@ -1069,22 +1086,19 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   if (rc) return rc;
   share.keep(P.split);
   bwl_ctx *c0 = ctxs[0];
-  DevBuf scratch;
-  if (hipMalloc(&scratch.p, P.scratch_bytes) != hipSuccess)
-    return fail(BWL_ERR_NOMEM, "device allocation failed");
-  // every group on its own stream so groups overlap on the device
-  std::vector<hipStream_t> streams;
-  struct StreamFreer {
-    std::vector<hipStream_t> *v;
-    ~StreamFreer() {
-      for (size_t k = 1; k < v->size(); ++k) (void)hipStreamDestroy((*v)[k]);
-    }
-  } sfree{&streams};
-  streams.push_back(c0->stream);
+  rc = ensure_scratch(c0, P.scratch_bytes);
+  if (rc) return rc;
+  char *const scratch = (char *)c0->d_scratch;
+  // every group on its own stream so groups overlap on the device; the
+  // context keeps the streams (as many as a batch has kernel variants)
+  std::vector<hipStream_t> streams(1, c0->stream);
   for (size_t k = 1; k < P.groups.size(); ++k) {
-    hipStream_t s = nullptr;
-    HIP_OK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    streams.push_back(s);
+    if (c0->side.size() < k) {
+      hipStream_t s = nullptr;
+      HIP_OK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+      c0->side.push_back(s);
+    }
+    streams.push_back(c0->side[k - 1]);
   }
   hipEvent_t ready = nullptr;
   HIP_OK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
@@ -1092,8 +1106,11 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
     hipEvent_t e;
     ~EventFreer() { (void)hipEventDestroy(e); }
   } efree{ready};
+  Pinned pin;
+  const bool pinned = P.up_bytes <= kPinnedSeries;
+  if (pinned && !pin.take(P.up_bytes, c0->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
-  rc = anneal_upload(P, (char *)scratch.p, c0->stream);
+  rc = anneal_upload(P, scratch, c0->stream, pin.p);
   if (rc) return rc;
   HIP_OK(hipEventRecord(ready, c0->stream));
   for (size_t k = 1; k < streams.size(); ++k) HIP_OK(hipStreamWaitEvent(streams[k], ready, 0));
@@ -1112,7 +1129,8 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   (void)hipEventElapsedTime(&ms, c0->ev0, c0->ev1);
   if (makespan_ms) *makespan_ms = ms;
   std::vector<int> again;
-  rc = anneal_collect(P, ctxs, energies_of_T, C_of_T, acceptance_of_T, stats, ms, c0->stream, rho_of_T, &again);
+  rc = anneal_collect(P, ctxs, energies_of_T, C_of_T, acceptance_of_T, stats, ms, c0->stream, rho_of_T, &again, pin.p);
+  pin.settled();
   if (rc || again.empty()) return rc;
   // chains whose division was given up run undivided, with the same results
   std::vector<bwl_ctx *> cs;

@@ -47,6 +47,7 @@ struct bwl_ctx {
   bwl::MT19937 mt;
   unsigned long long phase = 0;  // parallel-sampler round counter
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  std::vector<hipStream_t> side;  // further streams of the context's batches
   bool held = false;      // counted by pinned_hold
   bool borrowed = false;  // device memory and stream belong to someone else
   int32_t layout = 0;     // parallel-sampler layout: 0 by rule, else BWL_LAYOUT_*
@@ -91,8 +92,11 @@ inline int lds_limit() {
 // ctx_device_bytes) and whose uploads go on `stream`; bwl_destroy frees
 // neither.
 size_t ctx_device_bytes(const bwl_lattice_desc &d);
+// tables: ctx_tables_bytes of (pinned) memory for the upload, kept until it
+// has ended
+size_t ctx_tables_bytes(const Geo &g);
 int ctx_create_borrowed(const bwl_lattice_desc &d, const double *v_ex, char *mem, size_t bytes,
-                        hipStream_t stream, bwl_ctx **out);
+                        hipStream_t stream, char *tables, bwl_ctx **out);
 
 // Workgroups of divided chains on each XCD of a device.
 struct SplitLanes {
@@ -131,8 +135,8 @@ struct AnnealPlan {
   };
   std::vector<Item> items;
   std::vector<Group> groups;
-  std::vector<std::vector<ParArgs>> host_args;  // kept alive until the uploads finish
-  size_t scratch_bytes = 0;
+  std::vector<char> image;  // what goes up, kept alive until the upload has ended
+  size_t out_bytes = 0, up_bytes = 0, scratch_bytes = 0;
   char *base = nullptr;
   SplitLanes split;  // workgroups of its divided chains
 };
@@ -147,13 +151,14 @@ int anneal_kernel(const Geo &g, ParPlan &plan, NatGeo &nat, const void *&fn, int
 // divided); AnnealPlan::split says how many the divided chains take.
 int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P,
                 const SplitLanes *split = nullptr);
-// zero_by_kernel: clear the counters with a kernel instead of a memset
-int anneal_upload(AnnealPlan &P, char *scratch_dev, hipStream_t s, bool zero_by_kernel = false);
+// image: up_bytes of (pinned) memory for what goes up, else the plan's own.
+// No memset unless chains are divided.
+int anneal_upload(AnnealPlan &P, char *scratch_dev, hipStream_t s, char *image = nullptr);
 int anneal_launch(const AnnealPlan &P, const hipStream_t *streams);
 int anneal_collect(const AnnealPlan &P, bwl_ctx *const *ctxs, double *const *energies_of_T,
                    double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats,
                    double kernel_ms, hipStream_t s, double *const *rho_of_T = nullptr,
-                   std::vector<int> *again = nullptr);
+                   std::vector<int> *again = nullptr, char *host = nullptr);
 // The whole call: plan (dividing chains over idle CUs), upload, launch, wait,
 // collect.
 int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, double *const *energies_of_T,

@@ -243,9 +243,6 @@ size_t seq_lds_bytes(const Geo &g);
 size_t seq_spec_lds_bytes(const Geo &g);
 hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s);
 hipError_t launch_draw_sites(const DrawArgs &a, hipStream_t s);
-// Sets n 64-bit words to zero with a kernel (no memset node in a captured
-// graph).
-hipError_t launch_zero_i64(long long *p, int n, hipStream_t s);
 // n chains (args_dev[0..n)), one workgroup each
 hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, const SeqPick &pick, hipStream_t s);
 size_t par_lds_bytes(const Geo &g, const NatGeo *nat, int threads);

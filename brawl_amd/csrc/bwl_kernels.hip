@@ -429,15 +429,6 @@ hipError_t launch_draw_sites(const DrawArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-__global__ __launch_bounds__(64) void k_zero_i64(long long *p, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-
-hipError_t launch_zero_i64(long long *p, int n, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(64), 0, s, p, n);
-  return hipGetLastError();
-}
-
 // ------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------

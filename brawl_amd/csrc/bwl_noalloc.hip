@@ -63,7 +63,7 @@ int bwl_metropolis_anneal_noalloc(bwl_ctx *c, const bwl_anneal_params *p, double
   rc = scratch_ptr(c->device, &base);
   if (rc) return rc;
   HIP_OK(hipEventRecord(c->ev0, c->stream));
-  rc = anneal_upload(P, base, c->stream, true);  // counters cleared by a kernel
+  rc = anneal_upload(P, base, c->stream);  // (an undivided chain: no memset)
   if (rc) return rc;
   rc = anneal_launch(P, &c->stream);
   if (rc) return rc;

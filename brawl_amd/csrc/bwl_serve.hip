@@ -122,6 +122,7 @@ struct Request {
   size_t block_bytes = 0;
   char *block = nullptr;
   bwl_ctx *ctx = nullptr;
+  std::unique_ptr<Pinned> up;  // tables and configuration as uploaded
   // accounting
   double t_submit = 0, t_admit = 0, t_done = 0, kernel_ms = 0;
   int64_t trials = 0, accepted = 0;
@@ -188,6 +189,7 @@ int free_slot(bwl_server *s) {
 }
 
 void release_request(bwl_server *s, Request *r) {
+  r->up.reset();
   if (r->ctx) {
     bwl_destroy(r->ctx);
     r->ctx = nullptr;
@@ -214,18 +216,39 @@ int retire(bwl_server *s, Launch &L) {
       C[i] = L.reqs[i]->Cv;
       A[i] = L.reqs[i]->acc;
     }
-    status = anneal_collect(*L.plan, ctxs.data(), E.data(), C.data(), A.data(), stats.data(), ms, st);
-    for (size_t i = 0; i < n; ++i) {
-      Request *r = L.reqs[i];
-      r->trials = stats[i].trials;
-      r->accepted = stats[i].accepted;
-      if (status == BWL_OK && r->config_out) {
-        const Geo &g = r->g;
-        const size_t ref = (size_t)g.m[0] * g.m[1] * g.m[2];
-        if (launch_unpack(r->ctx->d_compact, r->ctx->d_ref, g, st) != hipSuccess ||
-            hipMemcpyAsync(r->config_out, r->ctx->d_ref, ref, hipMemcpyDeviceToHost, st) != hipSuccess)
-          status = fail(BWL_ERR_DEVICE, "result download failed");
+    // final configurations first, by way of pinned memory (in turn, as many
+    // at a time as that takes), so that they travel beside the results
+    auto grid = [](const Request *r) { return (size_t)r->g.m[0] * r->g.m[1] * r->g.m[2]; };
+    for (size_t i = 0; i < n && status == BWL_OK;) {
+      size_t bytes = 0, end = i;
+      while (end < n && (end == i || bytes + grid(L.reqs[end]) <= kPinnedConfig)) {
+        if (L.reqs[end]->config_out) bytes += grid(L.reqs[end]);
+        ++end;
       }
+      Pinned pin;
+      if (bytes > 0 && !pin.take(bytes, st)) status = fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+      size_t at = 0;
+      for (size_t k = i; k < end && bytes > 0 && status == BWL_OK; ++k) {
+        if (!L.reqs[k]->config_out) continue;
+        if (launch_unpack(L.reqs[k]->ctx->d_compact, (int8_t *)pin.p + at, L.reqs[k]->g, st) != hipSuccess)
+          status = fail(BWL_ERR_DEVICE, "result download failed");
+        at += grid(L.reqs[k]);
+      }
+      if (end == n && status == BWL_OK)
+        status = anneal_collect(*L.plan, ctxs.data(), E.data(), C.data(), A.data(), stats.data(), ms, st);
+      else if (bytes > 0 && hipStreamSynchronize(st) != hipSuccess && status == BWL_OK)
+        status = fail(BWL_ERR_DEVICE, "result download failed");
+      at = 0;
+      for (size_t k = i; k < end && bytes > 0 && status == BWL_OK; ++k) {
+        if (!L.reqs[k]->config_out) continue;
+        memcpy(L.reqs[k]->config_out, pin.p + at, grid(L.reqs[k]));
+        at += grid(L.reqs[k]);
+      }
+      i = end;
+    }
+    for (size_t i = 0; i < n; ++i) {
+      L.reqs[i]->trials = stats[i].trials;
+      L.reqs[i]->accepted = stats[i].accepted;
     }
   } else if (L.kind == KIND_WL) {
     for (size_t i = 0; i < L.reqs.size(); ++i) {
@@ -280,6 +303,7 @@ int retire(bwl_server *s, Launch &L) {
     r->kernel_ms = ms;
     r->t_done = t;
     if (status != BWL_OK && r->error == BWL_OK) r->error = status;
+    if (r->up) r->up->settled();
     r->state = r->error == BWL_OK ? ST_DONE : ST_FAILED;
     release_request(s, r);
     s->done_unpolled.push_back(r->id);
@@ -294,15 +318,22 @@ int retire(bwl_server *s, Launch &L) {
 // Device set-up of an admitted request on stream `st` (its block is
 // allocated): borrowed context, configuration or walkers.
 int stage_request(Request *r, hipStream_t st) {
-  const size_t cb = ctx_device_bytes(r->desc);
-  int rc = ctx_create_borrowed(r->desc, r->vex.data(), r->block, cb, st, &r->ctx);
+  const size_t cb = ctx_device_bytes(r->desc), tables = al(ctx_tables_bytes(r->g));
+  const size_t ref = (size_t)r->g.m[0] * r->g.m[1] * r->g.m[2];
+  const bool anneal = r->kind == KIND_ANNEAL, pinned = anneal && ref <= kPinnedConfig;
+  r->up = std::make_unique<Pinned>();
+  if (!r->up->take(tables + (pinned ? ref : 0), st)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+  int rc = ctx_create_borrowed(r->desc, r->vex.data(), r->block, cb, st, r->up->p, &r->ctx);
   if (rc) return rc;
-  if (r->kind == KIND_ANNEAL) {
-    rc = check_config(r->g, r->config.data(), g_err);
-    if (rc) return rc;
-    const size_t ref = (size_t)r->g.m[0] * r->g.m[1] * r->g.m[2];
-    HIP_OK(hipMemcpyAsync(r->ctx->d_ref, r->config.data(), ref, hipMemcpyHostToDevice, st));
-    HIP_OK(launch_pack(r->ctx->d_ref, r->ctx->d_compact, r->g, st));
+  if (anneal) {  // (its configuration was checked when it was submitted)
+    const int8_t *from = r->ctx->d_ref;
+    if (pinned) {
+      memcpy(r->up->p + tables, r->config.data(), ref);
+      from = (const int8_t *)r->up->p + tables;
+    } else {
+      HIP_OK(hipMemcpyAsync(r->ctx->d_ref, r->config.data(), ref, hipMemcpyHostToDevice, st));
+    }
+    HIP_OK(launch_pack(from, r->ctx->d_compact, r->g, st));
     r->ctx->has_config = true;
   }
   return BWL_OK;
@@ -677,8 +708,11 @@ int bwl_server_destroy(bwl_server *s) {
     (void)hipEventDestroy(L->ev0);
     (void)hipEventDestroy(L->ev1);
   }
-  for (auto &kv : s->reqs)
+  for (auto &kv : s->reqs) {
     if (kv.second->ctx) bwl_destroy(kv.second->ctx);
+    if (kv.second->up) kv.second->up->settled();
+    kv.second->up.reset();
+  }
   for (hipStream_t st : s->streams) (void)hipStreamDestroy(st);
   if (s->arena_mem) (void)hipFree(s->arena_mem);
   if (s->held) pinned_drop();
