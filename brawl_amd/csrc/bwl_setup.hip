@@ -11,12 +11,15 @@
 // both sides) goes to the first of them with atoms left; such a draw is
 // settled alone.
 //
-// One workgroup follows one stream: wavefront 0 places the walkers one after
-// another (where a walker starts in the stream depends on the one before it),
-// wavefront 1 makes the stream's next 624 draws meanwhile.  Wavefront 0's
-// instructions bound it.  128 walkers of 864 sites, 5 species: 1.8 ms on the
-// host, 1.6 ms here, but the streams of a batch run side by side: 32 such runs
-// 64 ms on the host, 1.6 ms here.
+// One workgroup follows one stream in a pipeline of blocks of 624 draws:
+// wavefront 1 makes a block's draws, wavefronts 2 and 3 then the species that
+// each names and, per 64 draws, the mask of those that name a species, and
+// wavefront 0 places the walkers one after another from those (where a walker
+// starts in the stream depends on the one before it); the four meet at one
+// barrier a block.  The chain of wavefront 0's steps bounds it.  128 walkers
+// of 864 sites, 5 species: 1.8 ms on the host, 1.6 ms with the masks formed in
+// the chain, 0.76 ms so; the streams of a batch run side by side (32 of them: 64 ms
+// on the host).
 #include <hip/hip_runtime.h>
 
 #include "bwl_kernels.h"
@@ -27,160 +30,138 @@ namespace bwl {
 namespace {
 
 constexpr long long kSetupDraws = 1LL << 26;  // a walker's; its mean is at most 10^4 a species beyond the sites
-constexpr int kAtOnce = 4;                    // groups of 64 draws
+constexpr int kSetupThreads = 256;
+constexpr int kGroups = 10;        // of 64 draws in a block, the last of 48
+constexpr int kAny = kMaxSpecies;  // masks of a group: per species, of all that name one,
+constexpr int kTwice = kAny + 1;   // of those that name two
+constexpr int kMasks = kTwice + 1;
 
-__global__ __launch_bounds__(128) void k_setup(const SetupArgs *__restrict__ args) {
+__device__ __forceinline__ unsigned long long lane_mask(unsigned long long v, int l) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l);
+  return ((unsigned long long)hi << 32) | lo;
+}
+
+__global__ __launch_bounds__(kSetupThreads) void k_setup(const SetupArgs *__restrict__ args) {
   __shared__ uint32_t raw[624];
-  __shared__ uint32_t tem[kRingWords];
-  __shared__ volatile int32_t last;  // the barrier after which wavefront 1 leaves, counted from 1
+  __shared__ uint32_t tem[3][624];
+  __shared__ uint8_t code[2][64 * kGroups];
+  __shared__ unsigned long long masks[2][kGroups][kMasks];
+  __shared__ volatile int32_t last;  // the barrier after which the helpers leave, counted from 1
   const SetupArgs &A = args[blockIdx.x];
   if (A.made || A.n_walkers < 1) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = wave_uniform(tid >> 6);
+  const int S = A.g.S;
   if (tid == 0) last = 0;
-  for (int i = tid; i < 624; i += 128) {
+  for (int i = tid; i < 624; i += kSetupThreads) {
     const uint32_t v = A.mt[i];
     raw[i] = v;
-    tem[i] = mt_temper(v);
+    tem[0][i] = mt_temper(v);
   }
   __syncthreads();
-  int half = 0, turn = 0;
+  // block b's draws lie in tem[b mod 3], what they name in slot b mod 2
+  auto classify = [&](int b) {
+    const uint32_t *t = tem[b % 3];
+    for (int j = wave - 2; j < kGroups; j += 2) {
+      const bool there = 64 * j + lane < 624;
+      const uint32_t k = t[there ? 64 * j + lane : 623];
+      unsigned long long any = 0, twice = 0, mine = 0;
+      int names = 0;
+      for (int s = 0; s < S; ++s) {
+        const bool in = there && k >= A.rule.lo[s] && k <= A.rule.hi[s];
+        const unsigned long long m = __ballot(in);
+        twice |= any & m;
+        any |= m;
+        if (in) names = s + 1;
+        if (lane == s) mine = m;
+      }
+      if (lane == kAny) mine = any;
+      if (lane == kTwice) mine = twice;
+      code[b & 1][64 * j + lane] = (uint8_t)names;
+      if (lane < kMasks) masks[b & 1][j][lane] = mine;
+    }
+  };
+  auto twist = [&](int b) { ring_twist(raw, tem[b % 3] - 624, 0); };  // (to tem[b mod 3])
+  if (wave == 1) twist(1);
+  if (wave >= 2) classify(0);
+  __syncthreads();
+  int turn = 0;  // barriers since, and the block that wavefront 0 uses
   if (wave != 0) {
     for (;;) {
-      ring_twist(raw, tem, half);
+      if (wave == 1)
+        twist(turn + 2);
+      else
+        classify(turn + 1);
       __syncthreads();
       if (last == ++turn) return;
-      half = 624 - half;
     }
   }
   int pos = wave_uniform(A.mt_index[0]);
-  const int n_atoms = A.g.n_atoms, S = A.g.S, n_walkers = A.n_walkers;
+  const int n_atoms = A.g.n_atoms, n_walkers = A.n_walkers;
+  // lane s keeps species s
+  const uint32_t lo = lane < S ? A.rule.lo[lane] : 1u, hi = lane < S ? A.rule.hi[lane] : 0u;
+  const int count = lane < S ? A.rule.count[lane] : 0;
+  int8_t *const orders = A.order;
+  double *const rnde = A.rnde;
   int status = 0;
   auto refill = [&]() {
     if (pos < 624) return;
     __syncthreads();
     ++turn;
-    half = 624 - half;
     pos = 0;
   };
-  uint32_t lo[kMaxSpecies], hi[kMaxSpecies];
-  int count[kMaxSpecies];
-#pragma unroll
-  for (int s = 0; s < kMaxSpecies; ++s) {
-    lo[s] = (uint32_t)wave_uniform((int)A.rule.lo[s]);
-    hi[s] = (uint32_t)wave_uniform((int)A.rule.hi[s]);
-    count[s] = wave_uniform(A.rule.count[s]);
-  }
-  int8_t *const orders = A.order;
-  double *const rnde = A.rnde;
   for (int w = 0; w < n_walkers; ++w) {
     int8_t *out = orders + (size_t)w * n_atoms;
-    int room[kMaxSpecies];
-#pragma unroll
-    for (int s = 0; s < kMaxSpecies; ++s) room[s] = s < S ? count[s] : 0;
-    int filled = 0;
+    int room = count, filled = 0;
     long long draws = 0;
     while (filled < n_atoms) {
       refill();
-      // up to 256 draws at once while no species runs out among them
-      {
-        const int ahead = 624 - pos;
-        uint32_t k[kAtOnce];
-        unsigned long long any[kAtOnce], twice = 0;
-        int mine[kAtOnce], left[kMaxSpecies];
-        bool fits = true;
-#pragma unroll
-        for (int j = 0; j < kAtOnce; ++j) {
-          k[j] = tem[half + min(pos + 64 * j + lane, 623)];
-          any[j] = 0;
-          mine[j] = 0;
-        }
-#pragma unroll
-        for (int s = 0; s < kMaxSpecies; ++s) {
-          left[s] = room[s];
-          if (s < S) {
-#pragma unroll
-            for (int j = 0; j < kAtOnce; ++j) {
-              const bool in = k[j] - lo[s] <= hi[s] - lo[s] && lo[s] <= hi[s] && 64 * j + lane < ahead;
-              const unsigned long long b = __ballot(in);
-              twice |= any[j] & b;
-              any[j] |= b;
-              left[s] -= __popcll(b);
-              if (in) mine[j] = s + 1;
-            }
-            fits = fits && left[s] >= 0;
-          }
-        }
-        if (fits && !twice) {
-#pragma unroll
-          for (int j = 0; j < kAtOnce; ++j) {
-            if (mine[j])
-              out[filled + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(any[j] >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)any[j], 0))] = (int8_t)mine[j];
-            filled += __popcll(any[j]);
-          }
-#pragma unroll
-          for (int s = 0; s < kMaxSpecies; ++s) room[s] = left[s];
-          // (the last site's draw is the last one taken)
-          int used = min(64 * kAtOnce, ahead);
-          if (filled == n_atoms) {
-            used = 0;
-#pragma unroll
-            for (int j = 0; j < kAtOnce; ++j)
-              if (any[j]) used = 64 * j + 64 - __clzll((long long)any[j]);
-          }
-          pos += used;
-          draws += used;
-          continue;
-        }
-      }
-      int n = min(64, 624 - pos);
-      const uint32_t k = tem[half + pos + min(lane, n - 1)];
-      const unsigned long long inside = n < 64 ? (1ull << n) - 1ull : ~0ull;
-      unsigned long long named[kMaxSpecies], any = 0, twice = 0;
-#pragma unroll
-      for (int s = 0; s < kMaxSpecies; ++s) {
-        named[s] = s < S ? __ballot(k >= lo[s] && k <= hi[s]) & inside : 0ull;
-        twice |= any & named[s];
-        any |= named[s];
-      }
+      const int j = pos >> 6, off = pos & 63;
+      const unsigned long long *M = masks[turn & 1][j];
+      const unsigned long long m = M[lane < kMasks ? lane : 0];
+      const int names = code[turn & 1][64 * j + lane];
+      unsigned long long window = ~0ull << off;
+      int end = min(64, 624 - 64 * j);
+      const unsigned long long twice = lane_mask(m, kTwice) & window;
       if (twice) {
         const int at = __ffsll((long long)twice) - 1;
-        n = at > 0 ? at : 1;
-        const unsigned long long keep = (1ull << n) - 1ull;
-        bool open = true;
-#pragma unroll
-        for (int s = 0; s < kMaxSpecies; ++s) {
-          named[s] &= keep;
-          if (at == 0) {
-            if (!open || room[s] == 0) named[s] = 0;
-            if (named[s]) open = false;
+        if (at == off) {
+          const uint32_t k = tem[turn % 3][pos];
+          const unsigned long long b = __ballot(k >= lo && k <= hi && room > 0);
+          if (b) {
+            const int s = __ffsll((long long)b) - 1;
+            if (lane == s) {
+              --room;
+              out[filled] = (int8_t)(s + 1);
+            }
+            ++filled;
           }
+          ++pos;
+          ++draws;
+          continue;
         }
+        window &= (1ull << at) - 1ull;
+        end = at;
       }
-      unsigned long long taken = 0;
-      int mine = 0;
-#pragma unroll
-      for (int s = 0; s < kMaxSpecies; ++s) {
-        int c = __popcll(named[s]);
-        if (c > room[s]) {
-          const bool first = ((named[s] >> lane) & 1) != 0 &&
-                             (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(named[s] >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)named[s], 0)) < room[s];
-          named[s] = __ballot(first);
-          c = room[s];
-        }
-        room[s] -= c;
-        taken |= named[s];
-        if ((named[s] >> lane) & 1) mine = s + 1;
+      const int c = lane < kMaxSpecies ? __popcll(m & window) : 0;
+      unsigned long long taken = lane_mask(m, kAny) & window;
+      if (__ballot(c > room && lane < kMaxSpecies)) {
+        // a species runs out: its first draws are taken
+        const unsigned long long own = M[names ? names - 1 : 0] & window;
+        const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(own >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)own, 0));
+        const int open = __shfl(room, names ? names - 1 : 0);
+        taken = __ballot(((taken >> lane) & 1) != 0 && before < open);
       }
-      if (mine)
+      room -= min(c, room);
+      if ((taken >> lane) & 1)
         out[filled + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(taken >> 32),
-                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)taken, 0))] = (int8_t)mine;
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)taken, 0))] = (int8_t)names;
       filled += __popcll(taken);
-      pos += filled == n_atoms ? 64 - __clzll((long long)taken) : n;
-      draws += n;
-      if (draws > kSetupDraws) {
+      draws += end - off;
+      // (the last site's draw is the last one taken)
+      pos = 64 * j + (filled == n_atoms ? 64 - __clzll((long long)taken) : end);
+      if (draws > kSetupDraws && filled < n_atoms) {
         // (every site gets a species: the kernels after this one read them all)
         for (int i = filled + lane; i < n_atoms; i += 64) out[i] = 1;
         filled = n_atoms;
@@ -189,13 +170,12 @@ __global__ __launch_bounds__(128) void k_setup(const SetupArgs *__restrict__ arg
     }
     if (rnde) {
       refill();
-      if (lane == 0) rnde[w] = (double)tem[half + pos] * (1.0 / 4294967296.0);
+      if (lane == 0) rnde[w] = (double)tem[turn % 3][pos] * (1.0 / 4294967296.0);
       ++pos;
     }
   }
-  // the state is the block in use; it lies in the other half of the draws
-  // than the one wavefront 1 is making
-  for (int i = lane; i < 624; i += 64) A.mt[i] = mt_untemper(tem[half + i]);
+  // the state is that of the block in use
+  for (int i = lane; i < 624; i += 64) A.mt[i] = mt_untemper(tem[turn % 3][i]);
   if (lane == 0) {
     A.mt_index[0] = pos;
     *A.status = status;
@@ -236,7 +216,7 @@ __global__ void k_order_to_compact(const SetupArgs *__restrict__ args, int max_w
 hipError_t launch_setup(const SetupArgs *args_dev, int n, int max_walkers, int max_atoms, bool any_drawn, hipStream_t s) {
   for (int first = 0; first < n; first += 65535) {
     const int m = n - first < 65535 ? n - first : 65535;
-    if (any_drawn) hipLaunchKernelGGL(k_setup, dim3(m), dim3(128), 0, s, args_dev + first);
+    if (any_drawn) hipLaunchKernelGGL(k_setup, dim3(m), dim3(kSetupThreads), 0, s, args_dev + first);
     const int blocks = (max_atoms + 1023) / 1024;
     hipLaunchKernelGGL(k_order_to_compact, dim3(blocks < 64 ? blocks : 64, max_walkers < 65535 ? max_walkers : 65535, m),
                        dim3(256), 0, s, args_dev + first, max_walkers);
