@@ -341,10 +341,28 @@ bool make_nat_fixed(const Geo &g, NatGeo &nat) {
   return nat_dims_fixed(g.lattice, g.R, g.n[0], nat);
 }
 
+namespace {
+
+// Whether a row of the doubled grid holds what it may: cells of x parity p
+// species 1..S, the others nothing (p < 0: all nothing).  Two cells a step by
+// the same arithmetic, which the compiler makes vectors of.
+bool row_ok(const int8_t *row, int len, int p, int S) {
+  const uint8_t base[2] = {(uint8_t)(p == 0), (uint8_t)(p == 1)};
+  const uint8_t top[2] = {(uint8_t)(p == 0 ? S - 1 : 0), (uint8_t)(p == 1 ? S - 1 : 0)};
+  uint8_t bad = 0;
+  for (int x = 0; x < len; x += 2)
+    for (int k = 0; k < 2; ++k) bad |= (uint8_t)((uint8_t)((uint8_t)row[x + k] - base[k]) > top[k]);
+  return bad == 0;
+}
+
+}  // namespace
+
 int check_config(const Geo &g, const int8_t *config, std::string &err) {
   const int m0 = g.m[0], m1 = g.m[1], m2 = g.m[2];
   for (int z = 0; z < m2; ++z)
-    for (int y = 0; y < m1; ++y)
+    for (int y = 0; y < m1; ++y) {
+      const int p = g.lattice == BWL_FCC ? (y + z) & 1 : (y & 1) == (z & 1) ? y & 1 : -1;
+      if (row_ok(config + (size_t)m0 * (y + (size_t)m1 * z), m0, p, g.S)) continue;
       for (int x = 0; x < m0; ++x) {
         int v = config[x + (size_t)m0 * (y + (size_t)m1 * z)];
         bool occ = g.lattice == BWL_FCC ? (((x + y + z) & 1) == 0)
@@ -355,6 +373,7 @@ int check_config(const Geo &g, const int8_t *config, std::string &err) {
           return BWL_ERR_ARG;
         }
       }
+    }
   return BWL_OK;
 }
 
@@ -362,22 +381,21 @@ int check_config(const Geo &g, const int8_t *config, std::string &err) {
 
 namespace bwl {
 
-void lattice_shells_host(const Geo &g, int wc, double *shells) {
-  // Distances are sqrt of integers, so the distinct values are those of the
-  // distinct squared distances; 0 is always present (site (1,1,1) is
-  // occupied, and the reference pads its sorted list with zeros).
-  const int m0 = g.m[0], m1 = g.m[1], m2 = g.m[2];
-  const long long dmax = (long long)(m0 - 1) * (m0 - 1) + (long long)(m1 - 1) * (m1 - 1) +
-                         (long long)(m2 - 1) * (m2 - 1);
-  std::vector<uint8_t> seen((size_t)dmax + 1, 0);
+// The shells among the distances up to `reach` on every axis (all of them
+// with 0 < reach2 = reach^2 or the box's end), from which sites are sure to be
+// complete; how many there are.
+static int shells_within(const Geo &g, int wc, int reach, double *shells) {
+  const int e[3] = {std::min(g.m[0] - 1, reach), std::min(g.m[1] - 1, reach), std::min(g.m[2] - 1, reach)};
+  const bool all = reach >= std::max(std::max(g.m[0], g.m[1]), g.m[2]) - 1;
+  const long long far = (long long)e[0] * e[0] + (long long)e[1] * e[1] + (long long)e[2] * e[2];
+  const long long dmax = all ? far : std::min(far, (long long)reach * reach);
+  std::vector<uint8_t> seen((size_t)far + 1, 0);
   seen[0] = 1;
-  for (int k = 0; k < m2; ++k)
-    for (int j = 0; j < m1; ++j)
-      for (int i = 0; i < m0; ++i) {
-        const bool occ = g.lattice == BWL_FCC ? (((i + j + k) & 1) == 0)
-                                              : ((i & 1) == (j & 1) && (j & 1) == (k & 1));
-        if (occ) seen[(size_t)(i * i + j * j + k * k)] = 1;
-      }
+  for (int k = 0; k <= e[2]; ++k)
+    for (int j = 0; j <= e[1]; ++j) {
+      if (g.lattice != BWL_FCC && (j & 1) != (k & 1)) continue;
+      for (int i = (g.lattice == BWL_FCC ? j + k : j) & 1; i <= e[0]; i += 2) seen[(size_t)(i * i + j * j + k * k)] = 1;
+    }
   std::vector<double> vals;
   for (long long d = 0; d <= dmax; ++d)
     if (seen[(size_t)d]) {
@@ -391,12 +409,34 @@ void lattice_shells_host(const Geo &g, int wc, double *shells) {
     if (fabs(vals[i] - vals[i + 1]) < 1e-3) continue;
     shells[cnt++] = vals[i];
   }
+  return all ? wc : cnt;
+}
+
+void lattice_shells_host(const Geo &g, int wc, double *shells) {
+  // Distances are sqrt of integers, so the distinct values are those of the
+  // distinct squared distances; 0 is always present (site (1,1,1) is
+  // occupied, and the reference pads its sorted list with zeros).  The shells
+  // are the nearest ones, so sites beyond a reach that holds them all are not
+  // looked at (bcc 32^3, 5 shells: 121 -> 1 us).
+  for (int reach = 8; shells_within(g, wc, reach, shells) < wc; reach *= 2) {
+  }
 }
 
 void asro_offsets_host(const Geo &g, int wc, const double *shells, std::vector<int32_t> &off3,
                        int32_t *shell_start) {
   const int w[3] = {std::min(g.n[0], 5), std::min(g.n[1], 5), std::min(g.n[2], 5)};
   std::vector<std::vector<int32_t>> per((size_t)wc);
+  // minimum image of the index difference, as the reference computes it from
+  // site (1,1,1): REAL(4) differences, NINT of the ratio; squared
+  double r2[3][11];
+  for (int a = 0; a < 3; ++a)
+    for (int d = -w[a]; d <= w[a]; ++d) {
+      const int m = g.m[a];
+      const int j = ((d % m) + m) % m + 1;
+      double v = (double)(float)(1 - j);
+      v = v - (double)(float)m * (double)lround(v / (double)(float)m);
+      r2[a][d + w[a]] = v * v;
+    }
   for (int dz = -w[2]; dz <= w[2]; ++dz)
     for (int dy = -w[1]; dy <= w[1]; ++dy)
       for (int dx = -w[0]; dx <= w[0]; ++dx) {
@@ -404,18 +444,7 @@ void asro_offsets_host(const Geo &g, int wc, const double *shells, std::vector<i
                              ? (((dx + dy + dz) & 1) == 0)
                              : (((dx ^ dy) & 1) == 0 && ((dy ^ dz) & 1) == 0);
         if (!lat) continue;
-        // minimum image of the index difference, as the reference computes
-        // it from site (1,1,1): REAL(4) differences, NINT of the ratio
-        const int d[3] = {dx, dy, dz};
-        double r[3];
-        for (int a = 0; a < 3; ++a) {
-          const int m = g.m[a];
-          const int j = ((d[a] % m) + m) % m + 1;
-          double v = (double)(float)(1 - j);
-          v = v - (double)(float)m * (double)lround(v / (double)(float)m);
-          r[a] = v;
-        }
-        const double dist = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+        const double dist = sqrt(r2[0][dx + w[0]] + r2[1][dy + w[1]] + r2[2][dz + w[2]]);
         for (int l = 0; l < wc; ++l)
           if (fabs(dist - shells[l]) < 1e-3) {
             per[(size_t)l].push_back(dx);
