@@ -118,6 +118,7 @@ struct AnnealPlan {
     size_t T = 0, off_muls = 0, off_out = 0, off_cnt = 0, off_rho = 0, rho_n = 0;
     size_t off_mail = 0, mail_n = 0;  // mailbox of a divided chain, in words
     const void *split_fn = nullptr;   // kernel that can divide the chain, if any
+    bool natural = false;             // held in lattice coordinates
     int chunks = 0, passes = 0;       // most pairs of a round, in 64s and per thread
     int lane = 0;                     // XCD of a divided chain's parts
     double rounds = 0.0;              // rounds of the whole anneal, about

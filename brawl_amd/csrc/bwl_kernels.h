@@ -267,6 +267,11 @@ const void *par_fixed_kernel(int lattice, int R, int words);
 // division suits the kernel's shape, and its launch (block b runs part
 // map[b].y of chain map[b].x, or nothing when that is negative).
 const void *par_split_kernel(const Geo &g, bool fixed);
+// The kernel of small chains at one site per lane (launch_metro_par_fn; LDS
+// par_split_lds_bytes), nullptr if there is none, and its block size for a
+// chain of `threads` threads with `passes` pairs each, 0 if it has too many.
+const void *par_alone_kernel(const Geo &g, bool fixed);
+int par_alone_threads(int threads, int passes);
 size_t par_split_lds_bytes(const Geo &g, const NatGeo &nat);
 size_t par_split_mail_words(const Geo &g, int threads, int parts);
 bool par_split_fits(const NatGeo &nat, int threads, int parts, int passes);
