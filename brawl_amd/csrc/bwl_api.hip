@@ -691,11 +691,14 @@ static double divided_us(const AnnealPlan::Item &it) { return it.rounds * 2.4; }
 // parts 7.4, 4 parts 7.7), else two.
 //
 // The parts of a chain go to one XCD (lane), which has n_cu / 8 CUs: as many
-// as other chains of this and other calls leave free.
+// as other chains of this and other calls leave free.  Parts and undivided
+// chains together have a CU each: a batch of 256 uneven chains, eight of them
+// fcc 24^3, took 184 ms with those eight divided (smaller chains then share
+// CUs with parts that all the others wait for) and 144 with none.
 static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu, int lim) {
   const int n = (int)P.items.size();
   const int cap = std::max(n_cu / 8 - (n + 7) / 8, n_cu / 16);
-  int lanes[8];
+  int lanes[8], blocks = n;
   bool any = false;
   for (int x = 0; x < 8; ++x) {
     lanes[x] = std::min(free_parts.parts[x], cap);
@@ -725,7 +728,8 @@ static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu,
       int to = 0;
       for (int x = 1; x < 8; ++x)
         if (lanes[x] > lanes[to]) to = x;
-      if (parts > lanes[to] || load_then > n_cu * undivided_us(it)) continue;
+      if (parts > lanes[to] || blocks + parts - 1 > n_cu || load_then > n_cu * undivided_us(it)) continue;
+      blocks += parts - 1;
       load = load_then;
       lanes[to] -= parts;
       it.a.parts = parts;
