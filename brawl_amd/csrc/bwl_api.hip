@@ -678,6 +678,12 @@ int anneal_kernel(const Geo &g, ParPlan &plan, NatGeo &nat, const void *&fn, int
 static double undivided_us(const AnnealPlan::Item &it) {
   return it.rounds * (0.7 + 0.135 * sqrt((double)it.chunks * (double)it.a.g.z));
 }
+double anneal_estimate_us(const Geo &g, const ParPlan &plan, const bwl_anneal_params &p) {
+  int pairs = 1;
+  for (const RoundVar &v : plan.vars) pairs = std::max(pairs, (int)v.n2);
+  const double rounds = (double)p.T_steps * ((double)p.n_sweeps + p.burn_in_sweeps) * g.n_atoms / pairs;
+  return rounds * (0.7 + 0.135 * sqrt((double)((pairs + 63) / 64) * (double)g.z));
+}
 static double divided_us(const AnnealPlan::Item &it) { return it.rounds * 2.4; }
 
 // Divides the longest chains over workgroups (a.parts, lane of their items)

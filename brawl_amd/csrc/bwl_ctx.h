@@ -148,6 +148,8 @@ struct AnnealPlan {
 // 0 then takes the first layout that can run them).
 int anneal_kernel(const Geo &g, ParPlan &plan, NatGeo &nat, const void *&fn, int &threads,
                   size_t &lds, bool *natural = nullptr, int layout = 0, int threads_req = 0);
+// About how long a chain takes in one workgroup, in us.
+double anneal_estimate_us(const Geo &g, const ParPlan &plan, const bwl_anneal_params &p);
 // split: the workgroups that chains may be divided into (none: no chain is
 // divided); AnnealPlan::split says how many the divided chains take.
 int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, AnnealPlan &P,

@@ -14,6 +14,7 @@
 // sampling and Wang-Landau walkers), so its result does not depend on what it
 // was batched with.
 #include <hip/hip_runtime.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -119,6 +120,7 @@ struct Request {
   std::vector<int32_t> wl_mti;    // a position per walker, then the set-ups' statuses
   double *lng_out = nullptr, *hist_out = nullptr;
   // device residency
+  double est_ms = 0;  // about how long its launch takes (place_groups)
   size_t block_bytes = 0;
   char *block = nullptr;
   bwl_ctx *ctx = nullptr;
@@ -131,6 +133,7 @@ struct Request {
 struct Launch {
   int kind = 0;
   int slot = -1;
+  double est_end = 0;  // about when it ends, on the server's clock
   std::vector<Request *> reqs;
   std::unique_ptr<AnnealPlan> plan;
   std::vector<NsArgs> ns_args;
@@ -154,6 +157,7 @@ struct bwl_server {
   void *arena_mem = nullptr;
   std::vector<hipStream_t> streams;
   std::vector<bool> slot_busy;
+  int hw_queues = 4;  // streams share them in turn
   std::deque<Request *> queue;
   std::vector<std::unique_ptr<Launch>> running;
   std::unordered_map<int64_t, std::unique_ptr<Request>> reqs;
@@ -182,10 +186,29 @@ size_t wl_block_bytes(const Request &r) {
          al(sizeof(double) * W * r.hstride) + al(8 * W);
 }
 
+// A free slot, of the hardware queue that is done soonest: launches on one
+// queue wait for each other, and the streams of the slots take the queues in
+// turn.
 int free_slot(bwl_server *s) {
-  for (size_t k = 0; k < s->slot_busy.size(); ++k)
-    if (!s->slot_busy[k]) return (int)k;
-  return -1;
+  int best = -1;
+  double soonest = 0.0;
+  for (size_t k = 0; k < s->slot_busy.size(); ++k) {
+    if (s->slot_busy[k]) continue;
+    double end = 0.0;
+    for (const auto &L : s->running)
+      if (L->slot % s->hw_queues == (int)k % s->hw_queues) end = std::max(end, L->est_end);
+    if (best < 0 || end < soonest) {
+      best = (int)k;
+      soonest = end;
+    }
+  }
+  return best;
+}
+
+double group_ms(const std::vector<Request *> &grp) {
+  double ms = 0.0;
+  for (const Request *r : grp) ms = std::max(ms, r->est_ms);
+  return ms;
 }
 
 void release_request(bwl_server *s, Request *r) {
@@ -603,6 +626,15 @@ int admit(bwl_server *s) {
       }
     if (!placed) groups.push_back({r});
   }
+  // of the groups that get a slot, the longest first: the short ones then
+  // share a hardware queue with each other, not with the longest
+  {
+    const size_t slots = (size_t)std::count(s->slot_busy.begin(), s->slot_busy.end(), false);
+    std::stable_sort(groups.begin(), groups.begin() + (long)std::min(slots, groups.size()),
+                     [](const std::vector<Request *> &a, const std::vector<Request *> &b) {
+                       return group_ms(a) > group_ms(b);
+                     });
+  }
   std::vector<Request *> back;  // not launched this time: return to the queue
   for (auto &gr : groups) {
     const int slot = free_slot(s);
@@ -626,6 +658,14 @@ int admit(bwl_server *s) {
     const int rc = ok[0]->kind == KIND_ANNEAL ? launch_anneal_group(s, ok, slot)
                    : ok[0]->kind == KIND_NS   ? launch_ns_group(s, ok, slot)
                                               : launch_wl_group(s, ok, slot);
+    // (it starts when the queue's launches before it have ended)
+    if (rc == BWL_OK) {
+      Launch &last = *s->running.back();
+      double start = now_ms(s->t0);
+      for (const auto &L : s->running)
+        if (L.get() != &last && L->slot % s->hw_queues == slot % s->hw_queues) start = std::max(start, L->est_end);
+      last.est_end = start + group_ms(ok);
+    }
     if (rc == BWL_ERR_NOMEM) {
       for (Request *r : ok) {
         release_request(s, r);
@@ -693,6 +733,7 @@ int bwl_server_create(const bwl_server_params *p, bwl_server **out) {
     s->slot_busy.push_back(false);
   }
   s->batch_wait_ms = p->batch_wait_us / 1000.0;
+  if (const char *q = getenv("GPU_MAX_HW_QUEUES")) s->hw_queues = std::max(1, atoi(q));
   s->t0 = std::chrono::steady_clock::now();
   pinned_hold();
   s->held = true;
@@ -746,6 +787,7 @@ int bwl_server_submit_anneal(bwl_server *s, const bwl_lattice_desc *desc, const 
     s->reqs.erase(r->id);
     return rc;
   }
+  r->est_ms = 1e-3 * anneal_estimate_us(g, plan, *p);
   r->config.assign(config, config + (size_t)g.m[0] * g.m[1] * g.m[2]);
   r->ap = *p;
   r->E = energies_of_T;
@@ -806,6 +848,7 @@ int bwl_server_submit_ns(bwl_server *s, const bwl_lattice_desc *desc, const doub
   memcpy(r->mt, mt.mt, sizeof(r->mt));
   r->mti = mt.mti;
   r->np = *p;
+  r->est_ms = 0.61e-3 * p->n_iter * (double)p->n_steps + 6e-3 * p->n_walkers;
   r->e_limits = e_limits;
   r->block_bytes = ns_block_bytes(*r);
   if (r->block_bytes > s->arena.size) {
@@ -830,6 +873,7 @@ int bwl_server_submit_wl(bwl_server *s, const bwl_lattice_desc *desc, const doub
   if (!r) return rc;
   const Geo &g = r->g;
   r->wp = *p;
+  r->est_ms = 0.37e-3 * p->mc_sweeps * (double)g.n_atoms;
   r->wl_f = wl_f;
   r->windows.resize((size_t)2 * p->num_windows);
   r->edges.resize((size_t)p->bins + 1);
