@@ -191,9 +191,6 @@ struct AsroArgs {
 constexpr int kMaxAsroShells = 16;
 
 hipError_t launch_pack(const int8_t *ref, int8_t *compact, const Geo &g, hipStream_t s);
-// `count` reference-layout lattices back to back -> compact lattices back to back
-hipError_t launch_pack_many(const int8_t *ref, int8_t *compact, const Geo &g, int count,
-                            hipStream_t s);
 // n streams (args_dev[0..n)); any_drawn: not all of them were made on the host
 hipError_t launch_setup(const SetupArgs *args_dev, int n, int max_walkers, int max_atoms, bool any_drawn, hipStream_t s);
 hipError_t launch_unpack(const int8_t *compact, int8_t *ref, const Geo &g, hipStream_t s);

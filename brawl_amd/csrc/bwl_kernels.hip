@@ -44,10 +44,7 @@ __device__ inline int ref_to_compact(const Geo &g, const RefWalk &w) {
 }
 
 __global__ void k_pack(const int8_t *__restrict__ ref, int8_t *__restrict__ compact, Geo g) {
-  // blockIdx.y selects one of several lattices laid out back to back
   const int total = g.m[0] * g.m[1] * g.m[2];
-  ref += (size_t)blockIdx.y * total;
-  compact += (size_t)blockIdx.y * g.compact_bytes;
   for (int idx = 8 * (blockIdx.x * blockDim.x + threadIdx.x); idx < total; idx += 8 * gridDim.x * blockDim.x) {
     const uint64_t v = *(const uint64_t *)(ref + idx);
     RefWalk w = ref_walk(g, idx);
@@ -433,20 +430,10 @@ hipError_t launch_draw_sites(const DrawArgs &a, hipStream_t s) {
 // launchers
 // ------------------------------------------------------------------
 hipError_t launch_pack(const int8_t *ref, int8_t *compact, const Geo &g, hipStream_t s) {
-  return launch_pack_many(ref, compact, g, 1, s);
-}
-
-hipError_t launch_pack_many(const int8_t *ref, int8_t *compact, const Geo &g, int count,
-                            hipStream_t s) {
   int total = g.m[0] * g.m[1] * g.m[2] / 8;
   int blocks = (total + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  for (int first = 0; first < count; first += 65535) {
-    const int n = count - first < 65535 ? count - first : 65535;
-    hipLaunchKernelGGL(k_pack, dim3(blocks, n), dim3(256), 0, s,
-                       ref + (size_t)first * g.m[0] * g.m[1] * g.m[2],
-                       compact + (size_t)first * g.compact_bytes, g);
-  }
+  hipLaunchKernelGGL(k_pack, dim3(blocks), dim3(256), 0, s, ref, compact, g);
   return hipGetLastError();
 }
 
