@@ -280,7 +280,7 @@ __device__ __forceinline__ void metro_seq_run(const SeqArgs &A, uint8_t *smem) {
 // 1.2, 1.6 and 3.1 on bcc), a single trial 0.9, 0.9, 1.2 and 1.2 (0.8, 0.8, 1.0
 // and 1.2).  20,000 trials at 10^6 K (nothing rejected) of fcc 3^3 with four
 // shells: 61.5 ms in batches, 24.1 so (26.7 by k_metro_seq); of bcc 4^3 with
-// three 31.9 -> 19.6 (20.7); fcc 8^3 with two at 2000 K, where no batch is that
+// three 31.9 -> 19.6 (21.0); fcc 8^3 with two at 2000 K, where no batch is that
 // short, 0.387 -> 0.394 us a trial.
 // ------------------------------------------------------------------
 constexpr int kSingly = 16;

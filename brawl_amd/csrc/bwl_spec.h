@@ -64,7 +64,7 @@ struct SpecLds {
 };
 
 template <int KEY>
-__device__ inline void stage_spec_tables(int32_t *offp, uint8_t *adj, const int32_t *__restrict__ off) {
+__device__ inline void stage_spec_offsets(int32_t *offp, const int32_t *__restrict__ off) {
   using D = SpecDims<KEY>;
   for (int i = threadIdx.x; i < D::NSUB * D::R * D::ML; i += blockDim.x) {
     const int k = i % D::ML, n = (i / D::ML) % D::R, s = i / (D::ML * D::R);
@@ -75,6 +75,12 @@ __device__ inline void stage_spec_tables(int32_t *offp, uint8_t *adj, const int3
     }
     offp[i] = k < len ? off[s * D::Z + first + k] : 0;
   }
+}
+
+template <int KEY>
+__device__ inline void stage_spec_tables(int32_t *offp, uint8_t *adj, const int32_t *__restrict__ off) {
+  using D = SpecDims<KEY>;
+  stage_spec_offsets<KEY>(offp, off);
   for (int i = threadIdx.x; i < D::TS * D::TS * D::TS; i += blockDim.x) {
     const int dx = i % D::TS - D::RC, dy = (i / D::TS) % D::TS - D::RC, dz = i / (D::TS * D::TS) - D::RC;
     int at = 255;

@@ -962,7 +962,9 @@ __global__ __launch_bounds__(64) void k_wl_energies(const WlArgs *__restrict__ a
 
 // Reference-order total energies of walkers by whole workgroups
 // (spec_total_energy): block w is Wang-Landau walker w, or walker w of
-// nested-sampling run blockIdx.y with its energy jitter.
+// nested-sampling run blockIdx.y with its energy jitter.  (No table of list
+// positions, which took longer than a small box's energy: 8 walkers of bcc
+// 4^3 with four shells 58 us with it, 35 by one wavefront each.)
 template <int KEY>
 __device__ __forceinline__ double walker_energy(const Geo &geo, const int8_t *compact, const int32_t *off,
                                                 const double *v, uint8_t *smem) {
@@ -979,12 +981,11 @@ __device__ __forceinline__ double walker_energy(const Geo &geo, const int8_t *co
   double *vex = (double *)take(sizeof(double) * S * S * D::R);
   double *ebuf = (double *)take(sizeof(double) * 2 * kEnergyChunk);
   int32_t *offp = (int32_t *)take(4 * D::NSUB * D::R * D::ML);
-  uint8_t *adj = take(D::TS * D::TS * D::TS);
   for (int i = threadIdx.x; i < S * S * D::R; i += kSpecThreads) vex[i] = v[i];
-  stage_spec_tables<KEY>(offp, adj, off);
+  stage_spec_offsets<KEY>(offp, off);
   stage_codes(lat, compact, g, D::NSUB, S);
   __syncthreads();
-  return spec_total_energy<KEY>(SpecLds{lat, offp, vex, adj}, g, geo.n_atoms, S, inverse_of(S), ebuf);
+  return spec_total_energy<KEY>(SpecLds{lat, offp, vex, nullptr}, g, geo.n_atoms, S, inverse_of(S), ebuf);
 }
 
 template <int KEY>
