@@ -207,26 +207,46 @@ hipError_t launch_site_energy(const SiteArgs &a, hipStream_t s);
 // key: the pair-sum variant they share (pair_sum_key), -1 if they differ.
 // spec: the kernel in speculative batches (bwl_spec.h), for launches whose
 // members share a key and can all use it with the LDS there is (it takes
-// about 13 KB more).  It was faster on every lattice it accepts (a walk of
-// nested sampling, quinary fcc 6^3, 4 shells: 0.61 against 1.31 us per trial;
-// a Wang-Landau walker, bcc 16^3, 2 shells: 0.37 against 1.22 us; bit-exact
-// Metropolis, fcc 8^3, 2 shells: 0.25 against 0.81 us); the kernels of one
-// trial at a time serve the rest: more than 4 shells, boxes as short as the
-// interaction range, launches that mix lattices.
+// about 13 KB more): a walk of nested sampling, quinary fcc 6^3, 4 shells,
+// 0.61 against 1.31 us per trial; a Wang-Landau walker, bcc 16^3, 2 shells,
+// 0.37 against 1.22 us; bit-exact Metropolis, fcc 8^3, 2 shells, 0.25 against
+// 0.81 us.  The kernels of one trial at a time serve the rest: more than 4
+// shells, boxes as short as the interaction range, launches that mix lattices,
+// and launches of more chains than spec_pays allows.
+// reach: the share of a member's pairs of trials of which one's swap would
+// reach the other, about (up to 4 for the smallest boxes).
 struct SeqPick {
   int key = -2;  // no member yet
   bool spec = true;
   size_t lds = 0, lds_spec = 0;
+  double reach = 0.0;
   void add(const Geo &g, size_t lds_one, size_t lds_batches) {
     const int k = pair_sum_key(g.lattice, g.R);
     key = key == -2 || key == k ? k : -1;
     spec = spec && spec_ok(g);
     lds = lds_one > lds ? lds_one : lds;
     lds_spec = lds_batches > lds_spec ? lds_batches : lds_spec;
+    double near = 4.0;
+    for (int a = 0; a < 3; ++a) near *= 2 * g.rcut + 1 < g.m[a] ? (double)(2 * g.rcut + 1) / (double)g.m[a] : 1.0;
+    reach = near > reach ? near : reach;
   }
   void settle(int limit) { spec = spec && key > 0 && lds_spec <= (size_t)limit; }
-  size_t bytes() const { return spec ? lds_spec : lds; }
 };
+
+// Whether a launch of n workgroups of the speculative kernel `fn` (nullptr:
+// there is none) is faster than one trial at a time.  A chain alone gains from
+// foreseeing; once the device is full what counts is the work, and a batch is
+// more of it than its trials one by one, whose single wavefronts fit the
+// device many more times.  So: while all workgroups are resident at once, and
+// up to twice as many where swaps seldom cut a batch short (reach at most
+// `far`).  Against one trial at a time, nothing rejected and all rejected:
+// Wang-Landau, resident 0.96-2.9x and 2.0-6.1x, twice that with reach 0.12
+// (fcc 8^3, 4 shells; bcc 8^3, 3) 1.21x and 1.19x, 2.6x and 2.8x, with reach
+// 0.5 (fcc 5^3, 4 shells) 0.76x; nested sampling, resident 0.97-2.5x, twice
+// that 1.3x with reach 0.12, 0.65x on the smallest boxes; Metropolis on fcc
+// 6^3, 4 shells, at 2000 K 1.1x with 256 chains (resident) and 0.30x with
+// 1024, on fcc 12^3, 2 shells, 1.3x with twice the resident chains.
+bool spec_pays(const void *fn, int n, const SeqPick &pick, double far);
 
 // Launches `fn` with `lds` bytes of dynamic LDS.
 inline hipError_t launch_dynamic(const void *fn, dim3 grid, int threads, void **kargs, size_t lds, hipStream_t s) {

@@ -655,17 +655,34 @@ size_t seq_spec_lds_bytes(const Geo &g) {
   return spec_table_bytes(g) + spec_ring_bytes() + spec_energy_bytes() + spec_align(sums);
 }
 
+bool spec_pays(const void *fn, int n, const SeqPick &pick, double far) {
+  if (!fn) return false;
+  int dev = 0, n_cu = 0, resident = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return false;
+  if (n <= n_cu) return true;
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pick.lds_spec) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, fn, kSpecThreads, pick.lds_spec) != hipSuccess)
+    return false;
+  const long long room = (long long)n_cu * resident;
+  return n <= room || (pick.reach <= far && n <= 2 * room);
+}
+
 hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s) {
   SeqArgs arg = a;
   void *kargs[] = {(void *)&arg};
-  return launch_dynamic(pick.spec ? metro_seq_spec_kernel(pick.key) : metro_seq_kernel(pick.key), dim3(1),
-                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
+  if (pick.spec) return launch_dynamic(metro_seq_spec_kernel(pick.key), dim3(1), kSpecThreads, kargs, pick.lds_spec, s);
+  return launch_dynamic(metro_seq_kernel(pick.key), dim3(1), 64, kargs, pick.lds, s);
 }
 
 hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  return launch_dynamic(pick.spec ? metro_seq_spec_batch_kernel(pick.key) : metro_seq_batch_kernel(pick.key), dim3(n),
-                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
+  const void *fn = pick.spec ? metro_seq_spec_batch_kernel(pick.key) : nullptr;
+  // (a batch here is 64 places' energies: the more shells, the sooner too much)
+  if (spec_pays(fn, n, pick, pick.key % 16 <= 2 ? 0.05 : 0.0))
+    return launch_dynamic(fn, dim3(n), kSpecThreads, kargs, pick.lds_spec, s);
+  return launch_dynamic(metro_seq_batch_kernel(pick.key), dim3(n), 64, kargs, pick.lds, s);
 }
 
 // ------------------------------------------------------------------

@@ -1346,14 +1346,24 @@ size_t ns_lds_bytes(const Geo &g, int n_walkers) {
                         sizeof(int32_t) * g.nsub * g.z);
 }
 
+constexpr double kWalkersFar = 0.125;  // see spec_pays
+
 hipError_t launch_ns(const NsArgs *args_dev, int n, const SeqPick &pick, int max_walkers, const SeqPick &energies,
                      hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  hipError_t e = launch_dynamic(energies.spec ? ns_energies_spec_kernel(energies.key) : (const void *)k_ns_energies,
-                                dim3(max_walkers, n), energies.spec ? kSpecThreads : 64, kargs, energies.bytes(), s);
+  const dim3 walkers(max_walkers, n);
+  const void *fn = pick.spec ? ns_spec_kernel(pick.key) : nullptr;
+  const bool spec = spec_pays(fn, n, pick, kWalkersFar);
+  // (energies in workgroups of one wavefront before runs of one: 1024 runs
+  // after workgroups of four were spread unevenly over the SIMDs, fcc 3^3 with
+  // four shells 2.34 ms against 1.81)
+  const hipError_t e =
+      energies.spec && spec
+          ? launch_dynamic(ns_energies_spec_kernel(energies.key), walkers, kSpecThreads, kargs, energies.lds_spec, s)
+          : launch_dynamic((const void *)k_ns_energies, walkers, 64, kargs, energies.lds, s);
   if (e != hipSuccess) return e;
-  return launch_dynamic(pick.spec ? ns_spec_kernel(pick.key) : ns_kernel(pick.key), dim3(n),
-                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
+  if (spec) return launch_dynamic(fn, dim3(n), kSpecThreads, kargs, pick.lds_spec, s);
+  return launch_dynamic(ns_kernel(pick.key), dim3(n), 64, kargs, pick.lds, s);
 }
 
 size_t ns_energies_lds_bytes(const Geo &g) {
@@ -1369,8 +1379,9 @@ size_t wl_lds_bytes(const Geo &g, int bins, int window_bins) {
 
 hipError_t launch_wl_sweeps(const WlArgs *args_dev, int n, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  return launch_dynamic(pick.spec ? wl_sweeps_spec_kernel(pick.key) : wl_sweeps_kernel(pick.key), dim3(n),
-                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
+  const void *fn = pick.spec ? wl_sweeps_spec_kernel(pick.key) : nullptr;
+  if (spec_pays(fn, n, pick, kWalkersFar)) return launch_dynamic(fn, dim3(n), kSpecThreads, kargs, pick.lds_spec, s);
+  return launch_dynamic(wl_sweeps_kernel(pick.key), dim3(n), 64, kargs, pick.lds, s);
 }
 
 hipError_t launch_wl_average(double *lng, double *hist, int n_windows, int wpw, int bins,
@@ -1383,8 +1394,9 @@ hipError_t launch_wl_average(double *lng, double *hist, int n_windows, int wpw, 
 
 hipError_t launch_wl_energies(const WlArgs *args_dev, int n, double *E, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev, (void *)&E};
-  return launch_dynamic(pick.spec ? wl_energies_spec_kernel(pick.key) : (const void *)k_wl_energies, dim3(n),
-                        pick.spec ? kSpecThreads : 64, kargs, pick.bytes(), s);
+  if (pick.spec)
+    return launch_dynamic(wl_energies_spec_kernel(pick.key), dim3(n), kSpecThreads, kargs, pick.lds_spec, s);
+  return launch_dynamic((const void *)k_wl_energies, dim3(n), 64, kargs, pick.lds, s);
 }
 
 size_t wl_exchange_lds_bytes(int W, int wpw) {

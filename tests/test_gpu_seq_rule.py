@@ -1,6 +1,7 @@
-"""Where the sequential sampler leaves its speculative batches (kBatchPays):
-chains that take their trials singly give the same results, and boxes whose
-batches are cut short no longer pay for whole ones."""
+"""Where the sequential samplers leave their speculative batches (spec_pays,
+kBatchPays): chains that take their trials singly and launches of more chains
+than are resident at once give the same results, and neither costs more than
+a run that never left them would show."""
 import numpy as np
 import pytest
 
@@ -86,3 +87,83 @@ def test_energies_of_small_boxes(hip):
     for L in Ls:
         L.close()
     assert ms < 0.1
+
+
+def _chains(hip, count, lat, n, S, R):
+    from brawl_amd import workloads
+    v = _v(S, R)
+    rng = np.random.default_rng(3)
+    cfg = workloads.random_config(lat, n, workloads.equal_counts(workloads.n_atoms_of(lat, n), S), rng)
+    out = []
+    for k in range(count):
+        L = hip.Lattice(lat, n, v)
+        L.set_config(cfg)
+        L.seed(50 + k)
+        out.append(L)
+    return out
+
+
+@pytest.mark.parametrize("lat,n,S,R", [(1, (3, 3, 3), 5, 4), (2, (4, 4, 4), 2, 1)])
+def test_more_chains_than_resident(hip, lat, n, S, R):
+    from brawl_amd.lattice import mc_steps_batch
+    from brawl_amd.nested_sampling import nested_sampling_batch
+    count = 2000 if R == 1 else 600
+    Ls = _chains(hip, count, lat, n, S, R)
+    acc, e, _ = mc_steps_batch(Ls, [hip.beta_of(2000.0)] * count, 300, sample_every=100)
+    alone = {}
+    for k in (0, 1, count // 2, count - 1):
+        alone[k], = _chains(hip, 1, lat, n, S, R)
+        alone[k].seed(50 + k)
+        a, ea = alone[k].mc_steps(hip.beta_of(2000.0), 300, sample_every=100)
+        assert a == acc[k] and np.array_equal(ea, e[k])
+        assert np.array_equal(alone[k].get_config(), Ls[k].get_config())
+        assert all(np.array_equal(x, y) for x, y in zip(alone[k].genrand_state(), Ls[k].genrand_state()))
+    p = dict(n_walkers=4, n_steps=20, n_iter=5, concentrations=np.full(S, 1.0 / S))
+    res, _ = nested_sampling_batch(Ls, [p] * count)
+    for k in alone:
+        one, _ = nested_sampling_batch([alone[k]], [p])
+        assert np.array_equal(one[0][0], res[k][0])
+        assert all(np.array_equal(x, y) for x, y in zip(alone[k].genrand_state(), Ls[k].genrand_state()))
+    for L in Ls + list(alone.values()):
+        L.close()
+
+
+def test_many_chains_do_not_take_turns(hip):
+    """1024 chains of 4 shells: 7 times as long as 256 in batches alone, which
+    one CU holds one chain of; about the same time one trial at a time."""
+    from brawl_amd.lattice import mc_steps_batch
+    Ls = _chains(hip, 1024, 1, (6, 6, 6), 4, 4)
+    beta = hip.beta_of(2000.0)
+
+    def kernel_ms(count):
+        return min(mc_steps_batch(Ls[:count], [beta] * count, 1000)[2] for _ in range(3))
+
+    few, many = kernel_ms(256), kernel_ms(1024)
+    print(f"256 chains {few:.2f} ms, 1024 chains {many:.2f} ms")
+    for L in Ls:
+        L.close()
+    assert many < 2.5 * few
+
+
+def test_more_walkers_than_resident(hip):
+    """Wang-Landau walkers of a launch taken one trial at a time against the
+    same walkers a few at a time, which take theirs in batches."""
+    from brawl_amd import workloads
+    from brawl_amd.wang_landau import WangLandau
+    n, S, R = (3, 3, 3), 5, 4
+    p = dict(bins=24, num_windows=1, bin_overlap=0.1, energy_min=-12.0, energy_max=12.0, mc_sweeps=2)
+    cfg = workloads.random_config(1, n, workloads.equal_counts(108, S), np.random.default_rng(2))
+
+    def run(walkers, first):
+        with WangLandau(1, n, _v(S, R), walkers_per_window=walkers, rank_offset=first, **p) as w:
+            for k in range(walkers):
+                w.set_walker(k, cfg)
+            acc, _ = w.sweeps(0.01, average=False)
+            return acc, *w.lng_hist(), [w.get_walker(k) for k in (0, walkers - 1)]
+
+    acc, lng, hist, ends = run(1500, 7)
+    for first in (0, 1496):
+        a, g, h, e = run(4, 7 + first)
+        assert np.array_equal(a, acc[first:first + 4]) and a.sum() > 0
+        assert np.array_equal(g, lng[first:first + 4]) and np.array_equal(h, hist[first:first + 4])
+        assert np.array_equal(e[0], ends[0]) if first == 0 else np.array_equal(e[1], ends[1])
