@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <mutex>
@@ -395,6 +396,7 @@ int bwl_mc_steps(bwl_ctx *c, double beta, int32_t nbr_swap, int64_t n_trials, in
   a.sample_every = energies ? sample_every : 0;
   memcpy(a.mt, c->mt.mt, 624 * 4);
   *a.mt_index = c->mt.mti;
+  const CuUse use(c->device, 1);
   HIP_OK(launch_metro_seq(a, pick, c->stream));
   if (n_samples && !e_pinned)
     HIP_OK(hipMemcpyAsync(energies, a.energies, e_bytes, hipMemcpyDeviceToHost, c->stream));
@@ -467,6 +469,7 @@ int bwl_mc_steps_batch(int32_t n, bwl_ctx *const *ctxs, const double *beta, int3
   }
   HIP_OK(hipMemcpyAsync(base, args, sizeof(SeqArgs) * (size_t)n, hipMemcpyHostToDevice, s));
   if (!io_pinned) HIP_OK(hipMemcpyAsync(io, host, io_bytes, hipMemcpyHostToDevice, s));
+  const CuUse use(ctxs[0]->device, n);
   HIP_OK(hipEventRecord(ctxs[0]->ev0, s));
   HIP_OK(launch_metro_seq_batch((const SeqArgs *)base, n, pick, s));
   HIP_OK(hipEventRecord(ctxs[0]->ev1, s));
@@ -697,13 +700,18 @@ static double divided_us(const AnnealPlan::Item &it) { return it.rounds * 2.4; }
 // parts 7.4, 4 parts 7.7), else two.
 //
 // The parts of a chain go to one XCD (lane), which has n_cu / 8 CUs: as many
-// as other chains of this and other calls leave free.  Parts and undivided
-// chains together have a CU each: a batch of 256 uneven chains, eight of them
-// fcc 24^3, took 184 ms with those eight divided (smaller chains then share
-// CUs with parts that all the others wait for) and 144 with none.
+// as this process's calls in flight (CuUse, SplitShare) and the call's other
+// chains leave free, but half an XCD in any case: the parts are launched
+// before those other chains (200 fcc 16^3 and one bcc 32^3, 16 parts: 20.0 ms,
+// undivided 30.5).  Parts and undivided chains together have a CU each: a
+// batch of 256 uneven chains, eight of them fcc 24^3, took 184 ms with those
+// eight divided (smaller chains then share CUs with parts that all the others
+// wait for) and 144 with none.  Equally free XCDs are taken from one on that
+// differs by process, since processes that share a device do not see each
+// other's.
 static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu, int lim) {
   const int n = (int)P.items.size();
-  const int cap = std::max(n_cu / 8 - (n + 7) / 8, n_cu / 16);
+  const int cap = std::max(n_cu / 8 - (n + 7) / 8, n_cu / 16), first = (int)((unsigned)getpid() % 8u);
   int lanes[8], blocks = n;
   bool any = false;
   for (int x = 0; x < 8; ++x) {
@@ -731,15 +739,22 @@ static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu,
       const int parts = (rows + rows_each - 1) / rows_each;
       if (!par_split_fits(it.a.nat, it.threads, parts, it.passes)) continue;
       const double load_then = load + parts * divided_us(it) - undivided_us(it) * share(it);
-      int to = 0;
+      int to = first;
       for (int x = 1; x < 8; ++x)
-        if (lanes[x] > lanes[to]) to = x;
+        if (lanes[(first + x) % 8] > lanes[to]) to = (first + x) % 8;
       if (parts > lanes[to] || blocks + parts - 1 > n_cu || load_then > n_cu * undivided_us(it)) continue;
       blocks += parts - 1;
       load = load_then;
       lanes[to] -= parts;
       it.a.parts = parts;
       it.lane = to;
+      // CUs that other processes hold may keep some of the parts from
+      // arriving; the others wait for a quarter of what the division saves,
+      // 0.2 to 5 ms, then the chain runs undivided (bcc 32^3, 40 sweeps, while
+      // another process's chains had 200 CUs: 11 to 18 ms, 1029 with 1 s of
+      // patience)
+      const double wait_us = std::min(5000.0, std::max(200.0, 0.25 * (undivided_us(it) - divided_us(it))));
+      it.a.patience = (int32_t)(100.0 * wait_us);
       return true;
     }
     return false;
@@ -1074,13 +1089,15 @@ int bwl_metropolis_anneal_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_annea
 
 namespace {
 
-// The workgroups of divided chains on each of a device's XCDs, over all calls
-// in this process: the parts of a chain wait for each other, so together they
-// must not outnumber the CUs.  A call takes what is free, keeps what its plan
-// uses and gives it back when its launches have ended.
+// The workgroups of divided chains on each of a device's XCDs, and the
+// undivided ones on the whole device (they go to the XCDs in turn), over all
+// calls in this process: the parts of a chain wait for each other, so together
+// they must not outnumber the CUs.  A call takes what is free, keeps what its
+// plan uses and gives it back when its launches have ended.
 constexpr int kMaxSplitDevices = 64;
 std::mutex g_split_mu;
 SplitLanes g_split_used[kMaxSplitDevices];
+long long g_undivided[kMaxSplitDevices];
 
 struct SplitShare {
   int device = -1;
@@ -1090,7 +1107,7 @@ struct SplitShare {
     std::lock_guard<std::mutex> lock(g_split_mu);
     device = dev;
     for (int x = 0; x < 8; ++x) {
-      held.parts[x] = std::max(0, n_cu / 8 - g_split_used[dev].parts[x]);
+      held.parts[x] = (int)std::max(0LL, n_cu / 8 - g_split_used[dev].parts[x] - (g_undivided[dev] + 7) / 8);
       g_split_used[dev].parts[x] += held.parts[x];
     }
   }
@@ -1109,6 +1126,22 @@ struct SplitShare {
 
 namespace bwl {
 
+CuUse::CuUse(int device, long long workgroups) {
+  if (device < 0 || device >= kMaxSplitDevices || workgroups < 1) return;
+  int n_cu = 0;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return;
+  device_ = device;
+  n_ = (int)std::min(workgroups, (long long)n_cu);
+  std::lock_guard<std::mutex> lock(g_split_mu);
+  g_undivided[device_] += n_;
+}
+
+CuUse::~CuUse() {
+  if (device_ < 0) return;
+  std::lock_guard<std::mutex> lock(g_split_mu);
+  g_undivided[device_] -= n_;
+}
+
 int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, double *const *energies_of_T,
                double *const *C_of_T, double *const *acceptance_of_T, bwl_run_stats *stats, double *makespan_ms,
                double *const *rho_of_T, bool divide) {
@@ -1126,6 +1159,8 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   if (rc) return rc;
   share.keep(P.split);
   bwl_ctx *c0 = ctxs[0];
+  const CuUse rest(c0->device, std::count_if(P.items.begin(), P.items.end(),
+                                             [](const AnnealPlan::Item &it) { return it.a.parts == 1; }));
   rc = ensure_scratch(c0, P.scratch_bytes);
   if (rc) return rc;
   char *const scratch = (char *)c0->d_scratch;

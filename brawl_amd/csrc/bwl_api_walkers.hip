@@ -336,6 +336,7 @@ int bwl_nested_sampling_batch(int32_t n, bwl_ctx *const *ctxs, const bwl_ns_para
   memcpy(host.data(), args.data(), sizeof(NsArgs) * (size_t)n);
   memcpy(host.data() + args_bytes, sets.data(), sizeof(SetupArgs) * (size_t)n);
   HIP_OK(hipMemcpyAsync(base, host.data(), io_bytes, hipMemcpyHostToDevice, c0->stream));
+  const CuUse use(c0->device, n);
   HIP_OK(launch_setup((const SetupArgs *)(base + args_bytes), n, max_w, max_atoms, any_drawn, c0->stream));
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
   HIP_OK(launch_ns((const NsArgs *)base, n, pick, max_w, energies, c0->stream));
@@ -612,6 +613,7 @@ int bwl_wl_enter_windows(bwl_wl *w, int64_t max_trials, int64_t *trials, int32_t
   const size_t lds = wl_enter_lds_bytes(g);
   bool first = true;
   std::vector<int8_t> cfg((size_t)g.m[0] * g.m[1] * g.m[2]);
+  const CuUse use(w->ctx->device, W);
   for (;;) {
     // walkers still walking (status 1 or 2) and under the trial bound
     std::vector<int> act;
@@ -696,6 +698,7 @@ int bwl_wl_sweeps(bwl_wl *w, double wl_f, int32_t average, int64_t *accepted, do
   SeqPick pick;
   pick.add(g, wl_lds_bytes(g, w->p.bins, w->hstride), wl_spec_lds_bytes(g, w->p.bins, w->hstride));
   pick.settle(lds_limit());
+  const CuUse use(w->ctx->device, W);
   HIP_OK(launch_wl_sweeps(w->d_args, W, pick, s));
   if (average)
     HIP_OK(launch_wl_average(w->d_lng, w->d_hist, w->p.num_windows, w->p.walkers_per_window,

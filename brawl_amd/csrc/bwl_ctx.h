@@ -103,6 +103,21 @@ struct SplitLanes {
   int parts[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 };
 
+// The undivided workgroups of a call or launch while it is in flight, a CU
+// each (a device's at most): those CUs are not offered to chains that could be
+// divided.  Calls of one short kernel (an energy, a configuration) are not
+// counted; the parts of a chain wait that long for their CUs.
+class CuUse {
+ public:
+  CuUse(int device, long long workgroups);
+  ~CuUse();
+  CuUse(const CuUse &) = delete;
+  CuUse &operator=(const CuUse &) = delete;
+
+ private:
+  int device_ = -1, n_ = 0;
+};
+
 // A batch of anneals prepared on the host (anneal_plan), its arguments and
 // buffers placed in caller-provided device memory (anneal_upload), its
 // launches enqueued one group per stream (anneal_launch), and its outputs

@@ -88,6 +88,7 @@ struct ParArgs {
   // a chain divided over several workgroups (bwl_metro_split.hip)
   int32_t parts;         // workgroups
   int32_t passes;        // most pairs a thread has in a round
+  int32_t patience;      // ticks of 10 ns that the parts wait for each other to arrive
   unsigned long long *mail;  // par_split_mail_words words, zeroed
 };
 

@@ -11,7 +11,10 @@ namespace {
 
 constexpr int kSplitThreads = 512;  // 8 wavefronts with up to 256 registers each: no spills
 constexpr int kSplitWaves = kSplitThreads / 64;
-constexpr long long kSplitPatience = 100000000LL;  // ticks of 10 ns a wait may take (1 s)
+// Ticks of 10 ns (1 s) that a wait for another part's word may take once all
+// have arrived: they are resident then, so only a device taken away for that
+// long ends one.  Arriving they wait ParArgs::patience.
+constexpr long long kSplitPatience = 100000000LL;
 
 // Mailbox, in 64-bit words.  Per round (4 slots in turn) and part: a header
 // per half row, then the records; then the sums of the rows (2 slots), the
@@ -33,14 +36,16 @@ __device__ __forceinline__ void mail_store(unsigned long long *p, unsigned long 
 // Whether a wait has lasted too long or the chain has been given up; called
 // once per poll.
 struct Patience {
+  long long limit = kSplitPatience;
+  uint32_t between = 1023;  // polls, less one, from one look at the clock to the next
   uint32_t tries = 0;
   long long since = 0;
   __device__ __forceinline__ bool over(unsigned long long *gone) {
-    if ((++tries & 1023u) != 0) return false;
+    if ((++tries & between) != 0) return false;
     const long long now = wall_clock64();
     if (since == 0) since = now;
     if (mail_load(gone) != 0) return true;
-    if (now - since <= kSplitPatience) return false;
+    if (now - since <= limit) return false;
     if ((threadIdx.x & 63) == 0) mail_store(gone, 1);
     return true;
   }
@@ -49,8 +54,7 @@ struct Patience {
 // Polls the lanes' words until each (of the lanes that want one) carries
 // `tag` in its upper half; false when the chain has been given up.
 __device__ __forceinline__ bool mail_wait(const unsigned long long *p, bool want, uint32_t tag, unsigned long long *gone,
-                                          unsigned long long &v) {
-  Patience wait;
+                                          unsigned long long &v, Patience wait = Patience()) {
   for (;;) {
     v = (unsigned long long)tag << 32;
     if (want) v = mail_load(p);
@@ -183,7 +187,9 @@ __device__ __forceinline__ void metro_split(const ParArgs &C, const int part, ui
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcd));
     if (tid == 0) mail_store(&mxcd[part], (1ull << 32) | xcd);
     unsigned long long v = 0;
-    if (!mail_wait(&mxcd[lane < parts ? lane : 0], lane < parts, 1, gone, v)) *dead = 1;
+    if (!mail_wait(&mxcd[lane < parts ? lane : 0], lane < parts, 1, gone, v, Patience{C.patience, 15}) ||
+        mail_load(gone) != 0)
+      *dead = 1;
     one_xcd = __ballot(lane < parts && (uint32_t)v != xcd) == 0;
   }
   auto post = [&](unsigned long long *p, unsigned long long v) {

@@ -62,6 +62,7 @@ int bwl_metropolis_anneal_noalloc(bwl_ctx *c, const bwl_anneal_params *p, double
   char *base = nullptr;
   rc = scratch_ptr(c->device, &base);
   if (rc) return rc;
+  const CuUse use(c->device, 1);
   HIP_OK(hipEventRecord(c->ev0, c->stream));
   rc = anneal_upload(P, base, c->stream);  // (an undivided chain: no memset)
   if (rc) return rc;

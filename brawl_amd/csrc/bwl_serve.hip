@@ -134,6 +134,7 @@ struct Launch {
   int kind = 0;
   int slot = -1;
   double est_end = 0;  // about when it ends, on the server's clock
+  std::unique_ptr<CuUse> use;
   std::vector<Request *> reqs;
   std::unique_ptr<AnnealPlan> plan;
   std::vector<NsArgs> ns_args;
@@ -380,6 +381,7 @@ int launch_anneal_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   L->scratch_bytes = L->plan->scratch_bytes;
   L->scratch = s->arena.alloc(L->scratch_bytes);
   if (!L->scratch) return BWL_ERR_NOMEM;  // caller requeues
+  L->use = std::make_unique<CuUse>(ctxs[0]->device, (long long)grp.size());
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
@@ -476,6 +478,7 @@ int launch_ns_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
   for (Request *r : grp) max_w = std::max(max_w, r->np.n_walkers);
   const int rc = launch_setups(*L, L->scratch + al(sizeof(NsArgs) * grp.size()), max_w, st);
   if (rc) return rc;
+  L->use = std::make_unique<CuUse>(grp[0]->ctx->device, (long long)grp.size());
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));
@@ -569,6 +572,7 @@ int launch_wl_group(bwl_server *s, std::vector<Request *> &grp, int slot) {
                         hipMemcpyHostToDevice, st));
   const int rc = launch_setups(*L, L->scratch + al(sizeof(WlArgs) * total_w), 1, st);
   if (rc) return rc;
+  L->use = std::make_unique<CuUse>(grp[0]->ctx->device, (long long)total_w);
   HIP_OK(hipEventCreate(&L->ev0));
   HIP_OK(hipEventCreate(&L->ev1));
   HIP_OK(hipEventRecord(L->ev0, st));

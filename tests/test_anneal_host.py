@@ -1,0 +1,87 @@
+"""The host side of an anneal without a device (tests/fake_hip.cpp): what is
+launched, in how many workgroups, and what has been waited for.  Each test
+runs in a process of its own, which loads the fake runtime before the library."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+PRELUDE = """
+import ctypes as C, os, sys
+sys.path.insert(0, {root!r})
+fake = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+import numpy as np
+from brawl_amd import Lattice, BrawlError, anneal_batch, workloads
+LAUNCH = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_longlong, C.c_void_p)
+launches = []
+def record(fn, grid, block, lds, stream):
+    launches.append((fn, grid, block, lds, stream))
+    return 0
+def on_launch(f):
+    on_launch.keep = LAUNCH(f)
+    fake.fake_on_launch(on_launch.keep)
+def lattice(lat, n, S, R):
+    v = workloads.random_v(S, [25.0 / k for k in range(1, R + 1)], 3)
+    L = Lattice(lat, n, v)
+    L.set_config(workloads.random_config(lat, n, workloads.equal_counts(L.n_atoms, S), np.random.default_rng(1)))
+    return L
+def grids(f):
+    launches.clear()
+    f()
+    return [l[1] for l in launches]
+P = dict(T=900.0, n_sweeps=50, seed=1)
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", so], check=True)
+
+    def go(body):
+        code = PRELUDE.format(root=ROOT, so=so) + textwrap.dedent(body)
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return go
+
+
+def test_divided_only_into_cus_that_are_free(run):
+    """A large anneal that starts while another call's chains are in flight
+    (its launch is made from inside that call's) is divided into what they
+    leave of an XCD, and is divided again once they have ended."""
+    run("""
+    big = lattice(2, (32, 32, 32), 4, 4)
+    small = [lattice(1, (16, 16, 16), 2, 2) for _ in range(200)]
+    few = small[:30]
+    anneal = lambda: big.metropolis_simulated_annealing(**P)
+    on_launch(record)
+    alone = grids(anneal)
+    # (nothing runs, so the division is given up and made good undivided)
+    assert len(alone) == 2 and alone[0] == 8 * 16 and alone[1] == 1, alone
+
+    def during(call, inner):
+        seen = []
+        def f(fn, grid, block, lds, stream):
+            if not seen:
+                seen.append(None)
+                on_launch(record)
+                seen[0] = grids(inner)
+            return 0
+        on_launch(f)
+        keep = on_launch.keep
+        call()
+        return seen[0]
+
+    batch = lambda chains: anneal_batch(chains, [dict(P, seed=k) for k in range(len(chains))])
+    assert during(lambda: batch(small), anneal) == [1]        # 25 a CU's worth on each XCD: 7 left
+    assert during(lambda: batch(few), anneal)[0] == 8 * 16     # 4 on each
+    from brawl_amd.lattice import mc_steps_batch
+    assert during(lambda: mc_steps_batch(small, [1.0] * 200, 10), anneal) == [1]
+    assert grids(anneal)[0] == 8 * 16
+    """)
