@@ -930,6 +930,7 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
       AnnealPlan::Item &it = P.items[(size_t)i];
       it.lds = par_split_lds_bytes(it.a.g, it.a.nat);
       it.fn = fn;
+      it.alone = true;
     }
   }
   // LDS per launch: the largest member's need at the group's block size
@@ -1187,6 +1188,15 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
   rc = anneal_upload(P, scratch, c0->stream, pin.p);
   if (rc) return rc;
+  static const unsigned long long kGone = 1;
+  for (int i = 0; i < n; ++i) {
+    const AnnealPlan::Item &it = P.items[(size_t)i];
+    ctxs[i]->ran[0] = it.a.parts;
+    ctxs[i]->ran[1] = 0;
+    ctxs[i]->ran[2] = it.alone ? 1 : 0;
+    if (it.mail_n && ctxs[i]->give_up)  // (the mailbox ends with the word that gives a chain up)
+      HIP_OK(hipMemcpyAsync(it.a.mail + it.mail_n - 1, &kGone, sizeof(kGone), hipMemcpyHostToDevice, c0->stream));
+  }
   HIP_OK(hipEventRecord(ready, c0->stream));
   for (size_t k = 1; k < streams.size(); ++k) HIP_OK(hipStreamWaitEvent(streams[k], ready, 0));
   rc = anneal_launch(P, streams.data());
@@ -1224,10 +1234,26 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   rc = anneal_run((int)again.size(), cs.data(), ps.data(), e.data(), cv.data(), ac.data(), st.data(), &more_ms,
                   rho_of_T ? rh.data() : nullptr, false);
   if (rc) return rc;
-  for (size_t k = 0; k < again.size(); ++k)
+  for (size_t k = 0; k < again.size(); ++k) {
     if (stats) stats[again[k]] = st[k];
+    cs[k]->ran[1] = 1;
+  }
   if (makespan_ms) *makespan_ms = ms + more_ms;
   return BWL_OK;
 }
 
 }  // namespace bwl
+
+extern "C" {
+
+int bwl_test_anneal_ran(const bwl_ctx *c, int32_t *ran3) {
+  memcpy(ran3, c->ran, sizeof(c->ran));
+  return BWL_OK;
+}
+
+int bwl_test_give_up(bwl_ctx *c, int32_t on) {
+  c->give_up = on != 0;
+  return BWL_OK;
+}
+
+}  // extern "C"

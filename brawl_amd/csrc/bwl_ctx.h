@@ -52,6 +52,10 @@ struct bwl_ctx {
   bool borrowed = false;  // device memory and stream belong to someone else
   int32_t layout = 0;     // parallel-sampler layout: 0 by rule, else BWL_LAYOUT_*
   int32_t threads = 0;    // parallel-sampler threads per chain: 0 by rule
+  // how the last anneal ran: workgroups, whether its division was given up,
+  // whether it took one site per lane in one workgroup
+  int32_t ran[3] = {0, 0, 0};
+  bool give_up = false;  // the parts of a divided anneal find it given up
 };
 
 namespace bwl {
@@ -134,6 +138,7 @@ struct AnnealPlan {
     size_t off_mail = 0, mail_n = 0;  // mailbox of a divided chain, in words
     const void *split_fn = nullptr;   // kernel that can divide the chain, if any
     bool natural = false;             // held in lattice coordinates
+    bool alone = false;               // runs k_metro_alone
     int chunks = 0, passes = 0;       // most pairs of a round, in 64s and per thread
     int lane = 0;                     // XCD of a divided chain's parts
     double rounds = 0.0;              // rounds of the whole anneal, about
@@ -192,3 +197,10 @@ struct DevBuf {
 };
 
 }  // namespace bwl
+
+// For the tests, which have no other way to see or to force it (not part of
+// include/brawl_hip.h): bwl_ctx::ran, and bwl_ctx::give_up.
+extern "C" {
+int bwl_test_anneal_ran(const bwl_ctx *c, int32_t *ran3);
+int bwl_test_give_up(bwl_ctx *c, int32_t on);
+}

@@ -85,3 +85,20 @@ def test_divided_only_into_cus_that_are_free(run):
     assert during(lambda: mc_steps_batch(small, [1.0] * 200, 10), anneal) == [1]
     assert grids(anneal)[0] == 8 * 16
     """)
+
+
+def test_given_up_division_is_made_good(run):
+    """The chain that did not complete is run again undivided, its results
+    and those of the others are whole."""
+    run("""
+    lib = Lattice(1, (1, 1, 1), np.zeros((2, 2, 1)))._L
+    on_launch(record)
+    chains = [lattice(1, (24, 24, 24), 3, 3), lattice(1, (8, 8, 8), 2, 2)]
+    got = grids(lambda: anneal_batch(chains, [P, dict(P, seed=2)]))
+    assert len(got) == 3 and got[0] > 8 and got[1:] == [1, 1], got
+    ran = (C.c_int32 * 3)()
+    lib.bwl_test_anneal_ran(chains[0]._h, ran)
+    assert list(ran)[:2] == [1, 1]
+    lib.bwl_test_anneal_ran(chains[1]._h, ran)
+    assert list(ran) == [1, 0, 1]
+    """)
