@@ -103,7 +103,10 @@ int bwl_destroy(bwl_ctx *c) {
   if (!c) return BWL_OK;
   (void)hipSetDevice(c->device);
   if (c->stream && !c->borrowed) (void)hipStreamSynchronize(c->stream);
-  for (hipStream_t s : c->side) (void)hipStreamDestroy(s);
+  for (hipStream_t s : c->side) {
+    (void)hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
+  }
   if (!c->borrowed) {
     (void)hipFree(c->d_compact);
     (void)hipFree(c->d_ref);
@@ -1185,6 +1188,15 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   Pinned pin;
   const bool pinned = P.up_bytes <= kPinnedSeries;
   if (pinned && !pin.take(P.up_bytes, c0->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
+  // what is queued when the call ends early reads the scratch and the pinned
+  // block and holds CUs: it is waited for before any of these is given back
+  struct Waits {
+    const std::vector<hipStream_t> *streams;
+    ~Waits() {
+      if (streams)
+        for (hipStream_t s : *streams) (void)hipStreamSynchronize(s);
+    }
+  } waits{&streams};
   HIP_OK(hipEventRecord(c0->ev0, c0->stream));
   rc = anneal_upload(P, scratch, c0->stream, pin.p);
   if (rc) return rc;
@@ -1210,6 +1222,7 @@ int anneal_run(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, dou
   }
   HIP_OK(hipEventRecord(c0->ev1, c0->stream));
   HIP_OK(hipStreamSynchronize(c0->stream));
+  waits.streams = nullptr;
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, c0->ev0, c0->ev1);
   if (makespan_ms) *makespan_ms = ms;

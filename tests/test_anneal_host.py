@@ -102,3 +102,34 @@ def test_given_up_division_is_made_good(run):
     lib.bwl_test_anneal_ran(chains[1]._h, ran)
     assert list(ran) == [1, 0, 1]
     """)
+
+
+def test_error_exits_wait_for_what_was_queued(run):
+    """A batch of three kernels whose first, second or third launch fails: no
+    stream has work in flight once the call has returned, on which the next
+    call's arguments or the context's end could come."""
+    run("""
+    chains = [lattice(1, (12, 12, 12), 2, 2), lattice(2, (12, 12, 12), 3, 2), lattice(1, (12, 12, 12), 3, 3)]
+    params = [dict(P, seed=k) for k in range(3)]
+    on_launch(record)
+    assert len(grids(lambda: anneal_batch(chains, params))) == 3
+    assert len({l[4] for l in launches}) == 3 and fake.fake_busy() == 0
+    for which in range(3):
+        count = [0]
+        def fail(fn, grid, block, lds, stream):
+            count[0] += 1
+            return int(count[0] == which + 1)
+        on_launch(fail)
+        keep = on_launch.keep
+        try:
+            anneal_batch(chains, params)
+        except BrawlError:
+            pass
+        else:
+            raise AssertionError("no error")
+        assert fake.fake_busy() == 0, (which, fake.fake_busy())
+    on_launch(record)
+    for L in chains:
+        L.close()
+    assert fake.fake_freed_busy() == 0
+    """)
