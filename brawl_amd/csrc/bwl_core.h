@@ -44,6 +44,11 @@ struct Geo {
   int32_t shell_start[kMaxShells + 1];
 };
 
+// Draws in which a species of a walker set up on the device is complete on the
+// mean, at most, and draws that the device makes for a walker.
+constexpr double kSetupMeanDraws = 1048576.0;
+constexpr long long kSetupDraws = 64 * (long long)kSetupMeanDraws;
+
 // What initial_setup draws by: a draw (32 bits) names species s when it lies
 // in [lo, hi] (inclusive, as the cumulative bounds are; empty when lo > hi),
 // and places one of its count atoms.

@@ -185,8 +185,12 @@ int setup_rule(const Geo &g, const int64_t *species_numbers, const double *conce
 }
 
 bool setup_on_device(const Geo &g, const SetupRule &rule) {
-  for (int s = 0; s < g.S; ++s)
-    if (rule.count[s] > 0 && (rule.lo[s] > rule.hi[s] || rule.hi[s] - rule.lo[s] < 429497u)) return false;
+  for (int s = 0; s < g.S; ++s) {
+    if (rule.count[s] == 0) continue;
+    if (rule.lo[s] > rule.hi[s]) return false;
+    const double named = (double)(rule.hi[s] - rule.lo[s]) + 1.0;  // of 2^32
+    if (named < 429497.0 || (double)rule.count[s] * 4294967296.0 > kSetupMeanDraws * named) return false;
+  }
   return true;
 }
 

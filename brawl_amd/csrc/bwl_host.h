@@ -30,9 +30,12 @@ struct MT19937 {
 int setup_rule(const Geo &g, const int64_t *species_numbers, const double *concentrations, SetupRule &rule,
                std::string &err);
 // Whether the device may make the draws (bwl_setup.hip): every species with
-// atoms is named by one draw in 10^4 at least, so a walker is soon complete.
-// Others (a concentration that rounds to one atom and back to no bound, say)
-// are drawn on the host, without end if need be.
+// atoms is named by one draw in 10^4 at least, and has all of its atoms named
+// within kSetupMeanDraws draws on the mean (a species of concentration c needs
+// about the number of sites, whatever c is; one whose count is not its
+// concentration's, as when these add up to little, needs more), a 64th of what
+// the device draws for a walker at most.  Others are drawn on the host, without
+// end if need be.
 bool setup_on_device(const Geo &g, const SetupRule &rule);
 // The draws on the host: species in the order in which sites are filled.
 bool setup_order(const Geo &g, const SetupRule &rule, MT19937 &mt, int8_t *order);

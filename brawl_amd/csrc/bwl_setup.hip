@@ -29,7 +29,6 @@ namespace bwl {
 
 namespace {
 
-constexpr long long kSetupDraws = 1LL << 26;  // a walker's; its mean is at most 10^4 a species beyond the sites
 constexpr int kSetupThreads = 256;
 constexpr int kGroups = 10;        // of 64 draws in a block, the last of 48
 constexpr int kAny = kMaxSpecies;  // masks of a group: per species, of all that name one,
