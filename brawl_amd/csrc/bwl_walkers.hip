@@ -813,7 +813,8 @@ __global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *_
       // The decisions, as far at a time as the next trial that changes the
       // walker: until then every trial sees the same energy, and a ln g that
       // has grown by wl_f per trial since (as a product here, which is near
-      // enough for a decision that is clear by 1e-4; added up trial by trial
+      // enough for a decision that is clear by 1e-4 while ln g is below 1e10,
+      // where a sum of 8 rounds by less than 1e-5; added up trial by trial
       // where it is kept).
       for (;;) {
         t0 = wave_uniform(t0);
@@ -833,7 +834,8 @@ __global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *_
         // trials for the full path below: another number of draws than
         // foreseen, or a bin or a decision too close to call here
         const bool close = differ & !((fabs(x) < 1e6) & (f > 1e-6) & (f < 1.0 - 1e-6));
-        const bool full = !quick | (inw != inside) | close | (inside & !acc & !(hardly > th));
+        const bool small = fabs(lcur) + 8.0 * fabs(grow) < 1e10;
+        const bool full = !quick | !small | (inw != inside) | close | (inside & !acc & !(hardly > th));
         const unsigned long long live = (~0ull << (8 * t0)) & (nt < 8 ? (1ull << (8 * nt)) - 1ull : ~0ull);
         const unsigned long long fulls = __ballot(full) & live;
         const unsigned long long events = fulls | (__ballot(acc & inw & differ) & live);
