@@ -762,7 +762,11 @@ __global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *_
     // |e0 / range * bins| and |x| stay below 1e6: the bin is its truncation
     // unless x lies within 1e-6 of an integer (then the reference's form)
     const double slope = bmap.rinv * bmap.nb, shift = -(bmap.e0 * slope);
-    const bool quick = wave_uniform(fabs(shift) < 1e6) != 0;
+    // ... and while no ln g reaches 1e10 in this call (see below)
+    bool small = true;
+    const double grown = fabs(wl_f) * ((double)A.mc_sweeps * (double)n_atoms);
+    for (int i = lane; i < bins; i += 64) small = small && fabs(lng[i]) + grown < 1e10;
+    const bool quick = wave_uniform(fabs(shift) < 1e6) != 0 && __ballot(!small) == 0;
     int ibin = wave_uniform(wl_bin_index(e_un, A.bin_edges, bins));  // bin of e_un, kept with it
     auto in_range = [&](int b) { return b >= 1 && b <= bins; };
     auto in_window = [&](int b) { return b >= start_idx && b <= end_idx; };
@@ -813,9 +817,8 @@ __global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *_
       // The decisions, as far at a time as the next trial that changes the
       // walker: until then every trial sees the same energy, and a ln g that
       // has grown by wl_f per trial since (as a product here, which is near
-      // enough for a decision that is clear by 1e-4 while ln g is below 1e10,
-      // where a sum of 8 rounds by less than 1e-5; added up trial by trial
-      // where it is kept).
+      // enough for a decision that is clear by 1e-4: below 1e10 a sum of 8
+      // rounds by less than 1e-5; added up trial by trial where it is kept).
       for (;;) {
         t0 = wave_uniform(t0);
         nt = wave_uniform(nt);
@@ -834,8 +837,7 @@ __global__ __launch_bounds__(kSpecThreads) void k_wl_sweeps_spec(const WlArgs *_
         // trials for the full path below: another number of draws than
         // foreseen, or a bin or a decision too close to call here
         const bool close = differ & !((fabs(x) < 1e6) & (f > 1e-6) & (f < 1.0 - 1e-6));
-        const bool small = fabs(lcur) + 8.0 * fabs(grow) < 1e10;
-        const bool full = !quick | !small | (inw != inside) | close | (inside & !acc & !(hardly > th));
+        const bool full = !quick | (inw != inside) | close | (inside & !acc & !(hardly > th));
         const unsigned long long live = (~0ull << (8 * t0)) & (nt < 8 ? (1ull << (8 * nt)) - 1ull : ~0ull);
         const unsigned long long fulls = __ballot(full) & live;
         const unsigned long long events = fulls | (__ballot(acc & inw & differ) & live);
