@@ -137,7 +137,10 @@ int bwl_set_config(bwl_ctx *c, const int8_t *config) {
   size_t ref_bytes = (size_t)c->g.m[0] * c->g.m[1] * c->g.m[2];
   Pinned pin;
   const int8_t *from = c->d_ref;
-  if (ref_bytes <= kPinnedConfig) {
+  // (no block is allocated for a context's first configuration: a program that
+  // creates a context, sets its configuration and destroys it took 192 us
+  // against 162 by copy)
+  if (ref_bytes <= kPinnedConfig && (c->has_config || pinned_ready(ref_bytes))) {
     if (!pin.take(ref_bytes, c->stream)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
     memcpy(pin.p, config, ref_bytes);
     from = (const int8_t *)pin.p;

@@ -49,6 +49,13 @@ void pinned_drop() {
   for (void *p : gone) (void)hipHostFree(p);
 }
 
+bool pinned_ready(size_t bytes) {
+  Pool &P = pool();
+  std::lock_guard<std::mutex> lock(P.mu);
+  const auto it = P.kept.find(block_size(bytes));
+  return it != P.kept.end() && !it->second.empty();
+}
+
 bool Pinned::take(size_t bytes, hipStream_t stream) {
   const size_t n = block_size(bytes);
   Pool &P = pool();

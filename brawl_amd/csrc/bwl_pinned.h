@@ -24,6 +24,9 @@ constexpr size_t kPinnedKept = size_t(32) << 20;
 void pinned_hold();
 void pinned_drop();
 
+// Whether the pool holds a block for that many bytes.
+bool pinned_ready(size_t bytes);
+
 // A block of pinned memory for work on `stream`.  It goes back to the pool
 // when the object does, after the stream's work unless settled() said that
 // the work has ended.

@@ -245,7 +245,7 @@ int retire(bwl_server *s, Launch &L) {
     auto grid = [](const Request *r) { return (size_t)r->g.m[0] * r->g.m[1] * r->g.m[2]; };
     for (size_t i = 0; i < n && status == BWL_OK;) {
       size_t bytes = 0, end = i;
-      while (end < n && (end == i || bytes + grid(L.reqs[end]) <= kPinnedConfig)) {
+      while (end < n && (end == i || bytes + grid(L.reqs[end]) <= kPinnedServed)) {
         if (L.reqs[end]->config_out) bytes += grid(L.reqs[end]);
         ++end;
       }
@@ -344,7 +344,7 @@ int retire(bwl_server *s, Launch &L) {
 int stage_request(Request *r, hipStream_t st) {
   const size_t cb = ctx_device_bytes(r->desc), tables = al(ctx_tables_bytes(r->g));
   const size_t ref = (size_t)r->g.m[0] * r->g.m[1] * r->g.m[2];
-  const bool anneal = r->kind == KIND_ANNEAL, pinned = anneal && ref <= kPinnedConfig;
+  const bool anneal = r->kind == KIND_ANNEAL, pinned = anneal && ref <= kPinnedServed;
   r->up = std::make_unique<Pinned>();
   if (!r->up->take(tables + (pinned ? ref : 0), st)) return fail(BWL_ERR_NOMEM, "pinned memory allocation failed");
   int rc = ctx_create_borrowed(r->desc, r->vex.data(), r->block, cb, st, r->up->p, &r->ctx);

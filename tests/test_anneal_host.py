@@ -133,3 +133,28 @@ def test_error_exits_wait_for_what_was_queued(run):
         L.close()
     assert fake.fake_freed_busy() == 0
     """)
+
+
+def test_pinned_blocks_of_a_context(run):
+    """A context that takes one configuration, or large ones only, makes no
+    pinned block; the blocks that it makes go with the last context."""
+    run("""
+    v = np.zeros((2, 2, 1))
+    def cfg(n):
+        return workloads.random_config(1, n, workloads.equal_counts(4 * n[0] * n[1] * n[2], 2), np.random.default_rng(1))
+    small, large = (8, 8, 8), (60, 60, 60)
+    for n, calls in ((small, 1), (large, 3)):
+        with Lattice(1, n, v) as L:
+            for _ in range(calls):
+                L.set_config(cfg(n))
+            if n is large:
+                L.get_config()
+            assert fake.fake_pinned_made() == 0
+    with Lattice(1, small, v) as L, Lattice(1, small, v) as M:
+        for _ in range(3):
+            L.set_config(cfg(small))
+            M.set_config(cfg(small))
+            L.get_config()
+        assert fake.fake_pinned_made() == fake.fake_pinned_held() == 1
+    assert fake.fake_pinned_held() == 0
+    """)
