@@ -106,7 +106,7 @@ struct SetupArgs {
   int32_t *status;        // out: 1 when a walker took too many draws (not written if made)
 };
 
-// Nested sampling (nested_sampling.f90:45-206), one wavefront per run.
+// Nested sampling (nested_sampling.f90:45-206), one workgroup per run.
 struct NsArgs {
   Geo g;
   const int32_t *off;
@@ -197,8 +197,10 @@ hipError_t launch_setup(const SetupArgs *args_dev, int n, int max_walkers, int m
 hipError_t launch_unpack(const int8_t *compact, int8_t *ref, const Geo &g, hipStream_t s);
 // LDS read-bandwidth probe: blocks x 1024 threads, iters 16-byte reads each
 hipError_t launch_lds_bandwidth(int blocks, int iters, uint32_t *sink, hipStream_t s);
-// LDS of a lattice held whole beside its tables: larger ones are refused by
-// the calls that measure a configuration
+// hist_lds_bytes, site_lds_bytes: LDS of a lattice held whole beside its
+// tables.  The calls that measure a configuration refuse larger ones, though
+// their kernels hold a few planes or nothing of it: what a lattice may be is
+// the same for all calls that need its energy.
 size_t hist_lds_bytes(const Geo &g, int threads);
 int hist_blocks(const Geo &g);
 hipError_t launch_histogram(const HistArgs &a, int blocks, hipStream_t s);

@@ -2,11 +2,13 @@
 //
 //   k_pack / k_unpack      reference doubled-grid layout <-> compact
 //                          per-sublattice layout (HBM)
-//   k_histogram            integer pair-count histogram, one workgroup per
-//                          lattice, lattice staged whole in LDS
+//   k_histogram            integer pair-count histogram, a part of one plane
+//                          of cells per workgroup
 //   k_site_energy          one site's energy in the reference's FP64 order
 //   k_metro_seq            bit-exact sequential Metropolis driven by the
-//                          reference's MT19937 stream (one wavefront)
+//                          reference's MT19937 stream: one trial at a time in
+//                          one wavefront, or in speculative batches in a
+//                          workgroup (k_metro_seq_spec); _batch: many chains
 // (the parallel Metropolis sampler is in bwl_metro_kernels.h)
 #include <hip/hip_runtime.h>
 

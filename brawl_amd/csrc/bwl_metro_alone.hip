@@ -33,6 +33,8 @@ const void *alone_of(int words) {
 
 const void *par_alone_kernel(const Geo &g, bool fixed) {
   const int words = par_count_words(g, true);
+  // the shape with its own pitch has no other layout in lattice coordinates;
+  // 400 sweeps of fcc 8^3 take 23.0 ms so, 24.6 at the fixed pitch
   if (!fixed)
     return words == 0 && g.lattice == 1 && g.R == 2 && g.n[0] == 8 ? (const void *)k_metro_alone<1, 2, uint32_t, 8, 8>
                                                                   : nullptr;

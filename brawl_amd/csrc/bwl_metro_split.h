@@ -543,8 +543,7 @@ __device__ __forceinline__ void metro_split(const ParArgs &C, const int part, ui
       for (int i = tid; i < S * S * R; i += n_threads) hacc[i] = 0ull;
     } else {
       // every part's to the first
-    __syncthreads();
-    {
+      __syncthreads();
       unsigned long long v = acc_local;
 #pragma unroll
       for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
@@ -590,7 +589,6 @@ __device__ __forceinline__ void metro_split(const ParArgs &C, const int part, ui
         __syncthreads();
         for (int i = tid; i < S * S * R; i += kSplitThreads) hacc[i] = 0ull;
       }
-    }
     }
     const double Er = recount();
     if (part == 0 && tid == 0) {

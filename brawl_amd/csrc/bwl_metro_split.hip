@@ -34,10 +34,11 @@
 // site of pair i, lane i + 32 its grid-2 site.
 //
 // The parts wait for each other, so all of a chain's parts have to be on the
-// device at once: the host asks for no more parts than there are CUs (over
-// all calls in flight), every wait ends after a time (the chain is then given
-// up, its configuration untouched, and the host runs it undivided), and parts
-// of one chain get block indices that fall on one XCD.
+// device at once: the host asks for no more parts than this process's calls in
+// flight leave CUs, every wait ends after a time, that for the parts' arrival
+// soonest (the chain is then given up, its configuration untouched, and the
+// host runs it undivided), and parts of one chain get block indices that fall
+// on one XCD.
 #include "bwl_metro_split.h"
 
 namespace bwl {
@@ -92,7 +93,8 @@ hipError_t launch_metro_split(const void *fn, const ParArgs *args_dev, const int
 const void *par_split_kernel(const Geo &g, bool fixed) {
   const int words = par_count_words(g, true);
   if (!fixed) {
-    // the shape with a kernel of its own that has rounds worth dividing
+    // the shape with its own pitch that has rounds worth dividing: 200 sweeps
+    // of bcc 32^3 in 16 parts 19.7 ms so, 21.4 at the fixed pitch
     return words == 0 && g.lattice == 2 && g.R == 4 && g.n[0] == 32
                ? (const void *)k_metro_split<2, 4, uint32_t, 32, 8>
                : nullptr;

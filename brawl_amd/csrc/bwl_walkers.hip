@@ -2,12 +2,14 @@
 // Wang-Landau walker sweeps and window entry, and the windowed pair-count
 // histogram behind the radial densities.
 //
-// Each nested-sampling run and each Wang-Landau walker is one wavefront
+// Each nested-sampling run and each Wang-Landau walker is one workgroup
 // that consumes its own MT19937 stream exactly as the reference's serial
 // code does (one MPI rank per walker there), with site and pair energies in
 // the reference's FP64 order, so every walker's trajectory is bit-identical
-// to the reference's.  Throughput comes from running many walkers (one per
-// CU) in one launch.
+// to the reference's: four wavefronts that take trials in speculative batches
+// (k_ns_spec, k_wl_sweeps_spec; see bwl_spec.h), or, where spec_pays says so
+// and for window entry, one wavefront and one trial at a time.  Throughput
+// comes from running many walkers in one launch.
 #include <hip/hip_runtime.h>
 
 #include "bwl_kernels.h"

@@ -2,7 +2,7 @@
 
 `nested_sampling` runs the reference's serial loop for one chain on the
 device; `nested_sampling_batch` runs many independent chains (requests) in
-one launch, one wavefront each.  Each run consumes its lattice's MT19937
+one launch, one workgroup each.  Each run consumes its lattice's MT19937
 stream exactly as the reference does, so its energy limits are the
 reference's for the same stream, alone or in a batch.
 """

@@ -132,7 +132,7 @@ int bwl_mc_steps(bwl_ctx *ctx, double beta, int32_t nbr_swap, int64_t n_trials,
                  int64_t sample_every, double *energies, int64_t *accepted);
 /* Batched form of bwl_mc_steps: n contexts on one device, each making
  * n_trials sequential trials at beta[i] on its own MT19937 stream, in one
- * launch (one wavefront per context) -- the reference's MPI replica
+ * launch (one workgroup per context) -- the reference's MPI replica
  * ensemble (comms.F90:122-160, one chain per rank), every chain
  * bit-identical to the same context's bwl_mc_steps.  accepted (n values),
  * energies (optional: n pointers of n_trials/sample_every values, NULL
@@ -302,7 +302,7 @@ typedef struct {
  * walk moves. */
 int bwl_nested_sampling(bwl_ctx *ctx, const bwl_ns_params *p, const int64_t *species_numbers,
                         const double *concentrations, double *e_limits, bwl_run_stats *stats);
-/* n independent runs (one wavefront each, each on its own context and
+/* n independent runs (one workgroup each, each on its own context and
  * stream of random numbers) in one launch; each run's result is the same
  * as alone.  species_numbers[i] / concentrations[i] may be NULL as for
  * bwl_initial_setup. */
