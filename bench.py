@@ -27,6 +27,7 @@ Prints ONE JSON line.  With --gpus N > 1 it exits: the library runs on one GPU.
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -53,13 +54,21 @@ def bytes_per_trial(z: int) -> int:
     return 2 * (z + 1) + 2
 
 
-# HBM bytes per launch of the plain anneal kernel, from rocprofv3 --pmc
-# FETCH_SIZE (106.125 KiB, x2.0 copy-kernel scale) and WRITE_SIZE
-# (221.25 KiB, x1.0): the lattice is read once into LDS and written back
+# The plain anneal's kernel, divided over workgroups or in one, and its HBM
+# bytes per launch, from rocprofv3 --pmc FETCH_SIZE (x2.0 copy-kernel scale) and
+# WRITE_SIZE (x1.0).  In one: the lattice is read once into LDS and written back
 # once, plus the per-T-step outputs and the register spills of the
-# radial-density reduction.
-TRAFFIC_BYTES = int(round((106.125 * 2.0 + 221.25) * 1024))
-PLAIN_KERNEL = "k_metro_nat<bcc, R=4, 32-bit counts, 32 cells>"
+# radial-density reduction.  Divided: each part reads the lattice, and the parts'
+# accepted swaps pass through their XCD's L2, which writes some of them back.
+PLAIN_KERNELS = {
+    True: ("k_metro_split<bcc, R=4, 32-bit counts, 32 cells>", int(round((1648.4375 * 2.0 + 9111.65625) * 1024)),
+           "a round's chain of steps on the workgroups of one XCD that hold the chain: evaluation "
+           "from LDS, the exchange of accepted swaps through L2, making them (HBM carries only "
+           "the load, the write-back and part of the exchange, 'traffic')"),
+    False: ("k_metro_nat<bcc, R=4, 32-bit counts, 32 cells>", int(round((106.125 * 2.0 + 221.25) * 1024)),
+            "VALU and LDS instruction issue of the one CU that holds the chain (the lattice is "
+            "resident in LDS; HBM carries only the load and the write-back, 'traffic')"),
+}
 # radial densities (alpha^(1..4)) sampled every 10 sweeps of each T step
 ASRO_EVERY = 10
 
@@ -375,17 +384,17 @@ def batched(steps: int, warmup: int, tune: bool = True):
     return out
 
 
-def lds_roofline(plain_gbs: float, batched_out=None):
+def lds_roofline(plain_gbs: float, plain_cus: int, batched_out=None):
     """The samplers' lattices live in LDS: their algorithmic bytes against
-    the LDS read bandwidth measured by the library's probe (all CUs, and one
-    CU's share for the one-chain plain form)."""
+    the LDS read bandwidth measured by the library's probe (all CUs, and those
+    of the one-chain plain form)."""
     from brawl_amd import _lib
     bps, cus = _lib.lds_bandwidth()
     peak = bps / 1e9
     out = {"bound": "lds", "unit": "GB/s", "peak": peak, "cus": cus, "peak_per_cu": peak / cus,
            "probe": "conflict-free 16-byte LDS reads, 8 blocks x 1024 threads per CU",
            "plain_achieved": plain_gbs, "plain_frac": plain_gbs / peak,
-           "plain_frac_of_one_cu": plain_gbs / (peak / cus)}
+           "plain_cus": plain_cus, "plain_frac_of_its_cus": plain_gbs / (peak / cus * plain_cus)}
     if batched_out:
         a = batched_out["bytes_per_step"] / (batched_out["makespan_ms"] / 1e3) / 1e9
         out["batched_achieved"] = a
@@ -844,6 +853,10 @@ def main():
     achieved = trials_per_launch * bpt / avg_kernel_s / 1e9
     peak = 8000.0
     last = results[-1]
+    ran = (ctypes.c_int32 * 3)()
+    lat._L.bwl_test_anneal_ran(lat._h, ran)
+    plain_cus = max(1, int(ran[0]))
+    plain_kernel, traffic, limited_by = PLAIN_KERNELS[plain_cus > 1]
     out = {
         "metric": "swap trials/s on 1 MI355X (plain vs batched-served); p50/p99 run latency",
         "value": value,
@@ -863,13 +876,11 @@ def main():
                    "form": "plain (one chain per call)", "trials_per_step": trials_per_launch,
                    "bytes_per_trial": bpt},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": peak, "unit": "GB/s",
-                     "frac": achieved / peak, "traffic": TRAFFIC_BYTES,
-                     "kernel": PLAIN_KERNEL, "kernel_ms": float(np.mean(kernel_ms)),
+                     "frac": achieved / peak, "traffic": traffic,
+                     "kernel": plain_kernel, "workgroups": plain_cus, "kernel_ms": float(np.mean(kernel_ms)),
                      "bytes_per_launch": trials_per_launch * bpt,
-                     "limited_by": "VALU and LDS instruction issue of the one CU that holds the "
-                                   "chain (the lattice is resident in LDS; HBM carries only "
-                                   "the load and the write-back, 'traffic')",
-                     "frac_of_one_cu_lds": None},
+                     "limited_by": limited_by,
+                     "frac_of_its_cus_lds": None},
         "results": {"E_per_atom_first_T": float(last.energies_of_T[0]),
                     "E_per_atom_last_T": float(last.energies_of_T[-1]),
                     "C_max": float(np.max(last.C_of_T)),
@@ -893,8 +904,8 @@ def main():
         out["wang_landau_walkers"] = wang_landau_walkers()
         out["nested_sampling_runs"] = nested_sampling_runs()
         out["sequential_bit_exact"] = sequential_bit_exact()
-    out["roofline_lds"] = lds_roofline(achieved, out.get("batched"))
-    out["roofline"]["frac_of_one_cu_lds"] = out["roofline_lds"]["plain_frac_of_one_cu"]
+    out["roofline_lds"] = lds_roofline(achieved, plain_cus, out.get("batched"))
+    out["roofline"]["frac_of_its_cus_lds"] = out["roofline_lds"]["plain_frac_of_its_cus"]
     out["cpu_baseline"] = cpu
     print(json.dumps(out))
 

@@ -203,8 +203,8 @@ struct DevBuf {
 
 }  // namespace bwl
 
-// For the tests, which have no other way to see or to force it (not part of
-// include/brawl_hip.h): bwl_ctx::ran, and bwl_ctx::give_up.
+// bwl_ctx::ran, for the tests and the benchmark's labels, and bwl_ctx::give_up,
+// for the tests (neither is part of include/brawl_hip.h).
 extern "C" {
 int bwl_test_anneal_ran(const bwl_ctx *c, int32_t *ran3);
 int bwl_test_give_up(bwl_ctx *c, int32_t on);

@@ -276,19 +276,19 @@ __device__ __forceinline__ void metro_seq_run(const SeqArgs &A, uint8_t *smem) {
 // two, and a batch costs 1.2 to 3 trials taken one by one (64 places' energies
 // in place of one's).  So while batches come out shorter than that, trials are
 // taken singly, both sites' neighbours over the lanes and each shell's sum in
-// a lane of its own, and a batch is tried again every kSingly of them.
+// a lane of its own, and a batch is tried again every kSingly of them (SINGLY:
+// boxes large enough have a kernel without, see BWL_KERNEL_SINGLY).
 //
 // A batch takes, one to four shells, 0.8, 1.6, 2.0 and 2.6 us on fcc (0.7,
 // 1.2, 1.6 and 3.1 on bcc), a single trial 0.9, 0.9, 1.2 and 1.2 (0.8, 0.8, 1.0
 // and 1.2).  20,000 trials at 10^6 K (nothing rejected) of fcc 3^3 with four
 // shells: 61.5 ms in batches, 24.1 so (26.7 by k_metro_seq); of bcc 4^3 with
-// three 31.9 -> 19.6 (21.0); fcc 8^3 with two at 2000 K, where no batch is that
-// short, 0.387 -> 0.394 us a trial.
+// three 31.9 -> 19.6 (21.0).
 // ------------------------------------------------------------------
 constexpr int kSingly = 16;
 // 8 times the mean length of a batch that is as fast as single trials
 template <int KEY>
-constexpr uint32_t kBatchPays = KEY % 16 == 1 ? 0 : KEY % 16 == 4 ? 24 : 17;
+constexpr uint32_t kBatchPays = KEY % 16 == 4 ? 24 : 17;
 
 template <int KEY>
 struct SingleDims {
@@ -365,7 +365,7 @@ __device__ __forceinline__ double single_delta(const SpecLds &L, const SeqGeo &g
   return (e[2] + e[3]) - (e[0] + e[1]);
 }
 
-template <int KEY>
+template <int KEY, bool SINGLY>
 __device__ __forceinline__ void metro_seq_spec_run(const SeqArgs &A, uint8_t *smem) {
   using D = SpecDims<KEY>;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -386,12 +386,15 @@ __device__ __forceinline__ void metro_seq_spec_run(const SeqArgs &A, uint8_t *sm
   volatile int32_t *cmd = (volatile int32_t *)take(16);
   double *vex = (double *)take(sizeof(double) * S * S * D::R);
   double *ebuf = (double *)take(sizeof(double) * 2 * kEnergyChunk);
-  double *sums = (double *)take(SingleDims<KEY>::kBytes);
+  double *sums = nullptr;
+  if constexpr (SINGLY) {
+    sums = (double *)take(SingleDims<KEY>::kBytes);
+    for (int i = tid; i < SingleDims<KEY>::kBytes / 8; i += kSpecThreads) sums[i] = 0.0;
+  }
   int32_t *offp = (int32_t *)take(4 * D::NSUB * D::R * D::ML);
   uint8_t *adj = take(D::TS * D::TS * D::TS);
   for (int i = tid; i < 624; i += kSpecThreads) raw[i] = A.mt[i];
   for (int i = tid; i < S * S * D::R; i += kSpecThreads) vex[i] = A.vex[i];
-  for (int i = tid; i < SingleDims<KEY>::kBytes / 8; i += kSpecThreads) sums[i] = 0.0;
   stage_spec_tables<KEY>(offp, adj, A.off);
   stage_codes(lat, A.compact, g, D::NSUB, S);
   __syncthreads();
@@ -423,7 +426,7 @@ __device__ __forceinline__ void metro_seq_spec_run(const SeqArgs &A, uint8_t *sm
       }
     };
     while (left > 0) {
-      if (length < kBatchPays<KEY>) {
+      if (SINGLY && length < kBatchPays<KEY>) {
         SingleLane<KEY> sl;
         sl.init(S);
         for (int k = 0; k < kSingly && left > 0; ++k) {
@@ -496,7 +499,7 @@ __device__ __forceinline__ void metro_seq_spec_run(const SeqArgs &A, uint8_t *sm
       conf |= conf >> 16;
       conf |= conf >> 8;
       if (conf & 0xffu) n = __ffs((int)(conf & 0xffu)) - 1;
-      length = (uint32_t)wave_uniform((int)(length - length / 8 + n));
+      if constexpr (SINGLY) length = (uint32_t)wave_uniform((int)(length - length / 8 + n));
       n = n < left ? n : (int)left;
       if (sampling && n > to_sample) n = (int)to_sample;
       const unsigned long long upto = n < kBatch ? (1ull << (8 * n)) - 1ull : ~0ull;
@@ -636,24 +639,61 @@ size_t seq_lds_bytes(const Geo &g) {
 template <int KEY>
 __global__ __launch_bounds__(kSpecThreads) void k_metro_seq_spec(SeqArgs A) {
   extern __shared__ __align__(16) uint8_t smem[];
-  metro_seq_spec_run<KEY>(A, smem);
+  metro_seq_spec_run<KEY, false>(A, smem);
 }
 
 template <int KEY>
 __global__ __launch_bounds__(kSpecThreads) void k_metro_seq_spec_batch(const SeqArgs *__restrict__ args) {
   extern __shared__ __align__(16) uint8_t smem[];
-  metro_seq_spec_run<KEY>(args[blockIdx.x], smem);
+  metro_seq_spec_run<KEY, false>(args[blockIdx.x], smem);
+}
+
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_metro_seq_singly(SeqArgs A) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  metro_seq_spec_run<KEY, true>(A, smem);
+}
+
+template <int KEY>
+__global__ __launch_bounds__(kSpecThreads) void k_metro_seq_singly_batch(const SeqArgs *__restrict__ args) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  metro_seq_spec_run<KEY, true>(args[blockIdx.x], smem);
 }
 
 namespace {
 const void *metro_seq_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_metro_seq, key) }
 const void *metro_seq_batch_kernel(int key) { BWL_KERNEL_FOR_PAIR_SUM_KEY(k_metro_seq_batch, key) }
-const void *metro_seq_spec_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec, key) }
-const void *metro_seq_spec_batch_kernel(int key) { BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec_batch, key) }
+// The kernel of template family `kern` that can take trials singly, nullptr if
+// none is needed.  It takes 0 to 4 % longer where it does not (fcc 8^3, two
+// shells, 8192 trials 2.08 ms -> 2.15), so boxes that are large enough for
+// batches to be as fast with nothing rejected have one without: against one
+// trial at a time 1.4x and 1.5x on fcc and bcc 6^3 with two shells (reach
+// 0.29), 1.4x on fcc 8^3 with three (0.12; 0.95x on 6^3), 1.18x on fcc 8^3 with
+// four and 1.02x on bcc 10^3 (0.17; 0.80x on 8^3).
+#define BWL_KERNEL_SINGLY(kern, pick)                          \
+  if (pick.reach > (pick.key % 16 == 2 ? 0.3 : 0.18)) {        \
+    switch (pick.key) {                                        \
+      case 16 + 2: return (const void *)kern<16 + 2>;          \
+      case 16 + 3: return (const void *)kern<16 + 3>;          \
+      case 16 + 4: return (const void *)kern<16 + 4>;          \
+      case 32 + 2: return (const void *)kern<32 + 2>;          \
+      case 32 + 3: return (const void *)kern<32 + 3>;          \
+      case 32 + 4: return (const void *)kern<32 + 4>;          \
+    }                                                          \
+  }
+const void *metro_seq_spec_kernel(const SeqPick &pick) {
+  BWL_KERNEL_SINGLY(k_metro_seq_singly, pick)
+  BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec, pick.key)
+}
+const void *metro_seq_spec_batch_kernel(const SeqPick &pick) {
+  BWL_KERNEL_SINGLY(k_metro_seq_singly_batch, pick)
+  BWL_KERNEL_FOR_SPEC_KEY(k_metro_seq_spec_batch, pick.key)
+}
 }  // namespace
 
 size_t seq_spec_lds_bytes(const Geo &g) {
-  const size_t sums = 8 * 4 * (size_t)g.R * (shell_max(g.lattice, g.R) | 1);  // SingleDims::kBytes
+  // SingleDims::kBytes, whether the launch's kernel uses them or not
+  const size_t sums = 8 * 4 * (size_t)g.R * (shell_max(g.lattice, g.R) | 1);
   return spec_table_bytes(g) + spec_ring_bytes() + spec_energy_bytes() + spec_align(sums);
 }
 
@@ -674,13 +714,13 @@ bool spec_pays(const void *fn, int n, const SeqPick &pick, double far) {
 hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s) {
   SeqArgs arg = a;
   void *kargs[] = {(void *)&arg};
-  if (pick.spec) return launch_dynamic(metro_seq_spec_kernel(pick.key), dim3(1), kSpecThreads, kargs, pick.lds_spec, s);
+  if (pick.spec) return launch_dynamic(metro_seq_spec_kernel(pick), dim3(1), kSpecThreads, kargs, pick.lds_spec, s);
   return launch_dynamic(metro_seq_kernel(pick.key), dim3(1), 64, kargs, pick.lds, s);
 }
 
 hipError_t launch_metro_seq_batch(const SeqArgs *args_dev, int n, const SeqPick &pick, hipStream_t s) {
   void *kargs[] = {(void *)&args_dev};
-  const void *fn = pick.spec ? metro_seq_spec_batch_kernel(pick.key) : nullptr;
+  const void *fn = pick.spec ? metro_seq_spec_batch_kernel(pick) : nullptr;
   // (a batch here is 64 places' energies: the more shells, the sooner too much)
   if (spec_pays(fn, n, pick, pick.key % 16 <= 2 ? 0.05 : 0.0))
     return launch_dynamic(fn, dim3(n), kSpecThreads, kargs, pick.lds_spec, s);
