@@ -261,6 +261,14 @@ inline hipError_t launch_dynamic(const void *fn, dim3 grid, int threads, void **
 
 size_t seq_lds_bytes(const Geo &g);
 size_t seq_spec_lds_bytes(const Geo &g);
+// The kernel of speculative batches that can take trials singly, for one chain
+// or a batch, nullptr where none is needed.  It takes 0 to 4 % longer where it
+// does not take them (fcc 8^3, two shells, 8192 trials 2.08 ms -> 2.15), so
+// boxes that are large enough for batches to be as fast with nothing rejected
+// do without: against one trial at a time 1.4x and 1.5x on fcc and bcc 6^3 with
+// two shells (reach 0.29), 1.4x on fcc 8^3 with three (0.12; 0.95x on 6^3),
+// 1.18x on fcc 8^3 with four and 1.02x on bcc 10^3 (0.17; 0.80x on 8^3).
+const void *metro_seq_singly_kernel(const SeqPick &pick, bool batch);
 hipError_t launch_metro_seq(const SeqArgs &a, const SeqPick &pick, hipStream_t s);
 hipError_t launch_draw_sites(const DrawArgs &a, hipStream_t s);
 // n chains (args_dev[0..n)), one workgroup each
