@@ -698,12 +698,23 @@ static double divided_us(const AnnealPlan::Item &it) { return it.rounds * 2.4; }
 // Divides the longest chains over workgroups (a.parts, lane of their items)
 // where the device would end the whole batch sooner than such a chain alone.
 //
-// A chain is worth dividing from chunks * z = 192 on: 1.16x at 216 (fcc 16^3,
-// 4 shells), 1.27x at 196 (bcc 24^3, 2), 1.67x at 588 (fcc 24^3, 3), 2.1x at
-// 1200 (bcc 32^3, 4), against 0.99x at 144 (fcc 20^3, 2) and 1.00x at 150
-// (bcc 16^3, 4).  One wavefront per SIMD and part (4 half rows) is best where
-// the CUs are there (bcc 32^3: 16 parts 5.1 ms, 8 parts 5.7; fcc 24^3: 7
-// parts 7.4, 4 parts 7.7), else two.
+// A chain is worth dividing from chunks * z = 192 on: 1.10x at 252 (fcc 18^3, 3
+// shells), 1.19x at 196 (bcc 24^3, 2), 1.6x at 588 (fcc 24^3, 3), 2.0x at 1200
+// (bcc 32^3, 4), against 0.99x at 144 (fcc 20^3, 2) and 1.00x at 150 (bcc 16^3,
+// 4).  Two kinds of chains from there on are not: those that k_metro_alone
+// takes whole (fcc 15^3 to 17^3 and bcc 18^3, 4 shells, in 2 parts: 0.77-0.97x,
+// 1.01x at best), and, with 64-bit count words, whose pairs cost more, chains of
+// less than 8 chunks unless z makes up for it (fcc 18^3, 3 shells, 0.95x; bcc
+// 19^3, 4 shells, 0.89x; fcc 20^3, 3 shells, 1.07x; fcc 18^3, 4 shells, 1.26x).
+// One wavefront per SIMD and part (4 half rows) is best where the CUs are there
+// (bcc 32^3: 16 parts 5.1 ms, 8 parts 5.7; fcc 24^3: 7 parts 7.4, 4 parts 7.7),
+// else two.
+//
+// With more than one shell that holds from the first sweep on, since the
+// recounts of the energy are divided too.  With one shell they are short, and
+// 16 wavefronts stage the lattice in 40 to 60 us less than the 8 of a part: fcc
+// 16^3 196 us for one sweep (divided 223) and 596 for twelve (533), bcc 18^3
+// 183 (211) and 447 (373), so such a chain has to be some 6 sweeps long.
 //
 // The parts of a chain go to one XCD (lane), which has n_cu / 8 CUs: as many
 // as this process's calls in flight (CuUse, SplitShare) and the call's other
@@ -739,6 +750,9 @@ static void divide_chains(AnnealPlan &P, const SplitLanes &free_parts, int n_cu,
   });
   auto divide = [&](AnnealPlan::Item &it) {
     if (!it.split_fn || it.chunks * it.a.g.z < 192 || par_split_lds_bytes(it.a.g, it.a.nat) > (size_t)lim) return false;
+    if (par_alone_kernel(it.a.g, it.split_fixed) && par_alone_threads(it.threads, it.passes) > 0) return false;
+    if (par_count_words(it.a.g, true) == 2 && it.chunks < 8 && it.chunks * it.a.g.z < 320) return false;
+    if (it.a.g.R == 1 && undivided_us(it) < 160.0) return false;
     const int rows = it.threads / 64;
     for (int units = 4; units <= 8; units += 4) {
       const int rows_each = std::max(1, units / (2 * it.passes));
@@ -822,7 +836,8 @@ int anneal_plan(int n, bwl_ctx *const *ctxs, const bwl_anneal_params *params, An
     it.rounds = (double)p->T_steps * (double)(p->n_sweeps + p->burn_in_sweeps) * (double)g.n_atoms / (double)max_pairs;
     // (a layout other than the rule's, where the caller asked for one, has
     // run-time neighbour offsets or none in lattice coordinates)
-    if (natural) it.split_fn = par_split_kernel(g, it.fn == par_fixed_kernel(g.lattice, g.R, par_count_words(g, true)));
+    it.split_fixed = natural && it.fn == par_fixed_kernel(g.lattice, g.R, par_count_words(g, true));
+    if (natural) it.split_fn = par_split_kernel(g, it.split_fixed);
     if (natural && it.split_fn && it.fn != par_fixed_kernel(g.lattice, g.R, par_count_words(g, true)) && !par_specialised(g))
       it.split_fn = nullptr;
     ParArgs &a = it.a;

@@ -143,6 +143,7 @@ struct AnnealPlan {
     size_t off_mail = 0, mail_n = 0;  // mailbox of a divided chain, in words
     const void *split_fn = nullptr;   // kernel that can divide the chain, if any
     bool natural = false;             // held in lattice coordinates
+    bool split_fixed = false;         // ... at the fixed pitch
     bool alone = false;               // runs k_metro_alone
     int chunks = 0, passes = 0;       // most pairs of a round, in 64s and per thread
     int lane = 0;                     // XCD of a divided chain's parts

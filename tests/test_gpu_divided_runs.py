@@ -49,7 +49,8 @@ def _same(a, b, A, B):
     assert np.array_equal(A.get_config(), B.get_config())
 
 
-@pytest.mark.parametrize("lat,n,S,R,parts", [(2, (32, 32, 32), 4, 4, 16), (1, (24, 24, 24), 2, 3, 7), (1, (16, 16, 16), 7, 4, 2)])
+@pytest.mark.parametrize("lat,n,S,R,parts", [(2, (32, 32, 32), 4, 4, 16), (1, (24, 24, 24), 2, 3, 7), (1, (18, 18, 18), 7, 4, 3),
+                                             (1, (19, 19, 19), 5, 3, 4)])
 def test_divided_and_made_good(lib, lat, n, S, R, parts):
     """Whole, given up on arrival, and whole again from where that left off."""
     print("case", lat, n, S, R, flush=True)
@@ -81,7 +82,7 @@ def test_given_up_in_a_batch(lib):
 
 
 @pytest.mark.parametrize("lat,n,S,R,chains,divided", [(2, (30, 30, 30), 3, 2, 9, 9), (1, (22, 22, 22), 4, 3, 26, 26),
-                                                      (1, (16, 16, 16), 4, 4, 40, 40)])
+                                                      (1, (18, 18, 18), 4, 4, 40, 40)])
 def test_batch_is_divided(lib, lat, n, S, R, chains, divided):
     """Every chain of the batches that are compared with undivided ones."""
     from brawl_amd import anneal_batch
@@ -95,22 +96,22 @@ def test_batch_is_divided(lib, lat, n, S, R, chains, divided):
 
 
 def test_more_rounds_than_tags(lib):
-    """Rounds (of at most 256 pairs) beyond 65,536: records are cleared at 32768
+    """Rounds (of at most 384 pairs) beyond 65,536: records are cleared at 32768
     and their tags come around at 65536; three temperature steps use the first
     one's slot again."""
-    A, B = _lattice(1, (16, 16, 16), 3, 4), _lattice(1, (16, 16, 16), 3, 4)
+    A, B = _lattice(1, (18, 18, 18), 3, 3), _lattice(1, (18, 18, 18), 3, 3)
     with A, B:
-        p = dict(T=1200.0, delta_T=-300.0, T_steps=3, n_sweeps=340, burn_in_sweeps=10, seed=5, asro_every=7)
+        p = dict(T=1200.0, delta_T=-300.0, T_steps=3, n_sweeps=360, burn_in_sweeps=10, seed=5, asro_every=7)
         a = A.metropolis_simulated_annealing(**p)
         assert _ran(lib, A)[0] > 1 and _ran(lib, A)[1] == 0
         _give_up(lib, B, True)
         b = B.metropolis_simulated_annealing(**p)
         assert _ran(lib, B)[:2] == [1, 1]
-        assert a.trials > 256 * 65536
+        assert a.trials > 384 * 65536
         _same(a, b, A, B)
 
 
-@pytest.mark.parametrize("lat,n,S,R,every", [(2, (24, 24, 24), 3, 4, 2), (1, (16, 16, 16), 5, 4, 3), (2, (30, 30, 30), 6, 2, 1)])
+@pytest.mark.parametrize("lat,n,S,R,every", [(2, (24, 24, 24), 3, 4, 2), (1, (18, 18, 18), 5, 3, 3), (2, (30, 30, 30), 6, 2, 1)])
 def test_radial_densities_of_several_samples(lib, lat, n, S, R, every):
     A, B = _lattice(lat, n, S, R), _lattice(lat, n, S, R)
     with A, B:
@@ -131,3 +132,16 @@ def test_which_small_chains_run_one_site_per_lane(lib):
         assert _ran(lib, small) == [1, 0, 1]
         anneal_batch([small, big], [p, dict(p, seed=2)])
         assert _ran(lib, small)[2] == 0 and _ran(lib, big)[2] == 0
+
+
+@pytest.mark.parametrize("lat,n,S,R,sweeps,divided", [
+    (1, 17, 3, 4, 40, False), (1, 18, 3, 4, 40, True),      # small enough for one site per lane in one workgroup
+    (1, 19, 7, 3, 40, False), (1, 20, 7, 3, 40, True),      # 64-bit counts
+    (2, 19, 6, 4, 40, False), (1, 18, 6, 4, 40, True),
+    (2, 18, 2, 1, 2, False), (2, 18, 2, 1, 40, True),       # one shell: short runs are not
+])
+def test_which_chains_are_divided(lib, lat, n, S, R, sweeps, divided):
+    """Each side of the rule's lines."""
+    with _lattice(lat, (n, n, n), S, R) as L:
+        L.metropolis_simulated_annealing(T=900.0, n_sweeps=sweeps, seed=1)
+        assert (_ran(lib, L)[0] > 1) == divided and _ran(lib, L)[1] == 0
