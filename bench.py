@@ -267,7 +267,7 @@ def cpu_walkers(budget_s: float):
 
 def nested_sampling_runs(n_runs: int = 64, n_iter: int = 200, fill_runs: int = 256):
     """Nested-sampling runs of the served stream's NS shape on the device:
-    one run alone (one wavefront), then n_runs runs (their own seeds) in
+    one run alone (one workgroup), then n_runs runs (their own seeds) in
     one batched launch, then fill_runs runs (one per CU of the MI355X)."""
     from brawl_amd import Lattice, nested_sampling
     q, walkers = ns_request_shape()
@@ -342,21 +342,22 @@ def batched(steps: int, warmup: int, tune: bool = True):
            "value": float(np.mean(rates)), "unit": "swap trials/s",
            "device_rate": trials / (np.mean(mks) / 1e3), "makespan_ms": float(np.mean(mks)),
            "bytes_per_step": int(alg_bytes)}
-    # the CUs' busy share over the makespan: each chain run alone from its
-    # start (the same trajectory as in the batch, bit for bit) for its own
-    # device time, summed, against every CU for the batch's makespan
+    # the CUs' busy share over the makespan: each chain run alone in one
+    # workgroup from its start (the same trajectory as in the batch, bit for
+    # bit) for its own device time, summed, against every CU for the batch's
+    # makespan
     from brawl_amd import _lib
     _, n_cus = _lib.lds_bandwidth()
     solo_ms = []
     for L, s0, p in zip(lats, starts, params):
         L.set_config(s0)
-        solo_ms.append(L.metropolis_simulated_annealing(**p).kernel_ms)
+        solo_ms.append(_undivided_ms(L, **p))
     out["cu_busy_share"] = float(sum(solo_ms) / (n_cus * out["makespan_ms"]))
-    out["cu_busy_note"] = (f"sum of the {len(solo_ms)} chains' device times alone "
+    out["cu_busy_note"] = (f"sum of the {len(solo_ms)} chains' device times alone in one workgroup "
                            f"({sum(solo_ms):.0f} ms; longest {max(solo_ms):.1f} ms) over {n_cus} CUs "
                            f"x the makespan")
     log(f"[bench] batched: CUs busy {out['cu_busy_share']:.2f} of the makespan "
-        f"(longest chain alone {max(solo_ms):.1f} ms)")
+        f"(longest chain alone in one workgroup {max(solo_ms):.1f} ms)")
     if tune:
         for L, s0 in zip(lats, starts):
             L.set_config(s0)
@@ -382,6 +383,19 @@ def batched(steps: int, warmup: int, tune: bool = True):
     for L in lats:
         L.close()
     return out
+
+
+def _undivided_ms(lat, *, T, n_sweeps, seed, delta_T=0.0, T_steps=1, burn_in_sweeps=0):
+    """Device time of an anneal in one workgroup (the entry point without
+    allocations divides no chain)."""
+    from brawl_amd import _lib
+    p = _lib.AnnealParams(float(T), float(delta_T), int(T_steps), int(n_sweeps), int(burn_in_sweeps), 0,
+                          int(seed) & (2**64 - 1))
+    outs = [np.zeros(T_steps) for _ in range(3)]
+    st = _lib.RunStats()
+    _lib.check(lat._L.bwl_metropolis_anneal_noalloc(
+        lat._h, ctypes.byref(p), *[o.ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for o in outs], ctypes.byref(st)))
+    return float(st.kernel_ms)
 
 
 def lds_roofline(plain_gbs: float, plain_cus: int, batched_out=None):
@@ -725,7 +739,7 @@ def sequential_bit_exact(sweeps: int = 100):
     log(f"[bench] sequential bit-exact replicas: {rtrials} trials in {rdt * 1e3:.1f} ms "
         f"({rms:.1f} ms device)")
     return {"workload": f"fcc 8^3 (2048 sites), S=2, 2 shells, 600 K, {sweeps} sweeps, energy "
-                        "recounted after every sweep; one wavefront, the reference's MT19937 stream",
+                        "recounted after every sweep; one workgroup, the reference's MT19937 stream",
             "trials": sweeps * N, "value": sweeps * N / dt, "unit": "swap trials/s",
             "us_per_trial": dt / (sweeps * N) * 1e6, "accepted": acc,
             "replicas": {"chains": reps, "sweeps": rsweeps, "trials": rtrials,
